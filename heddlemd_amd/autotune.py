@@ -4,7 +4,7 @@ choices that leave its physics unchanged and keeps the fastest.
 The choices are the neighbour skin (every skin gives the same forces: the
 rebuild is triggered by the displacement check, so the list always holds
 every pair within the cutoff), the pair-list form (`hd_set_pair_list`:
-packed 64-atom clusters or per-atom full lists) and the reciprocal-space
+row lists over 64-atom blocks or per-atom full lists) and the reciprocal-space
 transform (`hd_set_spme_dft`: FP32 LDS FFT or split-precision matrix-core
 DFT, the latter only on power-of-two axes of 32 to 128 points).  The
 reference has no autotuner; this is MI355X-side tuning of the same step.

@@ -148,6 +148,71 @@ __device__ __forceinline__ void hd_rel_to_center_rcp(float x, float y, float z, 
   rz = (float)dz;
 }
 
+// Periodic images within one box vector per axis, as a code 0..26:
+// (ka + 1) + 3 (kb + 1) + 9 (kc + 1).
+#define HD_IMAGE_NONE 13u
+#define HD_FIXED_FAR 1073741824  // hd_rel_fixed: out of every list's reach
+
+// An atom's position relative to a centre c: x - c + the lattice vectors of
+// two image codes (the list's image of the j-atom's cell, and the atom's own
+// return to the cell it was listed in).  Without a shift the f32 difference
+// is rounded once; with one the sum is formed in FP64 and rounded once.
+__device__ __forceinline__ void hd_rel_image(float x, float y, float z, float4 c, unsigned code,
+                                             unsigned own, const HdLattice& L, float& rx,
+                                             float& ry, float& rz) {
+  if (code == HD_IMAGE_NONE && own == HD_IMAGE_NONE) {
+    rx = x - c.x;
+    ry = y - c.y;
+    rz = z - c.z;
+    return;
+  }
+  double ka = (double)((int)(code % 3u + own % 3u) - 2),
+         kb = (double)((int)((code / 3u) % 3u + (own / 3u) % 3u) - 2),
+         kc = (double)((int)(code / 9u + own / 9u) - 2);
+  rx = (float)(((double)x - (double)c.x) +
+               (ka * (double)L.lx + kb * (double)L.xy + kc * (double)L.xz));
+  ry = (float)(((double)y - (double)c.y) + (kb * (double)L.ly + kc * (double)L.yz));
+  rz = (float)(((double)z - (double)c.z) + kc * (double)L.lz);
+}
+
+// The same in units of 1 / scale (a power of two), rounded to a whole
+// number: differences of two such offsets are exact, so a pair's
+// displacement is rounded once, at its own size, in whatever image.  The
+// caller's scale keeps offsets within 2^29; a position that is not (or is
+// not a number) goes to 2^30 along x, out of everything's reach.
+__device__ __forceinline__ int3 hd_rel_fixed(float x, float y, float z, float4 c, unsigned code,
+                                             unsigned own, const HdLattice& L, double scale) {
+  double dx = (double)x - (double)c.x, dy = (double)y - (double)c.y, dz = (double)z - (double)c.z;
+  if (code != HD_IMAGE_NONE || own != HD_IMAGE_NONE) {
+    const double ka = (double)((int)(code % 3u + own % 3u) - 2),
+                 kb = (double)((int)((code / 3u) % 3u + (own / 3u) % 3u) - 2),
+                 kc = (double)((int)(code / 9u + own / 9u) - 2);
+    dx += ka * (double)L.lx + kb * (double)L.xy + kc * (double)L.xz;
+    dy += kb * (double)L.ly + kc * (double)L.yz;
+    dz += kc * (double)L.lz;
+  }
+  const double lim = 536870912.0;
+  dx *= scale;
+  dy *= scale;
+  dz *= scale;
+  if (!(fabs(dx) <= lim && fabs(dy) <= lim && fabs(dz) <= lim))
+    return make_int3(HD_FIXED_FAR, 0, 0);
+  return make_int3(__double2int_rn(dx), __double2int_rn(dy), __double2int_rn(dz));
+}
+
+// The code of the lattice vector that takes a wrapped position p back to
+// the image nearest its wrapped position `ref` at the last rebuild (an atom
+// that has crossed a face since then was wrapped to the other side).
+__device__ __forceinline__ unsigned hd_own_image(float4 p, float4 ref, const HdLattice& L) {
+  float sa, sb, sc;
+  hd_cart_to_frac(p.x - ref.x, p.y - ref.y, p.z - ref.z, L, sa, sb, sc);
+  int ka = (int)floorf(sa + 0.5f), kb = (int)floorf(sb + 0.5f), kc = (int)floorf(sc + 0.5f);
+  ka = min(max(ka, -1), 1);
+  kb = min(max(kb, -1), 1);
+  kc = min(max(kc, -1), 1);
+  return (unsigned)(1 - ka) + 3u * (unsigned)(1 - kb) + 9u * (unsigned)(1 - kc);
+}
+
 // SPME spline origin of one atom: wrap into the primary cell, fractional
 // coordinate + 1/2, u = s * n, primary bin floor(u) (mod n) and offset
 // t = u - floor(u) (the geometry of kernels/spme_spread_gather.cuh:90-126).
@@ -219,6 +284,23 @@ __device__ __forceinline__ float hd_from_fixed48(long long v) {
   const float inv = (1.0f / 16777216.0f) / 16777216.0f;
   return (float)v * inv;
 }
+
+// Set bits of a wave mask below this lane.
+__device__ __forceinline__ unsigned hd_rank(unsigned long long m) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+// Orders one wave's LDS accesses: what its lanes wrote before is what its
+// lanes read after.
+__device__ __forceinline__ void hd_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Two words that may alias anything (16-bit list entries moved four at a time).
+typedef unsigned hd_u32x2 __attribute__((ext_vector_type(2), may_alias));
 
 __device__ __forceinline__ unsigned long long hd_lane_mask_lt() {
   unsigned lane = __lane_id();

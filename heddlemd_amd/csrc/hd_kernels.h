@@ -6,6 +6,24 @@
 #include <stdint.h>
 #include <string.h>
 
+// Row lists (k_build_rows, k_pair_rows).  Unit u = block * parts + part
+// holds one part of a block's neighbourhood:
+//   jcount[u]          active j-atoms | others << 16
+//   jslot              [u * jcap + k] slot | image code << 27 of j-atom k: the
+//                      active ones from k = 0 up, the others from jcap - 1 down
+//   rowhdr[u * 8 + w]  chunks of active entries | chunks of all entries << 16
+//                      of the rows of i-atoms 8 w .. 8 w + 7
+//   rows               [(u * 64 + i) * rcap] 16-bit entries of
+//                      i-atom i: 16 * index into the j-list, 16 * jcap for
+//                      padding
+#define HD_ROW_THREADS 512u
+#define HD_ROW_WAVES 8u
+#define HD_ROW_I 8
+#define HD_ROW_CHUNK 32u
+#define HD_ROW_SLOT_BITS 27
+#define HD_ROW_SLOTS (1u << HD_ROW_SLOT_BITS)
+#define HD_ROW_JMAX 4094u  // largest jcap (16 * jcap fits 16 bits)
+
 struct HdNeighborArgs {
   unsigned n, npad, nvox, cap;
   unsigned nv[3];
@@ -21,16 +39,22 @@ struct HdNeighborArgs {
   const unsigned *type, *key;
   unsigned *tile_type, *tile_key;
   float4* tile_posq;
+  float4* tile_ref;          // wrapped slot positions of the last rebuild
+  unsigned char* tile_img;   // image code back to them (hd_own_image)
   float4 *center, *half;
   unsigned *entry_atoms, *entry_count, *max_count;
   unsigned *status, *rebuild_count;
+  // row lists; entry_count then holds each unit's row chunks
+  unsigned parts, jcap, rcap, active_types;  // active_types: bit per LJ type
+  unsigned *jslot, *jcount, *rowhdr, *max_j;
+  unsigned short* rows;
   // atom-list mode: entry_atoms holds per-block rows of per-atom neighbour
   // lists (row k = k-th neighbour of each of the block's 64 atoms) and
   // entry_count the block's row count; exclusions are applied at build
   int atom_lists;
   unsigned excl_span;
   unsigned long long* block_mask;  // nblocks x hd_block_pair_chunks(nblocks) candidate masks
-  unsigned* block_order;           // blocks by entry count, heaviest first (rebuild steps)
+  unsigned* block_order;           // units by row chunks, heaviest first (rebuild steps)
   unsigned* build_ticket;          // zeroed word for the folded rebuild-clear
 };
 unsigned hd_block_pair_chunks(unsigned nblocks);
@@ -42,14 +66,15 @@ void hd_launch_disp_check(hipStream_t st, const HdNeighborArgs& a);
 // number of chunk sums of the voxel-count scan (the buffer needs one more)
 unsigned hd_voxel_scan_parts(unsigned nvox);
 // block_pairs = false when hd_launch_neighbor_small already ran the
-// block-pair box tests of this step; fold_clear: the packed-list build's
-// last workgroup orders the blocks and clears the rebuild request (no
-// separate launch; needs build_ticket)
+// block-pair box tests of this step; fold_clear: with few units the row
+// build's last workgroup clears the rebuild request (no separate launch;
+// needs build_ticket)
 void hd_launch_neighbor_build(hipStream_t st, const HdNeighborArgs& a, bool block_pairs = true,
                               bool fold_clear = false);
 void hd_launch_tile_gather(hipStream_t st, const float4* posq, const unsigned* sorted_id,
                            const float* lattice, float4* tile_posq, long long* fpj,
-                           long long* fpj_ew, unsigned n, unsigned npad);
+                           long long* fpj_ew, unsigned n, unsigned npad, float4* tile_ref,
+                           unsigned char* tile_img);
 // the same, and on rebuild steps the slot types and keys and the blocks'
 // bounding boxes (which the neighbour build then uses)
 void hd_launch_tile_gather_rebuild(hipStream_t st, const HdNeighborArgs& a, long long* fpj,
@@ -77,15 +102,26 @@ struct HdPairArgs {
   unsigned excl_span;  // pairs with |key_i - key_j| <= excl_span are excluded
   const float4 *center, *half;
   const unsigned *entry_atoms, *entry_count;
+  // atom-list mode: i-side sums (plain stores); the row lists add theirs to
+  // fpj, beside the bonded terms
   long long *fpi, *fpi_ew, *fpj, *fpj_ew;
-  int atom_lists;  // per-atom full lists (no j side) instead of the packed cluster list
+  int atom_lists;  // per-atom full lists instead of the row lists
   int ortho;       // no box tilt
-  const unsigned* block_order;  // workgroup -> block for the packed-list kernel
-  const float4* lj_tab;  // ntypes > 4: the type-pair table (hd_pair_lj_table), device
+  unsigned parts, jcap, rcap;
+  const unsigned *jslot, *jcount, *rowhdr;
+  const unsigned char* tile_img;
+  const unsigned short* rows;
+  const unsigned* block_order;  // workgroup -> unit for the row-list kernel
+  const float4* lj_tab;  // the type-pair table (hd_pair_lj_table), device
 };
-// Largest type count of the LDS table form of the pair kernels.
+// Bit per LJ type with a nonzero interaction with any type: the j-atoms of
+// the others are listed apart, so that their pairs skip the LJ terms.
+unsigned hd_pair_active_types(int nt, const double* sigma, const double* eps);
+// LDS bytes of the row-list pair kernel beside its j records
+unsigned hd_pair_rows_lds(int nt, unsigned jcap);
+// Largest type count of the pair kernels' LDS table.
 int hd_pair_table_max_types();
-// The type-pair table read by the pair kernels beyond four types: 8 floats
+// The type-pair table of the pair kernels: 8 floats
 // per pair k = i nt + j: 12 c12, 6 c6, c12, c6, cut^2 (-1 when eps = 0),
 // r_switch^2, 1/(cut^2 - r_switch^2) (0 without a switch), 0.
 void hd_pair_lj_table(int nt, const double* sigma, const double* eps, const double* cut,

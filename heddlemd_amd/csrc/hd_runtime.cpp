@@ -81,7 +81,7 @@ struct hd_ctx {
   int spline_order = 4;
   double r_skin = -1.0;
   unsigned excl_span = 0;
-  int atom_lists = 0;  // 1: per-atom full neighbour lists instead of the packed cluster list
+  int atom_lists = 0;  // 1: per-atom full neighbour lists instead of the row lists
   std::vector<uint32_t> h_angles;  // i, j, k per angle
   std::vector<double> h_ang_k, h_ang_t0;
   unsigned* d_angles = nullptr;
@@ -184,11 +184,18 @@ struct hd_ctx {
   unsigned *voxel_rank = nullptr, *atom_key = nullptr, *voxel_count = nullptr,
            *voxel_off = nullptr, *voxel_cursor = nullptr, *voxel_part = nullptr;
   unsigned *sorted_id = nullptr, *slot_of = nullptr, *tile_type = nullptr, *tile_key = nullptr;
-  float4 *tile_posq = nullptr, *center = nullptr, *half = nullptr;
+  float4 *tile_posq = nullptr, *center = nullptr, *half = nullptr, *tile_ref = nullptr;
+  unsigned char* tile_img = nullptr;
   unsigned *entry_atoms = nullptr, *entry_count = nullptr;
+  // row lists: parts per block, j-atoms per unit, entries per row
+  unsigned parts = 1, jcap = 0, rcap = 0, active_types = 0;
+  unsigned *jslot = nullptr, *jcount = nullptr, *rowhdr = nullptr;
+  unsigned short* rows = nullptr;
   unsigned long long* block_mask = nullptr;  // block-pair candidate masks
-  unsigned* block_order = nullptr;           // pair workgroup -> block
-  unsigned* ctrl = nullptr;  // [0] status, [1] rebuild count, [2] max entries, [3] build ticket
+  unsigned* block_order = nullptr;           // pair workgroup -> unit
+  // [0] status, [1] rebuild count, [2] most entries of a list row, [3] build
+  // ticket, [4] most j-atoms of a row-list unit
+  unsigned* ctrl = nullptr;
   long long *fpi = nullptr, *fpi_ew = nullptr, *fpj = nullptr, *fpj_ew = nullptr;
   // device: SPME
   long long* rho_fixed = nullptr;
@@ -419,6 +426,8 @@ HdNeighborArgs nb_args(hd_ctx* c) {
   a.tile_type = c->tile_type;
   a.tile_key = c->tile_key;
   a.tile_posq = c->tile_posq;
+  a.tile_ref = c->tile_ref;
+  a.tile_img = c->tile_img;
   a.center = c->center;
   a.half = c->half;
   a.entry_atoms = c->entry_atoms;
@@ -431,6 +440,15 @@ HdNeighborArgs nb_args(hd_ctx* c) {
   a.excl_span = c->excl_span;
   a.block_mask = c->block_mask;
   a.block_order = c->block_order;
+  a.parts = c->parts;
+  a.jcap = c->jcap;
+  a.rcap = c->rcap;
+  a.active_types = c->active_types;
+  a.jslot = c->jslot;
+  a.jcount = c->jcount;
+  a.rowhdr = c->rowhdr;
+  a.rows = c->rows;
+  a.max_j = c->ctrl + 4;
   return a;
 }
 
@@ -598,16 +616,28 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   // what it reads: it runs on the second stream, concurrent with them, and
   // joins before the finalize.  The stage-timing pass keeps one stream so
   // that every stage is timed alone.
-  bool fork = c->have_spme && !timed && c->spme_fork;
-  if (fork) {
+  //
+  // While the spread fits the chip (two workgroups per CU) it starts beside
+  // the build (24,576 atoms, 128 bricks: 152 us per step, 165 with the build
+  // first; 52,773 atoms, 250 bricks: 244 and 261).  A larger spread fills
+  // every CU's LDS, and the build's launch, idle on most steps, waited 30 to
+  // 40 us behind it: there the build goes first (196,608 atoms, 1,024
+  // bricks).
+  const bool fork = c->have_spme && !timed && c->spme_fork;
+  unsigned brick[3];
+  const bool fork_late =
+      fork && hd_spread_bricks(c->grid[0], c->grid[1], c->grid[2], brick) > 512u;
+  auto start_spme = [&] {
     (void)hipEventRecord(c->ev_fork, st);
     (void)hipStreamWaitEvent(c->side, c->ev_fork, 0);
     enqueue_spme(c, c->side, false, small_nb);
     (void)hipEventRecord(c->ev_join, c->side);
-  }
+  };
+  if (fork && !fork_late) start_spme();
   stage_begin(c, "neighbor_build", timed);
   hd_launch_neighbor_build(st, na, !small_nb, small_nb);
   stage_end(c, timed);
+  if (fork_late) start_spme();
   HdPairArgs pa;
   memset(&pa, 0, sizeof(pa));
   pa.n = (unsigned)c->n;
@@ -640,6 +670,14 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   pa.atom_lists = c->atom_lists;
   pa.ortho = box_ortho(c) ? 1 : 0;
   pa.lj_tab = c->d_lj_tab;
+  pa.parts = c->parts;
+  pa.jcap = c->jcap;
+  pa.rcap = c->rcap;
+  pa.jslot = c->jslot;
+  pa.tile_img = c->tile_img;
+  pa.jcount = c->jcount;
+  pa.rowhdr = c->rowhdr;
+  pa.rows = c->rows;
   stage_begin(c, "pair_force", timed);
   hd_launch_pair(st, pa, c->atom_lists && ev == 2 ? 1 : ev);
   if (!c->h_ang_k.empty())
@@ -664,7 +702,7 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   fa.npad = c->npad;
   fa.sorted_id = c->sorted_id;
   fa.tile_posq = c->tile_posq;
-  fa.fpi = c->fpi;
+  fa.fpi = c->atom_lists ? c->fpi : nullptr;
   fa.fpi_ew = c->fpi_ew;
   fa.fpj = c->fpj;
   fa.fpj_ew = c->fpj_ew;
@@ -2140,6 +2178,7 @@ static int build_list(hd_ctx* c) {
   HIPCHK(c, hipMemcpyAsync(c->ctrl, &force, sizeof(unsigned), hipMemcpyHostToDevice, c->stream));
   unsigned zero = 0;
   HIPCHK(c, hipMemcpyAsync(c->ctrl + 2, &zero, sizeof(unsigned), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->ctrl + 4, &zero, sizeof(unsigned), hipMemcpyHostToDevice, c->stream));
   HdNeighborArgs na = nb_args(c);
   hd_launch_neighbor_update(c->stream, na);
   hd_launch_tile_gather_rebuild(c->stream, na, c->fpj, c->fpj_ew);
@@ -2149,17 +2188,129 @@ static int build_list(hd_ctx* c) {
   return HD_OK;
 }
 
+// The pair kernel's unit order: identity until a rebuild orders the units
+static int alloc_units(hd_ctx* c, unsigned units) {
+  dfree(c, c->block_order);
+  dfree(c, c->entry_count);
+  c->block_order = c->entry_count = nullptr;
+  DALLOC(c, c->entry_count, units);
+  DALLOC(c, c->block_order, units);
+  std::vector<unsigned> ident(units);
+  for (unsigned b = 0; b < units; ++b) ident[b] = b;
+  return upload(c, c->block_order, ident.data(), units);
+}
+
 static int alloc_entries(hd_ctx* c, unsigned cap) {
-  if (c->entry_atoms) dfree(c, c->entry_atoms);
+  dfree(c, c->entry_atoms);
   c->entry_atoms = nullptr;
   c->cap = cap;
+  int r = alloc_units(c, c->nblocks);
+  if (r) return r;
   DALLOC(c, c->entry_atoms, (size_t)c->nblocks * cap * 64);
   return HD_OK;
 }
 
-// Probe the list size, then size the per-block regions with headroom.
+static int alloc_rows(hd_ctx* c, unsigned parts, unsigned jcap, unsigned rcap) {
+  for (void* p : {(void*)c->jslot, (void*)c->jcount, (void*)c->rowhdr, (void*)c->rows})
+    dfree(c, p);
+  c->jslot = c->jcount = c->rowhdr = nullptr;
+  c->rows = nullptr;
+  const size_t units = (size_t)c->nblocks * parts;
+  if (units >= (1ull << 31) / HD_ROW_WAVES)
+    return fail(c, HD_ERR_UNSUPPORTED, "row lists: %zu units", units);
+  c->parts = parts;
+  c->jcap = jcap;
+  c->rcap = rcap;
+  int r = alloc_units(c, (unsigned)units);
+  if (r) return r;
+  DALLOC(c, c->jslot, units * jcap);
+  DALLOC(c, c->jcount, units);
+  DALLOC(c, c->rowhdr, units * HD_ROW_WAVES);
+  DALLOC(c, c->rows, units * 64 * rcap);
+  return HD_OK;
+}
+
+// Largest j-list of a unit: 64 KB of LDS for its records beside the build's
+// candidate lists and the pair kernel's type table
+static unsigned rows_jcap_max(const hd_ctx* c) {
+  unsigned build = (65536u - 21u * 1024u) / 16u;
+  unsigned pair = (65536u - hd_pair_rows_lds(c->ntypes, 0) - 64u) / (c->ntypes > 1 ? 17u : 16u);
+  return std::min(std::min(build, pair), HD_ROW_JMAX) & ~7u;
+}
+
+// Blocks are split into `parts` units until the chip has work everywhere:
+// a unit is one 8-wave workgroup and 512 of them are the two per CU that the
+// build's LDS and registers allow.  Targets of 256 / 512 / 1,024 / 2,048
+// units measured, us per pass: 10,000 argon atoms (50 steps) 1752 / 1737 /
+// 1744 / 1815; 7,938 atoms of water (50 steps) 6850 / 6836 / 7014 / 7304;
+// four frames of 12,003 atoms in a tilted cell 1375 / 1432 / 1524 / 1632.
+static unsigned rows_parts(const hd_ctx* c) {
+  unsigned p = 1;
+  while (p < 32u && c->nblocks * p * 2u <= 512u) p *= 2;
+  return p;
+}
+
+// First guess of a unit's j-atoms and an i-atom's row at the mean density:
+// the atoms within r_search of a cube of 64 atoms, of one atom.
+static void rows_guess(const hd_ctx* c, unsigned parts, double* nj, double* nr) {
+  const double rho = (double)c->n / (c->lattice[0] * c->lattice[1] * c->lattice[2]);
+  const double rs = c->rmax + c->r_skin, e = cbrt(64.0 / rho);
+  const double sphere = 4.18879020478639 * rs * rs * rs;
+  *nj = rho * (e * e * e + 6.0 * e * e * rs + 3.0 * M_PI * e * rs * rs + sphere) / parts;
+  *nr = rho * sphere / parts;
+}
+
+// Row lists: probe the sizes with what there is, then give the j-lists and
+// rows headroom (never below the capacities they already have).  A j-list
+// beyond the LDS limit splits the blocks further.
+static int size_rows(hd_ctx* c) {
+  int r;
+  const unsigned floor_j = c->jcap, floor_r = c->rcap;  // 0 at set-up
+  unsigned parts = std::max(c->parts, rows_parts(c));
+  const unsigned jmax = rows_jcap_max(c);
+  double gj, gr;
+  rows_guess(c, parts, &gj, &gr);
+  unsigned jcap = std::min(std::max(floor_j, (unsigned)std::min(1.8 * gj + 128.0, 1e6) & ~7u), jmax);
+  unsigned rcap = std::max(floor_r, ((unsigned)std::min(1.8 * gr + 96.0, 1e6)) / HD_ROW_CHUNK *
+                                        HD_ROW_CHUNK);
+  for (int pass = 0; pass < 24; ++pass) {
+    if ((r = alloc_rows(c, parts, jcap, rcap))) return r;
+    if ((r = build_list(c))) return r;
+    unsigned ctrl[8];
+    HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
+    const unsigned need_j = ctrl[4], need_r = ctrl[2];
+    // a whole neighbourhood varies little between rebuilds, its parts more
+    // (which candidates a part gets changes); the limit may cut the headroom
+    unsigned want_j = parts > 1 ? ((unsigned)ceil(need_j * 1.75) + 64u + 7u) & ~7u
+                                : ((unsigned)ceil(need_j * 1.5) + 7u) & ~7u;
+    if (1.1 * need_j + 16.0 <= jmax) want_j = std::min(want_j, jmax);
+    unsigned want_r = ((unsigned)ceil(need_r * 1.5) + HD_ROW_CHUNK - 1u) / HD_ROW_CHUNK *
+                      HD_ROW_CHUNK;
+    if (want_j > jmax || ((ctrl[0] & NB_STATUS_OVERFLOW) && need_j <= jcap && need_r <= rcap)) {
+      // the j-list does not fit LDS, or the candidates their list
+      if (parts >= 4096u) return fail(c, HD_ERR_OVERFLOW, "neighbour list overflow while sizing");
+      parts *= 2;
+      continue;
+    }
+    // kept when it fits and the guess was not far too large
+    const bool fits = !(ctrl[0] & NB_STATUS_OVERFLOW) && want_j <= jcap && want_r <= rcap;
+    if (fits && (pass > 0 || floor_r || (jcap <= 2u * want_j && rcap <= 2u * want_r))) {
+      // set-up builds the list twice, as a probe and in its final size
+      if (pass == 0 && !floor_r && (r = build_list(c))) return r;
+      unsigned zero = 0;
+      HIPCHK(c, hipMemcpy(c->ctrl, &zero, sizeof(unsigned), hipMemcpyHostToDevice));
+      return HD_OK;
+    }
+    jcap = std::max(want_j, fits ? floor_j : jcap);
+    rcap = std::max(want_r, fits ? floor_r : rcap);
+  }
+  return fail(c, HD_ERR_OVERFLOW, "neighbour list overflow while sizing");
+}
+
+// Probe the list size, then size the regions with headroom.
 static int size_list(hd_ctx* c) {
   int r;
+  if (!c->atom_lists) return size_rows(c);
   if ((r = alloc_entries(c, 64))) return r;
   if ((r = build_list(c))) return r;
   unsigned ctrl[4];
@@ -2252,6 +2403,8 @@ int hd_setup(hd_ctx* c) {
   unsigned n = (unsigned)c->n;
   c->nblocks = (n + 63) / 64;
   c->npad = c->nblocks * 64;
+  // a row list's j-atoms are 27-bit slots
+  if (c->npad >= HD_ROW_SLOTS) c->atom_lists = 1;
   // voxel grid in fractional coordinates (so the order survives box
   // rescaling): a power of two per axis, about two atoms per voxel, ranked
   // along a Hilbert curve over the enclosing 2^bits cube
@@ -2289,7 +2442,8 @@ int hd_setup(hd_ctx* c) {
     DALLOC(c, c->vxlo, n); DALLOC(c, c->vylo, n); DALLOC(c, c->vzlo, n);
   }
   DALLOC(c, c->d_lattice, 6);
-  if (c->ntypes > 4) {
+  c->active_types = hd_pair_active_types(c->ntypes, c->lj_sigma.data(), c->lj_eps.data());
+  {
     std::vector<float> tab(8 * (size_t)c->ntypes * c->ntypes);
     hd_pair_lj_table(c->ntypes, c->lj_sigma.data(), c->lj_eps.data(), c->lj_cut.data(),
                      c->lj_rsw.data(), tab.data());
@@ -2309,19 +2463,10 @@ int hd_setup(hd_ctx* c) {
   DALLOC(c, c->sorted_id, c->npad); DALLOC(c, c->slot_of, n);
   DALLOC(c, c->tile_type, c->npad); DALLOC(c, c->tile_key, c->npad);
   DALLOC(c, c->tile_posq, c->npad);
+  DALLOC(c, c->tile_ref, c->npad); DALLOC(c, c->tile_img, c->npad);
   DALLOC(c, c->center, c->nblocks); DALLOC(c, c->half, c->nblocks);
-  DALLOC(c, c->entry_count, c->nblocks);
   DALLOC(c, c->block_mask, (size_t)c->nblocks * hd_block_pair_chunks(c->nblocks));
-  DALLOC(c, c->block_order, c->nblocks);
-  {
-    // identity until the first rebuild orders the blocks
-    std::vector<unsigned> ident(c->nblocks);
-    for (unsigned b = 0; b < c->nblocks; ++b) ident[b] = b;
-    if (hipMemcpy(c->block_order, ident.data(), ident.size() * sizeof(unsigned),
-                  hipMemcpyHostToDevice) != hipSuccess)
-      return fail(c, HD_ERR_HIP, "block order upload failed");
-  }
-  DALLOC(c, c->ctrl, 4);
+  DALLOC(c, c->ctrl, 8);
   DALLOC(c, c->fpi, (size_t)c->npad * 4); DALLOC(c, c->fpj, (size_t)c->npad * 4);
   DALLOC(c, c->fpi_ew, (size_t)c->npad * 2); DALLOC(c, c->fpj_ew, (size_t)c->npad * 2);
   DALLOC(c, c->red_partials, 2 * HD_REDUCE_BLOCKS);
@@ -2484,23 +2629,31 @@ int hd_setup(hd_ctx* c) {
 }
 
 static int check_status(hd_ctx* c) {
-  unsigned ctrl[4];
+  unsigned ctrl[8];
   HIPCHK(c, hipMemcpyAsync(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (ctrl[0] & 8u) {
+    if (c->atom_lists)
+      return fail(c, HD_ERR_OVERFLOW,
+                  "neighbour list overflow (a block needed %u entries, capacity %u)", ctrl[2],
+                  c->cap);
     return fail(c, HD_ERR_OVERFLOW,
-                "neighbour list overflow (a block needed %u entries, capacity %u)", ctrl[2],
-                c->cap);
+                "neighbour list overflow (a row needed %u entries, capacity %u; a unit %u j-atoms, "
+                "capacity %u)",
+                ctrl[2], c->rcap, ctrl[4], c->jcap);
   }
   if (ctrl[0] & 2u) {
-    // high water: grow the entry regions and rebuild before the next step
-    unsigned cap = (unsigned)ceil(ctrl[2] * 1.5) + 2;
+    // high water: grow the list's regions and rebuild before the next step
     drop_graphs(c);
-    int r = alloc_entries(c, std::max(cap, c->cap));
-    if (r) return r;
+    int r;
+    if (c->atom_lists) {
+      unsigned cap = (unsigned)ceil(ctrl[2] * 1.5) + 2;
+      if ((r = alloc_entries(c, std::max(cap, c->cap)))) return r;
+      if ((r = build_list(c))) return r;
+    } else if ((r = size_rows(c))) {
+      return r;
+    }
     unsigned zero = 0;
-    HIPCHK(c, hipMemcpy(c->ctrl, &zero, sizeof(unsigned), hipMemcpyHostToDevice));
-    if ((r = build_list(c))) return r;
     HIPCHK(c, hipMemcpy(c->ctrl, &zero, sizeof(unsigned), hipMemcpyHostToDevice));
   }
   return HD_OK;
@@ -3231,36 +3384,59 @@ int hd_get_scalars(hd_ctx* c, double* out) {
 int hd_get_pairs(hd_ctx* c, uint32_t* out, uint64_t cap, uint64_t* n_pairs) {
   if (!c || !c->ready || !n_pairs) return fail(c, HD_ERR_STATE, "not set up");
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  std::vector<unsigned> ents((size_t)c->nblocks * c->cap * 64), cnt(c->nblocks), sid(c->npad);
-  HIPCHK(c, hipMemcpy(ents.data(), c->entry_atoms, ents.size() * 4, hipMemcpyDeviceToHost));
-  HIPCHK(c, hipMemcpy(cnt.data(), c->entry_count, cnt.size() * 4, hipMemcpyDeviceToHost));
+  std::vector<unsigned> sid(c->npad);
   HIPCHK(c, hipMemcpy(sid.data(), c->sorted_id, sid.size() * 4, hipMemcpyDeviceToHost));
   std::vector<uint64_t> pairs;
   unsigned n = (unsigned)c->n;
+  auto add = [&](unsigned is, unsigned js) {
+    uint32_t iid = sid[is], jid = sid[js];
+    uint32_t lo = std::min(iid, jid), hi = std::max(iid, jid);
+    pairs.push_back(((uint64_t)lo << 32) | hi);
+  };
   if (c->atom_lists) {
+    std::vector<unsigned> ents((size_t)c->nblocks * c->cap * 64), cnt(c->nblocks);
+    HIPCHK(c, hipMemcpy(ents.data(), c->entry_atoms, ents.size() * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpy(cnt.data(), c->entry_count, cnt.size() * 4, hipMemcpyDeviceToHost));
     // row k of block b: the k-th neighbour of each of the block's atoms
     for (unsigned b = 0; b < c->nblocks; ++b)
       for (unsigned k = 0; k < cnt[b]; ++k)
         for (unsigned l = 0; l < 64; ++l) {
           unsigned js = ents[((size_t)b * c->cap + k) * 64 + l], is = b * 64 + l;
-          if (js >= n || is >= n) continue;
-          uint32_t iid = sid[is], jid = sid[js];
-          uint32_t lo = std::min(iid, jid), hi = std::max(iid, jid);
-          pairs.push_back(((uint64_t)lo << 32) | hi);
+          if (js < n && is < n) add(is, js);
         }
-  }
-  for (unsigned b = 0; b < c->nblocks && !c->atom_lists; ++b) {
-    for (unsigned e = 0; e < cnt[b]; ++e)
-      for (unsigned l = 0; l < 64; ++l) {
-        unsigned js = ents[((size_t)b * c->cap + e) * 64 + l];
-        if (js >= n) continue;
-        unsigned jid = sid[js];
-        for (unsigned m = 0; m < 64; ++m) {
-          unsigned is = b * 64 + m;
-          if (is >= n || is == js) continue;
-          unsigned iid = sid[is];
-          uint32_t lo = std::min(iid, jid), hi = std::max(iid, jid);
-          pairs.push_back(((uint64_t)lo << 32) | hi);
+  } else {
+    const size_t units = (size_t)c->nblocks * c->parts;
+    std::vector<unsigned> hdr(units * HD_ROW_WAVES), jslot(units * c->jcap);
+    const size_t stride = c->rcap;
+    std::vector<unsigned short> rows(units * 64 * stride);
+    HIPCHK(c, hipMemcpy(hdr.data(), c->rowhdr, hdr.size() * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpy(jslot.data(), c->jslot, jslot.size() * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpy(rows.data(), c->rows, rows.size() * 2, hipMemcpyDeviceToHost));
+    for (size_t uw = 0; uw < units * HD_ROW_WAVES; ++uw) {
+      const size_t u = uw / HD_ROW_WAVES;
+      for (unsigned q = 0; q < HD_ROW_I; ++q) {
+        const unsigned i = (unsigned)(uw % HD_ROW_WAVES) * HD_ROW_I + q;
+        const unsigned is = (unsigned)(u / c->parts) * 64u + i;
+        const unsigned short* rp = rows.data() + (u * 64 + i) * stride;
+        for (unsigned k = 0; is < n && k < (hdr[uw] >> 16) * HD_ROW_CHUNK; ++k) {
+          const unsigned j = rp[k] >> 4;
+          if (j < c->jcap) add(is, jslot[u * c->jcap + j] & (HD_ROW_SLOTS - 1u));
+        }
+      }
+    }
+    // the rows leave excluded pairs out; the pair set has them: the j-atoms
+    // of a block's neighbourhood that its atoms' keys exclude
+    std::vector<unsigned> cnt(units), key(c->npad);
+    HIPCHK(c, hipMemcpy(cnt.data(), c->jcount, cnt.size() * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpy(key.data(), c->tile_key, key.size() * 4, hipMemcpyDeviceToHost));
+    for (size_t u = 0; u < units; ++u)
+      for (unsigned q = 0; q < (cnt[u] & 0xFFFFu) + (cnt[u] >> 16); ++q) {
+        const unsigned na = cnt[u] & 0xFFFFu, k = q < na ? q : c->jcap - 1u - (q - na);
+        const unsigned js = jslot[u * c->jcap + k] & (HD_ROW_SLOTS - 1u);
+        for (unsigned l = 0; l < 64; ++l) {
+          const unsigned is = (unsigned)(u / c->parts) * 64u + l;
+          if (is < n && is != js && key[js] - key[is] + c->excl_span <= 2u * c->excl_span)
+            add(is, js);
         }
       }
   }
@@ -3292,12 +3468,19 @@ int hd_count_pairs(hd_ctx* c, uint64_t* out) {
   pa.excl_span = c->excl_span;
   pa.entry_atoms = c->entry_atoms;
   pa.entry_count = c->entry_count;
-  pa.block_order = c->block_order;
   pa.atom_lists = c->atom_lists;
   pa.ortho = box_ortho(c) ? 1 : 0;
+  pa.center = c->center;
+  pa.parts = c->parts;
+  pa.jcap = c->jcap;
+  pa.rcap = c->rcap;
+  pa.jslot = c->jslot;
+  pa.tile_img = c->tile_img;
+  pa.rowhdr = c->rowhdr;
+  pa.rows = c->rows;
   if (e == hipSuccess) {
     hd_launch_tile_gather(c->stream, c->posq, c->sorted_id, c->d_lattice, c->tile_posq, c->fpj,
-                          c->fpj_ew, (unsigned)c->n, c->npad);
+                          c->fpj_ew, (unsigned)c->n, c->npad, c->tile_ref, c->tile_img);
     hd_launch_count_pairs(c->stream, pa, d);
     e = hipGetLastError();
   }
@@ -3330,7 +3513,8 @@ int hd_get_barostat(hd_ctx* c, double* out) {
 int hd_get_neighbor_stats(hd_ctx* c, uint64_t* out) {
   if (!c || !c->ready || !out) return fail(c, HD_ERR_STATE, "not set up");
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  std::vector<unsigned> cnt(c->nblocks);
+  // atom lists: 64-wide rows of a block; row lists: 32-entry chunks of 8 rows
+  std::vector<unsigned> cnt(c->atom_lists ? c->nblocks : c->nblocks * c->parts);
   HIPCHK(c, hipMemcpy(cnt.data(), c->entry_count, cnt.size() * 4, hipMemcpyDeviceToHost));
   unsigned ctrl[4];
   HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
@@ -3340,7 +3524,7 @@ int hd_get_neighbor_stats(hd_ctx* c, uint64_t* out) {
     mx = std::max<uint64_t>(mx, v);
   }
   out[0] = c->nblocks;
-  out[1] = c->cap;
+  out[1] = c->atom_lists ? c->cap : c->rcap;
   out[2] = mx;
   out[3] = tot;
   out[4] = ctrl[1];

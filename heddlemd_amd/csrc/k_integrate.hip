@@ -943,14 +943,19 @@ __global__ void __launch_bounds__(256) k_finalize(HdFinalizeArgs a) {
   float pe = 0.f, vir = 0.f;
   if (live && q == 0) {
   unsigned id = a.sorted_id[s];
-  const longlong2* fi = reinterpret_cast<const longlong2*>(a.fpi) + 2 * s;
   const longlong2* fj = reinterpret_cast<const longlong2*>(a.fpj) + 2 * s;
-  longlong2 i01 = fi[0], i2x = fi[1], j01 = fj[0], j2x = fj[1];
+  longlong2 i01 = make_longlong2(0, 0), i2x = i01, j01 = fj[0], j2x = fj[1];
+  if (a.fpi) {  // atom lists: the pair sums apart from the bonded terms'
+    const longlong2* fi = reinterpret_cast<const longlong2*>(a.fpi) + 2 * s;
+    i01 = fi[0];
+    i2x = fi[1];
+  }
   float fx = hd_from_fixed48(i01.x + j01.x);
   float fy = hd_from_fixed48(i01.y + j01.y);
   float fz = hd_from_fixed48(i2x.x + j2x.x);
   if (EV) {
-    longlong2 ie = reinterpret_cast<const longlong2*>(a.fpi_ew)[s];
+    longlong2 ie = make_longlong2(0, 0);
+    if (a.fpi) ie = reinterpret_cast<const longlong2*>(a.fpi_ew)[s];
     longlong2 je = reinterpret_cast<const longlong2*>(a.fpj_ew)[s];
     pe = hd_from_fixed48(ie.x + je.x);
     vir = hd_from_fixed48(ie.y + je.y);

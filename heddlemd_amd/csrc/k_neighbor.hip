@@ -1,29 +1,43 @@
-// Neighbour maintenance for the packed 64-atom cluster list (gfx950).
+// Neighbour maintenance for the row lists and the per-atom lists (gfx950).
 //
 // Reference behaviour (what is kept):
 //   * displacement check |x - x_ref|^2 > (r_skin/2)^2 sets bit 0 of a status
 //     word (kernels/neighbor.cu:50-75);
-//   * the list holds, per i-block of consecutive sorted atoms, "entries" of
-//     individual j-atoms, each j-atom within r_search of at least one i-atom,
-//     j-blocks >= i-block only (kernels/neighbor.cu:416-631);
+//   * i-blocks of consecutive sorted atoms, each with the list of the
+//     individual j-atoms within r_search of it
+//     (kernels/neighbor.cu:416-631);
 //   * capacity overflow / high-water bits in the same status word
 //     (kernels/neighbor.cu:643-671).
 // MI355X design (what changes):
-//   * blocks are 64 atoms = one wave64; entries hold 64 j-atoms;
+//   * blocks are 64 atoms; a block's j-atoms are listed once (they are
+//     staged in LDS by the pair kernel) and every i-atom has a row of
+//     16-bit indices into that list, both sides of every pair, exclusions
+//     applied (k_build_rows);
 //   * atoms are ordered along a Hilbert curve over a fixed voxel grid
 //     (voxel = fractional-coordinate cell, so the order survives box
 //     rescaling) instead of by particle id inside r_search cells, which
 //     makes a block spatially compact;
-//   * each i-block owns a fixed-capacity entry region, written in a fixed
-//     order (no atomics, no scatter pass), so the list is deterministic;
+//   * each block owns fixed-capacity regions, written in a fixed order (no
+//     atomics, no scatter pass), so the list is deterministic;
 //   * every kernel here is gated on the status word on the device, so the
 //     whole rebuild lives inside a captured step and needs no host sync.
 #include "hd_device.h"
 #include "hd_kernels.h"
 
 
+// r_search^2 margins: the box tests and the row test are done in f32 on
+// block-relative coordinates; a relative 1e-5 (boxes) and 4e-6 (pairs)
+// covers their rounding, so no pair within r_search is ever lost
+#define NB_BOX_MARGIN 1.00001f
+#define NB_ROW_MARGIN 1.000004f
+
 __device__ __forceinline__ bool nb_rebuild_due(const unsigned* status) {
   return (*(volatile const unsigned*)status & (NB_STATUS_REBUILD | NB_STATUS_FORCE)) != 0u;
+}
+// The same in a kernel during which the request cannot change before every
+// workgroup has read it: one scalar load through the caches.
+__device__ __forceinline__ bool nb_rebuild_due_now(const unsigned* status) {
+  return (*status & (NB_STATUS_REBUILD | NB_STATUS_FORCE)) != 0u;
 }
 
 // Displacement check against the positions of the last rebuild.  A box
@@ -254,7 +268,10 @@ __global__ void k_voxel_sort(const unsigned* __restrict__ voxel_off,
 // Slot-order copy of the positions (wrapped into the cell) and clearing of
 // the j-side accumulators, every step.  On rebuild steps (status given and
 // the request set) it also fills the slots' types and keys and each 64-slot
-// block's bounding box (one wave per block), from the same positions.
+// block's bounding box (one wave per block), from the same positions, and
+// keeps those positions (tile_ref): on the other steps an atom that has
+// crossed a face since is marked with the image that takes it back
+// (tile_img), which the row lists' image codes assume.
 // One slot s < npad; the wave's 64 lanes hold the 64 slots of one block
 // (the bounding-box reduction is a wave reduction).
 __device__ __forceinline__ void nb_gather_slot(unsigned s, bool rebuild,
@@ -269,9 +286,11 @@ __device__ __forceinline__ void nb_gather_slot(unsigned s, bool rebuild,
                                                unsigned* __restrict__ tile_type,
                                                unsigned* __restrict__ tile_key,
                                                float4* __restrict__ center,
-                                               float4* __restrict__ half) {
-  float4 out;
-  unsigned id = 0u;
+                                               float4* __restrict__ half,
+                                               float4* __restrict__ tile_ref,
+                                               unsigned char* __restrict__ tile_img) {
+  float4 out = make_float4(0.f, 0.f, 0.f, 0.f);
+  unsigned id = 0u, img = HD_IMAGE_NONE;
   if (s < n) {
     HdLattice L = hd_load_lattice(lattice);
     id = sorted_id[s];
@@ -279,10 +298,11 @@ __device__ __forceinline__ void nb_gather_slot(unsigned s, bool rebuild,
     int a, b, c;
     hd_wrap_with_image(p.x, p.y, p.z, a, b, c, L);
     out = p;
-  } else {
-    out = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!rebuild) img = hd_own_image(p, tile_ref[s], L);
   }
   tile_posq[s] = out;
+  tile_img[s] = (unsigned char)img;
+  if (rebuild) tile_ref[s] = out;
   longlong2 z = make_longlong2(0, 0);
   reinterpret_cast<longlong2*>(fpj)[2 * s] = z;
   reinterpret_cast<longlong2*>(fpj)[2 * s + 1] = z;
@@ -302,9 +322,15 @@ __device__ __forceinline__ void nb_gather_slot(unsigned s, bool rebuild,
     hiz = fmaxf(hiz, __shfl_xor(hiz, off));
   }
   if ((threadIdx.x & 63u) == 0) {
+    // the centre is rounded to 1/16 Bohr: the offset of an atom from it is
+    // then exact in f32 whenever the coordinate is at least as large as the
+    // offset (the pair kernel works with those offsets)
     unsigned blk = s >> 6;
-    center[blk] = make_float4(0.5f * (lox + hix), 0.5f * (loy + hiy), 0.5f * (loz + hiz), 0.f);
-    half[blk] = make_float4(0.5f * (hix - lox), 0.5f * (hiy - loy), 0.5f * (hiz - loz), 0.f);
+    float cx = 0.0625f * rintf(8.0f * (lox + hix)), cy = 0.0625f * rintf(8.0f * (loy + hiy)),
+          cz = 0.0625f * rintf(8.0f * (loz + hiz));
+    center[blk] = make_float4(cx, cy, cz, 0.f);
+    half[blk] = make_float4(fmaxf(hix - cx, cx - lox), fmaxf(hiy - cy, cy - loy),
+                            fmaxf(hiz - cz, cz - loz), 0.f);
   }
 }
 
@@ -314,11 +340,13 @@ __global__ void k_tile_gather(const float4* __restrict__ posq, const unsigned* _
                               unsigned n, unsigned npad, const unsigned* status,
                               const unsigned* __restrict__ type, const unsigned* __restrict__ key,
                               unsigned* __restrict__ tile_type, unsigned* __restrict__ tile_key,
-                              float4* __restrict__ center, float4* __restrict__ half) {
+                              float4* __restrict__ center, float4* __restrict__ half,
+                              float4* __restrict__ tile_ref,
+                              unsigned char* __restrict__ tile_img) {
   unsigned s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= npad) return;  // whole waves: npad is a multiple of 64
   nb_gather_slot(s, status && nb_rebuild_due(status), posq, sorted_id, lattice, tile_posq, fpj,
-                 fpj_ew, n, type, key, tile_type, tile_key, center, half);
+                 fpj_ew, n, type, key, tile_type, tile_key, center, half, tile_ref, tile_img);
 }
 
 
@@ -354,8 +382,7 @@ __device__ __forceinline__ float nb_box_dist2(float4 ca, float4 ha, float4 cb, f
 }
 
 // Block-pair candidates: bit (jb % 64) of mask[b * nchunks + jb / 64] is
-// set when j-block jb's box lies within r_search of block b's (jb >= b only
-// for the half list).  Each wave handles (b, chunk of 64 j-blocks) items in
+// set when j-block jb's box lies within r_search of block b's.  Each wave handles (b, chunk of 64 j-blocks) items in
 // a grid-stride loop, so the box tests of a rebuild run at full width
 // instead of as a dependent loop inside each block's wave, while the launch
 // stays small on the steps where the rebuild gate closes it at once.
@@ -365,12 +392,12 @@ __device__ __forceinline__ void nb_block_pair_item(unsigned wv, const float4* __
                                                    const float4* __restrict__ half,
                                                    const HdLattice& L, float rs2,
                                                    unsigned long long* __restrict__ mask,
-                                                   unsigned nblocks, unsigned nchunks, int full) {
+                                                   unsigned nblocks, unsigned nchunks) {
   unsigned lane = threadIdx.x & 63;
   unsigned b = wv / nchunks, c = wv % nchunks;
   unsigned jb = c * 64 + lane;
   bool cand = false;
-  if (jb < nblocks && (full || jb >= b))
+  if (jb < nblocks)
     cand = nb_box_dist2(center[b], half[b], center[jb], half[jb], L) <= rs2;
   unsigned long long m = __ballot(cand);
   if (lane == 0) mask[wv] = m;
@@ -379,14 +406,14 @@ __global__ void __launch_bounds__(256) k_block_pairs(const float4* __restrict__ 
                                                      const float4* __restrict__ half,
                                                      const float* __restrict__ lattice, float rs2,
                                                      unsigned long long* __restrict__ mask,
-                                                     unsigned nblocks, unsigned nchunks, int full,
+                                                     unsigned nblocks, unsigned nchunks,
                                                      const unsigned* status) {
   if (!nb_rebuild_due(status)) return;
   unsigned nwaves = gridDim.x * (blockDim.x >> 6);
   HdLattice L = hd_load_lattice(lattice);
   for (unsigned wv = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; wv < nblocks * nchunks;
        wv += nwaves)
-    nb_block_pair_item(wv, center, half, L, rs2, mask, nblocks, nchunks, full);
+    nb_block_pair_item(wv, center, half, L, rs2, mask, nblocks, nchunks);
 }
 
 // Systems of at most NB_SMALL_ATOMS atoms and NB_SMALL_VOX voxels: the
@@ -489,7 +516,7 @@ __global__ void __launch_bounds__(NB_SMALL_THREADS) k_nb_small(HdNeighborArgs a,
   // blocks in every pass
   for (unsigned s = t; s < a.npad; s += NB_SMALL_THREADS)
     nb_gather_slot(s, rebuild, a.posq, a.sorted_id, a.lattice, a.tile_posq, fpj, fpj_ew, a.n,
-                   a.type, a.key, a.tile_type, a.tile_key, a.center, a.half);
+                   a.type, a.key, a.tile_type, a.tile_key, a.center, a.half, a.tile_ref, a.tile_img);
   if (spl) {
     // SPME spline records from the gathered positions (each thread reads
     // back the slots it wrote)
@@ -501,8 +528,8 @@ __global__ void __launch_bounds__(NB_SMALL_THREADS) k_nb_small(HdNeighborArgs a,
   // the box tests read every block's bounding box from the gather
   const unsigned nblocks = a.npad / 64u, nchunks = (nblocks + 63u) / 64u;
   for (unsigned wv = t >> 6; wv < nblocks * nchunks; wv += NB_SMALL_THREADS / 64u)
-    nb_block_pair_item(wv, a.center, a.half, L, a.rs2, a.block_mask, nblocks, nchunks,
-                       a.atom_lists);
+    nb_block_pair_item(wv, a.center, a.half, L, a.rs2 * NB_BOX_MARGIN, a.block_mask, nblocks,
+                       nchunks);
 }
 
 bool hd_neighbor_small(const HdNeighborArgs& a) {
@@ -551,232 +578,445 @@ __device__ __forceinline__ unsigned nb_collect(const unsigned long long* __restr
   return ncand;
 }
 
-// Build the packed list: one wave per i-block.  The candidate j-blocks
-// (>= b, increasing order) are streamed through the wave one block per step,
-// the next block's atoms loaded while the current one is handled.  A j-atom
-// farther than r_search from the i-block's box cannot hit any i-atom; the
-// others are queued in LDS, and every time 64 are queued each lane tests
-// one queued j-atom against the 64 i-atoms.  Queued j-atoms with at least
-// one hit are appended, in queue order, to a staging buffer flushed 64 at a
-// time.  The entries are therefore the hit j-atoms in (j-block, slot) order:
-// a pure function of the positions.
-#define NB_WAVES 4
-#define NB_CHUNK 4  // candidate blocks whose loads are in flight together
+#define NB_WAVES 4  // waves (i-blocks) per workgroup of the atom-list build
 
-// A j-atom's offset from the i-block centre in the image nearest it, as
-// hd_rel_to_center computes it (FP64 difference less whole box lengths,
-// rounded once), with the image count from an f32 product with the
-// reciprocal box length.  The counts can differ only for an offset within
-// an ulp of half a box length, and such an atom is rejected by the box
-// test in either image (the block lies at least r_search inside the half
-// box on this path).
-__device__ __forceinline__ void nb_rel_to_center(float x, float y, float z, float4 cb,
-                                                 const HdLattice& L, float ilx, float ily,
-                                                 float ilz, float& rx, float& ry, float& rz) {
-  double nx = (double)rintf((x - cb.x) * ilx);
-  double ny = (double)rintf((y - cb.y) * ily);
-  double nz = (double)rintf((z - cb.z) * ilz);
-  rx = (float)(((double)x - (double)cb.x) - (double)L.lx * nx);
-  ry = (float)(((double)y - (double)cb.y) - (double)L.ly * ny);
-  rz = (float)(((double)z - (double)cb.z) - (double)L.lz * nz);
-}
+// Row lists.  A unit is one part of one i-block's neighbourhood: the
+// block's candidate (j-block, periodic image) pairs are dealt out to
+// `parts` units in pieces of 8 atoms, so that small systems still fill the
+// chip.  One workgroup of 8 waves per unit:
+//   1. the candidates from the block-pair mask, each expanded into the
+//      images (of -1, 0, 1 box vectors per axis) whose box lies within
+//      r_search: with an image per j-atom the pair kernel needs no minimum
+//      image, in narrow and tilted boxes too;
+//   2. the j-atoms within r_search of the box of one of the block's 16-atom
+//      quarters, in a fixed order, to the unit's
+//      j-list and to LDS: those of Lennard-Jones-active types from the front
+//      of the list, the others from its back;
+//   3. rows: wave w owns i-atoms 8 w .. 8 w + 7, octet w (coordinates in
+//      scalar registers), queues the j-atoms within r_search of the octet's
+//      box and tests 64 of them at a time against each i-atom; the ballot of the hits gives every hit its place in the row.  A row
+//      holds the hits' LDS byte offsets (16 index) among the active
+//      j-atoms, padded to a multiple of 32 entries common to the wave's 8
+//      rows, then those among the others, padded alike; padding points to
+//      a dummy record past the list.
+// The pair kernel's lane 8 r + s reads entries 4 s .. 4 s + 3 of a 32-entry
+// chunk of row r as one 8-byte load: 64 contiguous bytes per row.
+// Bound by instruction issue (two 8-wave workgroups per CU; a unit's waves
+// spend 55 % of their cycles listing j-atoms and 45 % on the rows): 75 us at
+// 24,576 atoms and a 0.27 nm skin, 190 for the packed tiles' build; 250 us
+// at 196,608 atoms and 0.14 nm, where that took 190.  The list is a pure
+// function of the positions.
+#define NB_PER_WAVE 2u
+#define NB_ROUND (HD_ROW_WAVES * NB_PER_WAVE)
+#define NB_STAGE 96u         // entries of a row staged in LDS: a rest below 32 and 64 hits
+#define NB_WORDS_MAX 512u    // mask words (64 blocks each) with candidates
+#define NB_IMAGES_MAX 1024u  // images listed from 512 blocks at a time
+#define NB_FOLD_MAX_UNITS 1024u  // unit counts whose build also clears the request
 
-// one pass of the 64 x 64 test over the queued j-atoms (lane = queue
-// position); returns whether this lane's j-atom hits any i-atom
-__device__ __forceinline__ bool nb_test_queued(const float4* ipos, float4 pj, unsigned jslot,
-                                               bool jvalid, bool rel, unsigned b, unsigned ni,
-                                               float rs2, const HdLattice& L) {
-  bool hit = false;
-  if (!jvalid) return false;
-  if (rel) {
-#pragma unroll 8
-    for (unsigned m = 0; m < 64; ++m) {
-      float4 a = ipos[m];
-      float dx = a.x - pj.x, dy = a.y - pj.y, dz = a.z - pj.z;
-      float r2 = dx * dx + dy * dy + dz * dz;
-      hit |= (r2 <= rs2) & (m < ni) & ((b * 64 + m) != jslot);
-    }
-  } else {
-#pragma unroll 8
-    for (unsigned m = 0; m < 64; ++m) {
-      float4 a = ipos[m];
-      float dx = a.x - pj.x, dy = a.y - pj.y, dz = a.z - pj.z;
-      hd_min_image(dx, dy, dz, L);
-      float r2 = dx * dx + dy * dy + dz * dz;
-      hit |= (r2 <= rs2) & (m < ni) & ((b * 64 + m) != jslot);
-    }
+__device__ __forceinline__ unsigned nb_scan512(unsigned v, unsigned* wsum, unsigned& total) {
+  const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  unsigned inc = v;
+#pragma unroll
+  for (unsigned off = 1; off < 64; off <<= 1) {
+    unsigned u = __shfl_up(inc, off);
+    if (lane >= off) inc += u;
   }
-  return hit;
+  __syncthreads();  // wsum free for reuse
+  if (lane == 63) wsum[w] = inc;
+  __syncthreads();
+  unsigned before = 0;
+  total = 0;
+#pragma unroll
+  for (unsigned k = 0; k < HD_ROW_WAVES; ++k) {
+    unsigned c = wsum[k];
+    before += k < w ? c : 0u;
+    total += c;
+  }
+  return before + inc - v;
 }
 
-#define NB_FOLD_MAX_BLOCKS 128u  // block counts the folded ordering handles
+// Images (bit = code) of j-block box (cj, hj) within r_search of the
+// i-block's.  Orthorhombic: the images of each axis that are close enough
+// along it, then (almost always one per axis) their combinations.
+__device__ __forceinline__ unsigned nb_images(float4 ci, float4 hi, float4 cj, float4 hj,
+                                              const HdLattice& L, float rs2) {
+  const float dx = cj.x - ci.x, dy = cj.y - ci.y, dz = cj.z - ci.z;
+  unsigned m = 0;
+  if (L.xy == 0.f && L.xz == 0.f && L.yz == 0.f) {
+    float ex[3], ey[3], ez[3];
+    unsigned ok = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      ex[k] = fmaxf(fabsf(dx + (float)(k - 1) * L.lx) - (hi.x + hj.x), 0.f);
+      ey[k] = fmaxf(fabsf(dy + (float)(k - 1) * L.ly) - (hi.y + hj.y), 0.f);
+      ez[k] = fmaxf(fabsf(dz + (float)(k - 1) * L.lz) - (hi.z + hj.z), 0.f);
+      ex[k] *= ex[k];
+      ey[k] *= ey[k];
+      ez[k] *= ez[k];
+      ok |= (ex[k] <= rs2 ? 1u << k : 0u) | (ey[k] <= rs2 ? 8u << k : 0u) |
+            (ez[k] <= rs2 ? 64u << k : 0u);
+    }
+    for (int c = 0; c < 3; ++c) {
+      if (!((ok >> (6 + c)) & 1u)) continue;
+      const float zc = c == 0 ? ez[0] : (c == 1 ? ez[1] : ez[2]);
+      for (int b = 0; b < 3; ++b) {
+        if (!((ok >> (3 + b)) & 1u)) continue;
+        const float yz = zc + (b == 0 ? ey[0] : (b == 1 ? ey[1] : ey[2]));
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+          if (ex[a] + yz <= rs2) m |= 1u << (a + 3 * b + 9 * c);
+      }
+    }
+    return m;
+  }
+  unsigned code = 0;
+  for (int c = -1; c <= 1; ++c)
+    for (int b = -1; b <= 1; ++b)
+      for (int a = -1; a <= 1; ++a, ++code) {
+        float sx = dx + (float)a * L.lx + (float)b * L.xy + (float)c * L.xz;
+        float sy = dy + (float)b * L.ly + (float)c * L.yz;
+        float sz = dz + (float)c * L.lz;
+        if (nb_box_gap2(sx, sy, sz, hi, hj) <= rs2) m |= 1u << code;
+      }
+  return m;
+}
 
-// FOLD (at most NB_FOLD_MAX_BLOCKS blocks): the workgroup that takes the
-// last ticket (*ticket, 0 between launches) also does k_rebuild_clear's
-// work once every block's entry count is written: blocks ordered by entry
-// count, heaviest first (ties by block index), the rebuild request cleared
-// and the rebuild counted.  The order only maps workgroups to blocks in
-// the pair kernel, so any permutation gives the same forces.
+// FOLD (few units): the workgroup that takes the last ticket (*ticket, 0
+// between launches) clears the rebuild request and counts the rebuild once
+// every unit's list is written, in place of k_rebuild_clear; the units of
+// such a system all run at once, so they keep their index order.
 template <bool FOLD>
-__global__ void __launch_bounds__(256) k_build_entries(
-    const float4* __restrict__ tile_posq, const float4* __restrict__ center,
-    const float4* __restrict__ half, const float* __restrict__ lattice, float rs2,
-    const unsigned long long* __restrict__ mask, unsigned nchunks,
-    unsigned* __restrict__ entry_atoms, unsigned* __restrict__ entry_count, unsigned cap,
-    unsigned* __restrict__ max_count, unsigned* status, unsigned n, unsigned nblocks,
-    unsigned* ticket, unsigned* rebuild_count, unsigned* __restrict__ order) {
-  if (!nb_rebuild_due(status)) return;
-  __shared__ float4 ipos[NB_WAVES][64];
-  __shared__ unsigned buf[NB_WAVES][128];
-  __shared__ float4 qpos[NB_WAVES][128];
-  __shared__ unsigned qslot[NB_WAVES][128];
-  __shared__ unsigned cand[NB_WAVES][NB_CAND_MAX];
-  unsigned w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  unsigned b = blockIdx.x * NB_WAVES + w;
-  if (b < nblocks) {
-  HdLattice L = hd_load_lattice(lattice);
-  unsigned islot = b * 64 + lane;
-  float4 pi = tile_posq[islot];
-  if (islot >= n) pi = make_float4(1.0e30f, 1.0e30f, 1.0e30f, 0.f);
-  ipos[w][lane] = pi;
-  __builtin_amdgcn_wave_barrier();
-  float4 cb = center[b], hb = half[b];
-  unsigned ni = min(64u, n - b * 64);
-  // When the block is far from every periodic boundary (orthorhombic box,
-  // L/2 - half extent >= r_search), hold i and j relative to the block
-  // centre with the periodic shift applied once per atom, so each of the
-  // 64 x 64 distance tests is plain arithmetic (no min-image, no division).
-  float rsearch = sqrtf(rs2);
-  bool rel = (L.xy == 0.f && L.xz == 0.f && L.yz == 0.f) && (0.5f * L.lx - hb.x >= rsearch) &&
-             (0.5f * L.ly - hb.y >= rsearch) && (0.5f * L.lz - hb.z >= rsearch);
-  if (rel) {
-    float4 r;
-    hd_rel_to_center(pi.x, pi.y, pi.z, cb.x, cb.y, cb.z, L, r.x, r.y, r.z);
-    r.w = 0.f;
-    ipos[w][lane] = r;
+__global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs a,
+                                                                  unsigned nchunks) {
+  if (!nb_rebuild_due_now(a.status)) return;
+  extern __shared__ float4 jrec[];  // x, y, z relative to the block centre; key
+  __shared__ unsigned words[NB_WORDS_MAX];
+  __shared__ unsigned images[NB_IMAGES_MAX];  // j-block * 32 + image code
+  __shared__ unsigned wsum[HD_ROW_WAVES];
+  __shared__ unsigned wcnt[2][HD_ROW_WAVES];
+  __shared__ unsigned s_cost, s_need;
+  __shared__ float4 quart[4][2];
+  __shared__ unsigned short ring[HD_ROW_WAVES][128];
+  __shared__ __align__(16) unsigned short stage[HD_ROW_WAVES][HD_ROW_I][NB_STAGE];
+  const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  const unsigned unit = blockIdx.x;
+  const unsigned b = unit / a.parts, part = unit - b * a.parts;
+  HdLattice L = hd_load_lattice(a.lattice);
+  const float4 cb = a.center[b], hb = a.half[b];
+  const float rs2 = a.rs2 * NB_BOX_MARGIN, rs2p = a.rs2 * NB_ROW_MARGIN;
+  if (t == 0) s_cost = s_need = 0u;
+  // 1. the mask words with candidates
+  unsigned nw = 0;
+  for (unsigned base = 0; base < nchunks; base += HD_ROW_THREADS) {
+    const unsigned c = base + t;
+    const bool nz = c < nchunks && a.block_mask[(size_t)b * nchunks + c] != 0ull;
+    unsigned total;
+    const unsigned o = nw + nb_scan512(nz ? 1u : 0u, wsum, total);
+    if (nz && o < NB_WORDS_MAX) words[o] = c;
+    nw += total;
   }
-  bool too_many = false;
-  unsigned ncand = nb_collect(mask, b, nchunks, lane, cand[w], &too_many);
-  __builtin_amdgcn_wave_barrier();
-  const float filx = 1.0f / L.lx, fily = 1.0f / L.ly, filz = 1.0f / L.lz;
-  unsigned nbuf = 0, nent = 0, nq = 0;
-  unsigned* out = entry_atoms + (size_t)b * cap * 64;
-  // test 64 queued atoms at a time (the remainder after the last block)
-  auto drain = [&](bool last) {
-    while (nq >= 64 || (last && nq > 0)) {
-      bool qvalid = lane < nq;
-      float4 qp = qpos[w][lane];
-      unsigned qs = qvalid ? qslot[w][lane] : HD_SENTINEL;
-      bool hit = nb_test_queued(ipos[w], qp, qs, qvalid, rel, b, ni, rs2, L);
-      unsigned rem = nq > 64 ? nq - 64 : 0;
-      float4 rp = qpos[w][64 + (lane < rem ? lane : 0)];
-      unsigned rsl = qslot[w][64 + (lane < rem ? lane : 0)];
-      __builtin_amdgcn_wave_barrier();
-      if (lane < rem) {
-        qpos[w][lane] = rp;
-        qslot[w][lane] = rsl;
+  bool too_many = nw > NB_WORDS_MAX;
+  nw = min(nw, NB_WORDS_MAX);
+  // boxes, relative to the block centre, of the block's 16-atom quarters
+  // (which j-atoms to list) and of this wave's 8-atom octet (which of them
+  // to test); lane = atom
+  float4 oc, oh;
+  {
+    const unsigned islot = b * 64u + lane;
+    float4 p = a.tile_posq[islot];
+    hd_rel_image(p.x, p.y, p.z, cb, HD_IMAGE_NONE, HD_IMAGE_NONE, L, p.x, p.y, p.z);
+    const bool v = islot < a.n;
+    float lx = v ? p.x : 3.0e18f, ly = v ? p.y : 3.0e18f, lz = v ? p.z : 3.0e18f;
+    float hx = v ? p.x : -3.0e18f, hy = v ? p.y : -3.0e18f, hz = v ? p.z : -3.0e18f;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) {
+      if (off == 8) {
+        // octet w's box (no atoms: lo > hi, a negative half that nothing
+        // reaches)
+        const int src = (int)(w * 8u);
+        const float ax = __shfl(lx, src), bx = __shfl(hx, src), ay = __shfl(ly, src),
+                    by = __shfl(hy, src), az = __shfl(lz, src), bz = __shfl(hz, src);
+        oc = make_float4(0.5f * (ax + bx), 0.5f * (ay + by), 0.5f * (az + bz), 0.f);
+        oh = make_float4(0.5f * (bx - ax), 0.5f * (by - ay), 0.5f * (bz - az), 0.f);
       }
-      nq = rem;
-      unsigned long long hmask = __ballot(hit);
-      if (hit) {
-        unsigned pos = nbuf + __popcll(hmask & hd_lane_mask_lt());
-        buf[w][pos] = qs;
-      }
-      nbuf += __popcll(hmask);
-      __builtin_amdgcn_wave_barrier();
-      if (nbuf >= 64) {
-        if (nent < cap) out[(size_t)nent * 64 + lane] = buf[w][lane];
-        ++nent;
-        unsigned brem = nbuf - 64;
-        unsigned v = (lane < brem) ? buf[w][64 + lane] : 0u;
-        __builtin_amdgcn_wave_barrier();
-        if (lane < brem) buf[w][lane] = v;
-        nbuf = brem;
-        __builtin_amdgcn_wave_barrier();
-      }
+      lx = fminf(lx, __shfl_xor(lx, off)); hx = fmaxf(hx, __shfl_xor(hx, off));
+      ly = fminf(ly, __shfl_xor(ly, off)); hy = fmaxf(hy, __shfl_xor(hy, off));
+      lz = fminf(lz, __shfl_xor(lz, off)); hz = fmaxf(hz, __shfl_xor(hz, off));
     }
+    if (w == 0 && (lane & 15u) == 0u) {
+      quart[lane >> 4][0] =
+          make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz), 0.f);
+      quart[lane >> 4][1] =
+          make_float4(0.5f * (hx - lx), 0.5f * (hy - ly), 0.5f * (hz - lz), 0.f);
+    }
+  }
+  __syncthreads();
+  // 2. j-atoms.  Eight mask words at a time (thread = block): the candidate
+  // blocks' images are listed, and the unit takes the 8-atom pieces
+  // 8 e + (lane / 8) of the images e that are `part` modulo parts (a power
+  // of two).  Rounds of 16 images, two per wave and the next two in flight;
+  // the list keeps the images' order, active types from the front, the
+  // others from the back.
+  const unsigned pm = a.parts - 1u;
+  unsigned nact = 0, nina = 0, e0 = 0, buf = 0;
+  for (unsigned w0 = 0; w0 < nw; w0 += HD_ROW_WAVES) {
+    unsigned ne;
+    {
+      unsigned m = 0, jb = 0;
+      if (w0 + w < nw) {
+        const unsigned c = words[w0 + w];
+        jb = c * 64u + lane;
+        if ((a.block_mask[(size_t)b * nchunks + c] >> lane) & 1ull)
+          m = nb_images(cb, hb, a.center[jb], a.half[jb], L, rs2);
+      }
+      unsigned o = nb_scan512((unsigned)__popc(m), wsum, ne);
+      for (; m; m &= m - 1u, ++o)
+        if (o < NB_IMAGES_MAX) images[o] = jb * 32u + (unsigned)__builtin_ctz(m);
+      too_many = too_many || ne > NB_IMAGES_MAX;
+      ne = min(ne, NB_IMAGES_MAX);
+    }
+    __syncthreads();
+    float4 np[NB_PER_WAVE];
+    unsigned nt[NB_PER_WAVE], nk[NB_PER_WAVE];
+    auto load = [&](unsigned r0) {
+#pragma unroll
+      for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
+        const unsigned it = r0 + w * NB_PER_WAVE + u;
+        // past the end: block 0, not used
+        const unsigned sl = (it < ne ? images[it] >> 5 : 0u) * 64u + lane;  // < npad
+        np[u] = a.tile_posq[sl];
+        nt[u] = a.tile_type[sl];
+        nk[u] = a.tile_key[sl];
+      }
+    };
+    load(0u);
+    for (unsigned r0 = 0; r0 < ne; r0 += NB_ROUND) {
+      float4 p[NB_PER_WAVE];
+      unsigned js[NB_PER_WAVE], ca = 0, ci = 0;
+      unsigned long long ma[NB_PER_WAVE], mi[NB_PER_WAVE];
+#pragma unroll
+      for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
+        const unsigned it = r0 + w * NB_PER_WAVE + u;
+        const unsigned img = it < ne ? images[it] : HD_IMAGE_NONE, slot = (img >> 5) * 64u + lane;
+        hd_rel_image(np[u].x, np[u].y, np[u].z, cb, img & 31u, HD_IMAGE_NONE, L, p[u].x, p[u].y,
+                     p[u].z);
+        p[u].w = __uint_as_float(nk[u]);
+        js[u] = slot | ((img & 31u) << HD_ROW_SLOT_BITS);
+        bool near = false;
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+          const float4 qc = quart[o][0], qh = quart[o][1];
+          near = near || nb_box_gap2(p[u].x - qc.x, p[u].y - qc.y, p[u].z - qc.z, qh,
+                                     make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2;
+        }
+        near = near && it < ne && slot < a.n && (((e0 + it) * 8u + (lane >> 3)) & pm) == part;
+        const unsigned long long mn = __ballot(near),
+                                 mt = __ballot((a.active_types >> nt[u]) & 1u);
+        ma[u] = mn & mt;
+        mi[u] = mn & ~mt;
+        ca += (unsigned)__popcll(ma[u]);
+        ci += (unsigned)__popcll(mi[u]);
+      }
+      load(r0 + NB_ROUND);
+      if (lane == 0) wcnt[buf][w] = ca | (ci << 16);
+      __syncthreads();  // two buffers: the next round's counts land elsewhere
+      unsigned before = 0, all = 0;
+#pragma unroll
+      for (unsigned v = 0; v < HD_ROW_WAVES; ++v) {
+        const unsigned cv = wcnt[buf][v];
+        if (v < w) before += cv;
+        all += cv;
+      }
+      buf ^= 1u;
+      unsigned ja = nact + (before & 0xFFFFu), ji = nina + (before >> 16);
+#pragma unroll
+      for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
+        const bool act = __builtin_amdgcn_inverse_ballot_w64(ma[u]);
+        if (__builtin_amdgcn_inverse_ballot_w64(ma[u] | mi[u])) {
+          const unsigned k = act ? ja + hd_rank(ma[u]) : ji + hd_rank(mi[u]);
+          if (k < a.jcap) {
+            const unsigned o = act ? k : a.jcap - 1u - k;
+            jrec[o] = p[u];
+            a.jslot[(size_t)unit * a.jcap + o] = js[u];
+          }
+        }
+        ja += (unsigned)__popcll(ma[u]);
+        ji += (unsigned)__popcll(mi[u]);
+      }
+      nact += all & 0xFFFFu;
+      nina += all >> 16;
+    }
+    e0 += ne;
+  }
+  __syncthreads();
+  const unsigned need_j = nact + nina;
+  nact = min(nact, a.jcap);
+  nina = min(nina, a.jcap - nact);  // less on overflow, flagged below
+  // 3. rows
+  const unsigned rcap = a.rcap;
+  unsigned short* rows = a.rows + ((size_t)unit * 64u + w * HD_ROW_I) * rcap;
+  const unsigned short dummy = (unsigned short)(a.jcap << 4);
+  // r^2 <= rs^2 as j.(j - 2 i) <= rs^2 - i.i: three multiply-adds per pair.
+  // The terms reach (r_search + half extent)^2, so the test is wider by
+  // their rounding.
+  float sx[HD_ROW_I], sy[HD_ROW_I], sz[HD_ROW_I], sr[HD_ROW_I];
+  unsigned sk[HD_ROW_I], cnt[HD_ROW_I];
+  {
+    unsigned islot = b * 64u + w * HD_ROW_I + (lane & 7u);
+    float4 p = a.tile_posq[islot];
+    unsigned key = a.tile_key[islot];
+    hd_rel_image(p.x, p.y, p.z, cb, HD_IMAGE_NONE, HD_IMAGE_NONE, L, p.x, p.y, p.z);
+    const float reach = sqrtf(rs2) + hb.x + hb.y + hb.z;
+    // no j-atom is within reach of a slot without atom
+    float lim = islot < a.n ? rs2p + 2.0e-6f * reach * reach - (p.x * p.x + p.y * p.y + p.z * p.z)
+                            : -3.0e38f;
+#pragma unroll
+    for (int q = 0; q < HD_ROW_I; ++q) {
+      sx[q] = -2.0f * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.x), q));
+      sy[q] = -2.0f * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.y), q));
+      sz[q] = -2.0f * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.z), q));
+      sr[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lim), q));
+      sk[q] = (unsigned)__builtin_amdgcn_readlane((int)key, q);
+      cnt[q] = 0u;
+    }
+  }
+  unsigned done = 0;  // entries of every row so far (a multiple of 32)
+  unsigned nact_chunks = 0;
+  // the j-atoms near this wave's octet are queued, and tested 64 at a time
+  // (lane = queue position) against its 8 i-atoms
+  unsigned short* queue = ring[w];
+  unsigned short(*st)[NB_STAGE] = stage[w];
+  const unsigned fq = lane >> 3, fs = (lane & 7u) * 4u;  // row and entries of the lane's stores
+  unsigned short* frow = rows + fq * rcap + fs;
+  // Hits are staged in LDS behind the row's rest (cnt mod 32 entries) and
+  // leave in whole chunks of 32, eight lanes of 8 bytes per row: storing
+  // each hit by itself, a 2-byte store per lane, took as long as all the
+  // rest of the build together.
+  auto flush = [&](unsigned before, unsigned pops) {
+    // lane q < 8: row q's entries before the group, and those added
+    const unsigned c0 = __shfl(before, fq), add = __shfl(pops, fq);
+    const unsigned rest = c0 & (HD_ROW_CHUNK - 1u), nf = (rest + add) / HD_ROW_CHUNK;
+    const unsigned base = c0 - rest;
+    hd_wave_sync();
+#pragma unroll
+    for (unsigned c = 0; c < 2; ++c)
+      if (c < nf && base + c * HD_ROW_CHUNK < rcap)
+        *reinterpret_cast<hd_u32x2*>(frow + base + c * HD_ROW_CHUNK) =
+            *reinterpret_cast<const hd_u32x2*>(&st[fq][c * HD_ROW_CHUNK + fs]);
+    hd_u32x2 tail = {0u, 0u};
+    if (nf) tail = *reinterpret_cast<const hd_u32x2*>(&st[fq][nf * HD_ROW_CHUNK + fs]);
+    hd_wave_sync();
+    if (nf) *reinterpret_cast<hd_u32x2*>(&st[fq][fs]) = tail;
+    hd_wave_sync();
   };
-  // the candidate blocks' atoms are loaded NB_CHUNK blocks at a time, the
-  // next group while the current one is queued and tested
-  float4 pn[NB_CHUNK];
+  unsigned cntv = 0u;  // lane q < 8: row q's entries
+  auto test = [&](unsigned nq) {
+    const bool kv = lane < nq;
+    const unsigned k = queue[kv ? lane : 0u];  // idle lanes: a written record, too far off below
+    const float4 r = jrec[k];
+    const float j2 = kv ? r.x * r.x + r.y * r.y + r.z * r.z : 3.0e38f;
+    const unsigned jkey = __float_as_uint(r.w);
+    const unsigned before = cntv;
+    unsigned pops = 0u;
 #pragma unroll
-  for (unsigned u = 0; u < NB_CHUNK; ++u)
-    pn[u] = (u < ncand) ? tile_posq[cand[w][u] * 64 + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
-  for (unsigned c0 = 0; c0 < ncand; c0 += NB_CHUNK) {
-    float4 pc[NB_CHUNK];
-#pragma unroll
-    for (unsigned u = 0; u < NB_CHUNK; ++u) {
-      pc[u] = pn[u];
-      unsigned cn = c0 + NB_CHUNK + u;
-      if (cn < ncand) pn[u] = tile_posq[cand[w][cn] * 64 + lane];
+    for (int q = 0; q < HD_ROW_I; ++q) {
+      const float d = fmaf(r.x, sx[q], fmaf(r.y, sy[q], fmaf(r.z, sz[q], j2)));
+      const unsigned long long m =
+          __ballot(d <= sr[q]) & __ballot((jkey - sk[q] + a.excl_span) > 2u * a.excl_span);
+      if (__builtin_amdgcn_inverse_ballot_w64(m))
+        st[q][(cnt[q] & (HD_ROW_CHUNK - 1u)) + hd_rank(m)] = (unsigned short)(k << 4);
+      const unsigned add = (unsigned)__popcll(m);
+      pops = lane == (unsigned)q ? add : pops;
+      cnt[q] += add;
     }
-#pragma unroll
-    for (unsigned u = 0; u < NB_CHUNK; ++u) {
-      if (c0 + u >= ncand) break;
-      unsigned jb = cand[w][c0 + u];
-      unsigned jslot = jb * 64 + lane;
-      bool jvalid = jslot < n;
-      float4 pj = pc[u];
-      // distance from the j-atom to the i-block's box
-      float dx, dy, dz;
-      if (rel) {
-        nb_rel_to_center(pj.x, pj.y, pj.z, cb, L, filx, fily, filz, dx, dy, dz);
-        pj.x = dx; pj.y = dy; pj.z = dz;
-      } else {
-        dx = pj.x - cb.x; dy = pj.y - cb.y; dz = pj.z - cb.z;
-        hd_min_image(dx, dy, dz, L);
+    cntv += pops;
+    flush(before, pops);
+  };
+  for (int seg = 0; seg < 2; ++seg) {
+    const unsigned nk = seg ? nina : nact;
+    unsigned nq = 0;
+    for (unsigned k0 = 0; k0 < nk; k0 += 64u) {
+      const unsigned k = k0 + lane, o = seg ? a.jcap - 1u - k : k;
+      bool near = false;
+      if (k < nk) {
+        const float4 p = jrec[o];
+        near = nb_box_gap2(p.x - oc.x, p.y - oc.y, p.z - oc.z, oh,
+                           make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2;
       }
-      float ex = fmaxf(fabsf(dx) - hb.x, 0.f), ey = fmaxf(fabsf(dy) - hb.y, 0.f),
-            ez = fmaxf(fabsf(dz) - hb.z, 0.f);
-      bool near = jvalid && (ex * ex + ey * ey + ez * ez <= rs2);
-      unsigned long long nmask = __ballot(near);
-      if (near) {
-        unsigned pos = nq + __popcll(nmask & hd_lane_mask_lt());
-        qpos[w][pos] = pj;
-        qslot[w][pos] = jslot;
+      const unsigned long long m = __ballot(near);
+      if (near) queue[nq + hd_rank(m)] = (unsigned short)o;
+      nq += (unsigned)__popcll(m);
+      hd_wave_sync();
+      if (nq >= 64u) {
+        test(64u);
+        const unsigned short rest = queue[64u + lane];
+        hd_wave_sync();
+        nq -= 64u;
+        if (lane < nq) queue[lane] = rest;
+        hd_wave_sync();
       }
-      nq += __popcll(nmask);
-      __builtin_amdgcn_wave_barrier();
-      drain(false);
     }
+    if (nq) test(nq);
+    unsigned mx = 0;
+#pragma unroll
+    for (int q = 0; q < HD_ROW_I; ++q) mx = max(mx, cnt[q]);
+    done = max(done, (mx + HD_ROW_CHUNK - 1u) / HD_ROW_CHUNK * HD_ROW_CHUNK);
+    // the rows' rests padded to a chunk, then whole chunks of padding
+    {
+      const unsigned before = cntv;
+      cntv = done;
+#pragma unroll
+      for (int q = 0; q < HD_ROW_I; ++q) {
+        const unsigned rest = cnt[q] & (HD_ROW_CHUNK - 1u);
+        if (lane >= rest && lane < HD_ROW_CHUNK) st[q][lane] = dummy;
+        cnt[q] = done;
+      }
+      hd_wave_sync();
+      const unsigned c0 = __shfl(before, fq), rest = c0 & (HD_ROW_CHUNK - 1u);
+      unsigned base = c0 - rest;
+      if (rest && base < rcap)
+        *reinterpret_cast<hd_u32x2*>(frow + base) = *reinterpret_cast<const hd_u32x2*>(&st[fq][fs]);
+      base += rest ? HD_ROW_CHUNK : 0u;
+      const unsigned d2 = (unsigned)dummy * 0x10001u;
+      for (; base < min(done, rcap); base += HD_ROW_CHUNK)
+        *reinterpret_cast<hd_u32x2*>(frow + base) = hd_u32x2{d2, d2};
+      hd_wave_sync();
+    }
+    if (seg == 0) nact_chunks = done / HD_ROW_CHUNK;
   }
-  drain(true);
-  if (nbuf > 0) {
-    if (nent < cap) out[(size_t)nent * 64 + lane] = (lane < nbuf) ? buf[w][lane] : HD_SENTINEL;
-    ++nent;
-  }
+  const unsigned cap_chunks = a.rcap / HD_ROW_CHUNK;
+  const unsigned nchunk = done / HD_ROW_CHUNK;
   if (lane == 0) {
-    entry_count[b] = min(nent, cap);
-    atomicMax(max_count, nent);
-    if (nent > cap || too_many) atomicOr(status, NB_STATUS_OVERFLOW);
-    else if (4 * nent > 3 * cap) atomicOr(status, NB_STATUS_HIGHWATER);
+    a.rowhdr[unit * HD_ROW_WAVES + w] =
+        min(nact_chunks, cap_chunks) | (min(nchunk, cap_chunks) << 16);
+    atomicAdd(&s_cost, nchunk);
+    atomicMax(&s_need, done);
   }
-  }  // b < nblocks
+  __syncthreads();
+  if (t == 0) {
+    a.entry_count[unit] = s_cost;
+    a.jcount[unit] = nact | (nina << 16);
+    // global maxima: device atomics on one word queue up (about 20 ns each,
+    // a millisecond for every wave of a large system), so a unit reads the
+    // word first and only raises it
+    const unsigned need_r = s_need;
+    if (need_r > *(volatile unsigned*)a.max_count) atomicMax(a.max_count, need_r);
+    if (need_j > *(volatile unsigned*)a.max_j) atomicMax(a.max_j, need_j);
+    unsigned bits = 0u;
+    if (need_r > rcap || need_j > a.jcap || too_many) bits = NB_STATUS_OVERFLOW;
+    else if (4u * need_r > 3u * rcap ||
+             (a.parts > 1u ? 4u * need_j > 3u * a.jcap : 16u * need_j > 15u * a.jcap))
+      bits = NB_STATUS_HIGHWATER;
+    if (bits & ~*(volatile unsigned*)a.status) atomicOr(a.status, bits);
+  }
   if (!FOLD) return;
-  __shared__ unsigned s_last;
-  __syncthreads();
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     __threadfence();
-    s_last = atomicAdd(ticket, 1u) == gridDim.x - 1u ? 1u : 0u;
-  }
-  __syncthreads();
-  if (!s_last) return;
-  __threadfence();  // every block's counts and status bits are visible
-  __shared__ unsigned s_cnt[NB_FOLD_MAX_BLOCKS];
-  for (unsigned i = threadIdx.x; i < nblocks; i += blockDim.x) s_cnt[i] = entry_count[i];
-  __syncthreads();
-  for (unsigned i = threadIdx.x; i < nblocks; i += blockDim.x) {
-    unsigned ci = s_cnt[i], pos = 0;
-    for (unsigned j = 0; j < nblocks; ++j) {
-      unsigned cj = s_cnt[j];
-      pos += (cj > ci || (cj == ci && j < i)) ? 1u : 0u;
+    if (atomicAdd(a.build_ticket, 1u) == gridDim.x - 1u) {
+      atomicAnd(a.status, ~(NB_STATUS_REBUILD | NB_STATUS_FORCE));
+      atomicAdd(a.rebuild_count, 1u);
+      atomicExch(a.build_ticket, 0u);
     }
-    order[pos] = i;
-  }
-  if (threadIdx.x == 0) {
-    atomicAnd(status, ~(NB_STATUS_REBUILD | NB_STATUS_FORCE));
-    atomicAdd(rebuild_count, 1u);
-    atomicExch(ticket, 0u);
   }
 }
 
@@ -882,10 +1122,11 @@ __global__ void __launch_bounds__(256) k_build_alist(
 // End of a rebuild: remember the reference positions and clear the
 // rebuild request bits (sticky overflow/high-water bits stay for the host).
 
-// Clears the rebuild request and, on rebuild steps, orders the blocks by
-// entry count, heaviest first, as the pair kernel's workgroup order: block
-// costs vary about twofold, and a heavy block dispatched last runs alone at
-// the end of the launch.  One workgroup: a histogram of the counts, suffix
+// Clears the rebuild request and, on rebuild steps, orders the pair
+// kernel's work units (blocks in the atom-list mode, whose kernel takes them
+// in index order) by row chunks, heaviest first: unit costs vary about
+// twofold, and a heavy unit dispatched last runs alone at the end of the
+// launch.  One workgroup: a histogram of the counts, suffix
 // sums, a scatter (the order among equal counts is arbitrary; the forces do
 // not depend on it, their sums being integer).
 #define NB_ORDER_BINS 1024u
@@ -966,17 +1207,19 @@ void hd_launch_neighbor_update(hipStream_t st, const HdNeighborArgs& a, bool che
 
 void hd_launch_tile_gather(hipStream_t st, const float4* posq, const unsigned* sorted_id,
                            const float* lattice, float4* tile_posq, long long* fpj,
-                           long long* fpj_ew, unsigned n, unsigned npad) {
+                           long long* fpj_ew, unsigned n, unsigned npad, float4* tile_ref,
+                           unsigned char* tile_img) {
   hipLaunchKernelGGL(k_tile_gather, dim3(cdiv(npad, 256)), dim3(256), 0, st, posq, sorted_id,
                      lattice, tile_posq, fpj, fpj_ew, n, npad, nullptr, nullptr, nullptr,
-                     nullptr, nullptr, nullptr, nullptr);
+                     nullptr, nullptr, nullptr, nullptr, tile_ref, tile_img);
 }
 
 void hd_launch_tile_gather_rebuild(hipStream_t st, const HdNeighborArgs& a, long long* fpj,
                                    long long* fpj_ew) {
   hipLaunchKernelGGL(k_tile_gather, dim3(cdiv(a.npad, 256)), dim3(256), 0, st, a.posq,
                      a.sorted_id, a.lattice, a.tile_posq, fpj, fpj_ew, a.n, a.npad, a.status,
-                     a.type, a.key, a.tile_type, a.tile_key, a.center, a.half);
+                     a.type, a.key, a.tile_type, a.tile_key, a.center, a.half, a.tile_ref,
+                     a.tile_img);
 }
 
 unsigned hd_block_pair_chunks(unsigned nblocks) { return cdiv(nblocks, 64); }
@@ -984,29 +1227,25 @@ unsigned hd_block_pair_chunks(unsigned nblocks) { return cdiv(nblocks, 64); }
 void hd_launch_neighbor_build(hipStream_t st, const HdNeighborArgs& a, bool block_pairs,
                               bool fold_clear) {
   unsigned nblocks = a.npad / 64;
-  const bool fold = fold_clear && !a.atom_lists && nblocks <= NB_FOLD_MAX_BLOCKS;
+  const unsigned units = a.atom_lists ? nblocks : nblocks * a.parts;
+  const bool fold = fold_clear && !a.atom_lists && units <= NB_FOLD_MAX_UNITS;
+  const size_t lds = (size_t)a.jcap * sizeof(float4);
   unsigned nchunks = hd_block_pair_chunks(nblocks);
   unsigned pair_waves = min(nblocks * nchunks, (unsigned)NB_PAIR_WAVES);
   if (block_pairs)
     hipLaunchKernelGGL(k_block_pairs, dim3(cdiv(pair_waves * 64, 256)), dim3(256), 0, st,
-                       a.center, a.half, a.lattice, a.rs2, a.block_mask, nblocks, nchunks,
-                       a.atom_lists, a.status);
+                       a.center, a.half, a.lattice, a.rs2 * NB_BOX_MARGIN, a.block_mask, nblocks,
+                       nchunks, a.status);
   if (a.atom_lists)
     hipLaunchKernelGGL(k_build_alist, dim3(cdiv(nblocks, NB_WAVES)), dim3(64 * NB_WAVES), 0, st,
                        a.tile_posq, a.tile_key, a.excl_span, a.center, a.half, a.lattice, a.rs2,
                        a.block_mask, nchunks, a.entry_atoms, a.entry_count, a.cap, a.max_count,
                        a.status, a.n, nblocks);
   else if (fold)
-    hipLaunchKernelGGL(k_build_entries<true>, dim3(cdiv(nblocks, NB_WAVES)), dim3(64 * NB_WAVES),
-                       0, st, a.tile_posq, a.center, a.half, a.lattice, a.rs2, a.block_mask,
-                       nchunks, a.entry_atoms, a.entry_count, a.cap, a.max_count, a.status, a.n,
-                       nblocks, a.build_ticket, a.rebuild_count, a.block_order);
+    hipLaunchKernelGGL(k_build_rows<true>, dim3(units), dim3(HD_ROW_THREADS), lds, st, a, nchunks);
   else
-    hipLaunchKernelGGL(k_build_entries<false>, dim3(cdiv(nblocks, NB_WAVES)), dim3(64 * NB_WAVES),
-                       0, st, a.tile_posq, a.center, a.half, a.lattice, a.rs2, a.block_mask,
-                       nchunks, a.entry_atoms, a.entry_count, a.cap, a.max_count, a.status, a.n,
-                       nblocks, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(k_build_rows<false>, dim3(units), dim3(HD_ROW_THREADS), lds, st, a, nchunks);
   if (!fold)
     hipLaunchKernelGGL(k_rebuild_clear, dim3(1), dim3(NB_ORDER_BINS), 0, st, a.status,
-                       a.rebuild_count, a.entry_count, nblocks, a.block_order);
+                       a.rebuild_count, a.entry_count, units, a.block_order);
 }

@@ -1,36 +1,23 @@
-// Fused Lennard-Jones + real-space Ewald pair forces over the packed
-// 64-atom cluster list (gfx950, wave64).
+// Fused Lennard-Jones + real-space Ewald pair forces over the row lists and
+// the per-atom lists, and the bonded terms (gfx950, wave64).
 //
 // Reference: the JIT-composed packed pair kernel
 // (src/forces/jit_composed.rs:1490-1838) with the LJ functor
 // (src/forces/lj.rs:225-335) and the SPME real-space functor
 // (src/forces/spme.rs:708-783).  Kept: per-pair arithmetic (f32, Hastings
-// erfc A&S 7.1.26, optional cubic LJ switch), per-entry f32 sums folded
-// into i64 fixed point at 2^48 with truncation, Newton's third law with the
-// j-side suppressed for j-atoms that belong to the i-block, per-atom energy
-// and virial split half/half.
+// erfc A&S 7.1.26, optional cubic LJ switch), f32 partial sums folded into
+// i64 fixed point at 2^48 with truncation, per-atom energy and virial split
+// half/half.  Exclusions (|key_i - key_j| <= span) are applied when the
+// lists are built.
 //
-// MI355X design:
-//   * one workgroup of 4 waves per 64-atom i-block; lane = i-atom; the 64
-//     j-atoms of an entry rotate through the wave with DPP wave_rol:1
-//     (a VALU modifier, no LDS round trip) in 64 lock-step steps;
-//   * i-side sums stay in registers across entries, are combined across the
-//     4 waves in LDS and stored once with a plain store (no atomics, no
-//     clearing pass); only the j-side uses i64 atomics;
-//   * the LJ type-pair row of the i-atom is held in registers (<= 4 types)
-//     and selected per pair, so the inner loop touches no memory;
-//   * exclusions by key: a pair is excluded when the atoms' keys differ by
-//     at most a span.  Span 0 with one key per molecule excludes every
-//     intra-molecule pair of a rigid group, as the reference derives them
-//     (src/forces/topology.rs:1225-1245); keys chain * stride + bead index
-//     with span 2 exclude the 1-2 and 1-3 pairs of linear chains.  The
-//     atom's self pair is excluded the same way;
-//   * when the box is orthorhombic and wide enough, every j-atom is shifted
-//     once per entry to the image nearest the i-block centre, so the inner
-//     loop needs no minimum-image arithmetic (the single-periodic-copy path,
-//     jit_composed.rs:1565-1600); both i and j are then held relative to
-//     the block centre (shift computed in FP64, rounded once), which keeps
-//     the f32 pair displacement accurate in boxes of 100+ Bohr.
+// MI355X design: every pair is evaluated from both sides, which costs twice
+// the useful pairs but leaves no j-side sums to rotate, reduce or add with
+// atomics, and lets a list hold exactly the pairs within the search radius:
+// (r_search / r_c)^3 x 2 slots per useful pair and the rows' padding, 3.4 on
+// water at a 0.14 nm skin where packed 64 x 64 tiles evaluated 5.2.  The
+// gather that such lists need runs out of LDS: the i-atoms of a 64-atom
+// block share one neighbourhood (about 1,700 j-atoms of water at that skin,
+// 27 KB), staged once per block; 16-bit list entries are LDS byte offsets.
 #include "hd_device.h"
 #include "hd_kernels.h"
 
@@ -45,10 +32,9 @@ struct PairParams {
   float inv_delta[PAIR_MAXT * PAIR_MAXT];  // 1/(rc^2 - rs^2), 0 when no switch
   int ntypes;
   float kc, alpha, coul_rc2;  // coul_rc2 < 0 disables the Coulomb term
-  float rmax2;
-  float spc_margin;  // minimum (L/2 - half_extent) that enables the shifted path
-  unsigned excl_span;  // |key_i - key_j| <= excl_span excludes the pair
-  int ortho;           // the box has no tilt
+  int ortho;  // the box has no tilt
+  float reach;  // of a list beyond its block's box, with what atoms move
+  int active_type;  // the LJ-active type when there is only one
   // 1: one cutoff for every interacting type pair and Coulomb, no switch;
   // 2: LJ only (no Coulomb), one cutoff for every interacting type pair, no
   // switch; 0: neither (the general loop)
@@ -57,32 +43,6 @@ struct PairParams {
   float cg;  // -alpha^2 log2(e): exp(-(alpha r)^2) = exp2(cg r^2)
   float pa;  // 0.3275911 alpha, the Hastings t = 1 / (1 + pa r)
 };
-
-// 32768-bit map of the i-block's keys widened by the exclusion span, used
-// to skip the per-pair key test in entries with no excludable j-atom; with
-// a wider span every entry runs the test
-#define PAIR_KEYMAP_WORDS 1024
-#define PAIR_KEYMAP_SPAN 8
-
-// One wave's copy of the current entry's j-atoms for the regrouped loop,
-// written twice over so that step t reads record lane + t with no wrap:
-// positions (block-centre relative) and charges; the LJ force coefficients
-// (12 c12, 6 c6) of the j-atom against each i type, so a lane reads its own
-// type's row with no per-pair select; types (energy steps) and keys.
-template <int NT>
-struct PairJStage {
-  float4 pq[128];
-  float2 lj[NT > 0 ? NT : 1][128];
-  unsigned type[128];
-  unsigned key[128];
-};
-
-// Orders one wave's LDS writes before its lanes read each other's records.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The i-atom's row of the LJ type-pair table, held in VGPRs for the whole
 // kernel.  NT = table width (1, 2 or 4).  Each value passes through an
@@ -196,24 +156,6 @@ __device__ __forceinline__ LjRow<NT> load_row(const PairParams& P, unsigned ityp
   }
 }
 
-// The j-atom's offset from the block centre in the image nearest it, as
-// hd_rel_to_center computes it (FP64 difference less a whole number of box
-// lengths, rounded once), with the image count taken from an f32 product
-// with the reciprocal box length instead of an FP64 division.  On the
-// shifted path every staged j-atom lies within the search radius plus the
-// block half-extent of the centre, at least the skin away from half a box
-// length, so the f32 count is the FP64 one.
-__device__ __forceinline__ void pair_rel_to_center(float x, float y, float z, float4 cb,
-                                                   const HdLattice& L, float ilx, float ily,
-                                                   float ilz, float& rx, float& ry, float& rz) {
-  double nx = (double)rintf((x - cb.x) * ilx);
-  double ny = (double)rintf((y - cb.y) * ily);
-  double nz = (double)rintf((z - cb.z) * ilz);
-  rx = (float)(((double)x - (double)cb.x) - (double)L.lx * nx);
-  ry = (float)(((double)y - (double)cb.y) - (double)L.ly * ny);
-  rz = (float)(((double)z - (double)cb.z) - (double)L.lz * nz);
-}
-
 // One axis of a minimum-image pair displacement in an orthorhombic box.
 // Within the box the f32 difference of the two coordinates is exact or
 // rounds at the pair's own scale; across a face it would round at the
@@ -248,367 +190,272 @@ __device__ __forceinline__ void pair_tri_disp(float pix, float piy, float piz, f
   dz = (float)(((double)piz - (double)pjz) - c * L.lz);
 }
 
-// Far-away coordinates for padding lanes on the shifted path: any pair
-// with one of them fails both cutoffs, and |d|^2 stays finite (< 1e37).
-#define PAIR_FAR_I 1.0e18f
-#define PAIR_FAR_J -1.0e18f
+// ---- row lists -----------------------------------------------------------
 
-// The 64 steps of one entry on the shifted path when one cutoff serves LJ
-// and Coulomb and there is no switch.  Lane l meets j-atom (l + t) mod 64 at
-// step t, read from the wave's LDS stage (jb, jt, jk point at record l); the
-// j-side sums still rotate with DPP, so they meet the same j-atoms and are
-// back in the loading lane after 64 steps.  Same terms as the general loop,
-// regrouped for fewer instructions per pair: exp(-(alpha r)^2) as
-// exp2(cg r^2); the Ewald force factor erfc(alpha r)/r^3 +
-// 2 alpha/sqrt(pi) exp(-(alpha r)^2)/r^2 as gauss * (poly(t) t / r +
-// 2 alpha/sqrt(pi)) / r^2; the LJ and Coulomb factors summed before the
-// shared 1/r^2 and a single cutoff select.  The force arithmetic is the same
-// for every EV, so energy steps move atoms exactly as force-only steps do.
-// XK = false drops the key test (no j-atom of the entry can be excluded
-// against the block).
-template <int EV, int NT, bool XK, bool COUL>
-__device__ __forceinline__ void uc_steps(const LjRow<NT>& R, float pix, float piy, float piz,
-                                         unsigned ikey, unsigned span, float kqi, float rc2,
-                                         float cg, float pa, float k2, const float4* jb,
-                                         const float2* jl, const unsigned* jt,
-                                         const unsigned* jk, float& efx,
-                                         float& efy, float& efz, float& jfx, float& jfy,
-                                         float& jfz, float& ee, float& je) {
-#pragma unroll 8
-  for (int t = 0; t < 64; ++t) {
-    float4 pq = jb[t];
-    float2 ljc;
-    if constexpr (NT == 0) {
-      float4 q = R.a[jt[t]];
-      ljc = make_float2(q.x, q.y);
-    } else {
-      ljc = (NT > 1) ? jl[t] : make_float2(R.f12[0], R.f6[0]);
-    }
-    float qj = pq.w;
-    float dx = pix - pq.x, dy = piy - pq.y, dz = piz - pq.z;
-    float r2 = dx * dx + dy * dy + dz * dz;
+// What one lane needs of its i-atom and of the pair terms.
+struct RowI {
+  int x, y, z;                // offset from the block centre in 1 / scale
+  float kq, inv2;             // k_C q_i; 1 / scale^2
+  float f12, f6, c12, c6;     // KIND 0: coefficients against the one active type
+  const float4 *ta, *tb;      // KIND 1, 2: the i-type's table rows (LDS)
+  const unsigned char* jt;    // KIND 1, 2: j types (LDS)
+  float rc2, cg, pa, k2;      // KIND 0, 1: shared cutoff^2, see PairParams
+  float alpha, coul_rc2;      // KIND 2
+};
+
+struct RowSum {
+  float fx, fy, fz, e, w;
+};
+
+// One pair of a row.  KIND 0: one cutoff for LJ and Coulomb, no switch, one
+// LJ-active type; 1: the same with several active types (table row of the
+// i-type, one LDS read per pair); 2: per-type cutoffs and the cubic switch.
+// LJ = false: the j-atom's type has no LJ interaction.  Terms of KIND 0 and
+// 1 are regrouped for fewer instructions: exp(-(alpha r)^2) as exp2(cg r^2);
+// the Ewald force factor erfc(alpha r)/r^3 + 2 alpha/sqrt(pi)
+// exp(-(alpha r)^2)/r^2 as gauss * (poly(t) t / r + 2 alpha/sqrt(pi)) / r^2;
+// one 1/r^2 and one cutoff select for the sum.  The force arithmetic is the
+// same for every EV, so energy steps move atoms as force-only steps do.
+template <int EV, int KIND, bool COUL, bool LJ>
+__device__ __forceinline__ void row_pair(const RowI& I, const int4* __restrict__ jrec,
+                                         unsigned off, RowSum& S) {
+  const int4 jr = *reinterpret_cast<const int4*>(reinterpret_cast<const char*>(jrec) + off);
+  const float jq = __int_as_float(jr.w);
+  float4 ta = make_float4(0.f, 0.f, 0.f, 0.f), tb = ta;
+  if (KIND != 0 && LJ) {
+    unsigned jt = I.jt[off >> 4];
+    ta = I.ta[jt];
+    if (KIND == 2) tb = I.tb[jt];
+  }
+  const float dx = (float)(I.x - jr.x), dy = (float)(I.y - jr.y), dz = (float)(I.z - jr.z);
+  const float r2 = (dx * dx + dy * dy + dz * dz) * I.inv2;
+  float factor, energy = 0.f;
+  if (KIND < 2) {
+    const float f12 = KIND == 0 ? I.f12 : ta.x, f6 = KIND == 0 ? I.f6 : ta.y;
     // LJ only: 1/r^2 from one reciprocal (half the rounding of squaring a
     // reciprocal square root, and one instruction fewer)
-    float inv_r = COUL ? __builtin_amdgcn_rsqf(r2) : 0.f;
-    float inv_r2 = COUL ? inv_r * inv_r : __builtin_amdgcn_rcpf(r2);
-    float ir6 = inv_r2 * inv_r2 * inv_r2;
-    float lj = ir6 * (ljc.x * ir6 - ljc.y);
-    float qq = 0.f, gauss = 0.f, poly = 0.f, factor;
+    const float inv_r = COUL ? __builtin_amdgcn_rsqf(r2) : 0.f;
+    const float inv_r2 = COUL ? inv_r * inv_r : __builtin_amdgcn_rcpf(r2);
+    float lj = 0.f, ir6 = 0.f;
+    if (LJ) {
+      ir6 = inv_r2 * inv_r2 * inv_r2;
+      lj = ir6 * (f12 * ir6 - f6);
+    }
     if (COUL) {
-      float r = r2 * inv_r;
-      gauss = __builtin_amdgcn_exp2f(cg * r2);
-      float tt = __builtin_amdgcn_rcpf(fmaf(pa, r, 1.0f));
-      poly =
+      const float r = r2 * inv_r;
+      const float gauss = __builtin_amdgcn_exp2f(I.cg * r2);
+      const float tt = __builtin_amdgcn_rcpf(fmaf(I.pa, r, 1.0f));
+      const float poly =
           (0.254829592f +
            (-0.284496736f + (1.421413741f + (-1.453152027f + 1.061405429f * tt) * tt) * tt) * tt) *
           tt;
-      float ci = gauss * fmaf(poly, inv_r, k2);
-      qq = kqi * qj;
-      factor = inv_r2 * fmaf(qq, ci, lj);
+      const float ci = gauss * fmaf(poly, inv_r, I.k2);
+      const float qq = I.kq * jq;
+      factor = LJ ? inv_r2 * fmaf(qq, ci, lj) : inv_r2 * (qq * ci);
+      if (EV == 1) energy = qq * gauss * (poly * inv_r);
     } else {
       factor = inv_r2 * lj;
     }
-    bool on = r2 <= rc2;
-    if (XK) on = on & ((jk[t] - ikey + span) > 2u * span);
+    if (EV == 1 && LJ) {
+      const float c12 = KIND == 0 ? I.c12 : ta.z, c6 = KIND == 0 ? I.c6 : ta.w;
+      energy += ir6 * (c12 * ir6 - c6);
+    }
+    const bool on = r2 <= I.rc2;
     factor = on ? factor : 0.f;
-    float nfactor = -factor;
-    efx = fmaf(factor, dx, efx); efy = fmaf(factor, dy, efy); efz = fmaf(factor, dz, efz);
-    jfx = fmaf(nfactor, dx, jfx); jfy = fmaf(nfactor, dy, jfy); jfz = fmaf(nfactor, dz, jfz);
-    if (EV == 1) {
-      // LJ energy (lj.rs:237-247) and qq erfc(alpha r) / r (spme.rs:744-770)
-      unsigned jtype = (NT != 1) ? jt[t] : 0u;
-      float elj = ir6 * (lj_c12(R, jtype) * ir6 - lj_c6(R, jtype));
-      float energy = on ? (COUL ? fmaf(qq * gauss, poly * inv_r, elj) : elj) : 0.f;
-      ee = fmaf(0.5f, energy, ee);
-      je = fmaf(0.5f, energy, je);
+    if (EV == 1) energy = on ? energy : 0.f;
+  } else {
+    const float inv_r = __builtin_amdgcn_rsqf(r2);
+    const float inv_r2 = inv_r * inv_r;
+    factor = 0.f;
+    if (LJ) {
+      // LJ (lj.rs:237-247) and the cubic switch (lj.rs:250-287); without a
+      // switch tb.z = 0, tau = 0 and the factors below are exactly 1 and 0
+      const float ir6 = inv_r2 * inv_r2 * inv_r2;
+      float flj = inv_r2 * ir6 * (ta.x * ir6 - ta.y);
+      float elj = ir6 * (ta.z * ir6 - ta.w);
+      const float tau = fmaxf((r2 - tb.y) * tb.z, 0.0f), omt = 1.0f - tau;
+      const float s = omt * omt * (1.0f + 2.0f * tau), chain = 12.0f * tau * omt * tb.z;
+      flj = s * flj + chain * elj;
+      elj = s * elj;
+      const bool on = r2 <= tb.x;
+      factor = on ? flj : 0.f;
+      if (EV == 1) energy = on ? elj : 0.f;
     }
-    jfx = hd_rot1(jfx); jfy = hd_rot1(jfy); jfz = hd_rot1(jfz);
-    if (EV == 1) je = hd_rot1(je);
-  }
-}
-
-// One wave's share of the entries of block b.  Lane = i-atom; the 64
-// j-atoms of an entry rotate through the wave with DPP wave_rol:1 and the
-// j-side partial sums travel with them, arriving back in the loading lane
-// after 64 steps.  SPC: coordinates are relative to the block centre (no
-// per-pair minimum image); otherwise general-cell minimum image per pair.
-template <int EV, int NT, bool SW, bool SPC, bool UC>
-__device__ __forceinline__ void pair_entries(
-    const PairParams& P, const HdLattice& L, unsigned b, unsigned w, unsigned lane, float pix,
-    float piy, float piz, float qi, unsigned ikey, const LjRow<NT>& R, float4 cb,
-    const float4* __restrict__ tile_posq, const unsigned* __restrict__ tile_type,
-    const unsigned* __restrict__ tile_key, const unsigned* __restrict__ ents, unsigned nent,
-    unsigned n, unsigned long long* __restrict__ fpj, unsigned long long* __restrict__ fpj_ew,
-    long long& ai_fx, long long& ai_fy, long long& ai_fz, long long& ai_e, long long& ai_w,
-    const unsigned* keymap, PairJStage<NT>* stage, unsigned itype) {
-  const float two_a_sqrtpi = 2.0f * P.alpha * 0.5641895835477563f;
-  const float alpha = P.alpha, coul_rc2 = P.coul_rc2;
-  const float kqi = P.kc * qi;
-  const float ilx = 1.0f / L.lx, ily = 1.0f / L.ly, ilz = 1.0f / L.lz;
-  for (unsigned e = w; e < nent; e += PAIR_WAVES) {
-    unsigned jslot = ents[(size_t)e * 64 + lane];
-    bool jvalid = jslot < n;
-    unsigned jsafe = jvalid ? jslot : 0u;
-    float4 pj = tile_posq[jsafe];
-    unsigned jtype = (NT != 1) ? tile_type[jsafe] : 0u;
-    unsigned jkey = tile_key[jsafe];
-    bool jin = jvalid && (jslot >> 6) == b;
-    float pjx = pj.x, pjy = pj.y, pjz = pj.z, qj = jvalid ? pj.w : 0.f;
-    if (SPC) {
-      pair_rel_to_center(pj.x, pj.y, pj.z, cb, L, ilx, ily, ilz, pjx, pjy, pjz);
-      if (!jvalid) pjx = pjy = pjz = PAIR_FAR_J;
-    } else {
-      // validity travels in the key: padding lanes can never pass the
-      // key test (i padding carries HD_SENTINEL - 1, j padding HD_SENTINEL)
-      jkey = jvalid ? jkey : HD_SENTINEL;
-    }
-    float jfx = 0.f, jfy = 0.f, jfz = 0.f, je = 0.f, jw = 0.f;
-    float efx = 0.f, efy = 0.f, efz = 0.f, ee = 0.f, ew = 0.f;
-    if constexpr (UC) {
-      // a j-atom can be excluded only when its key is in the block's map
-      unsigned word = keymap[(jkey >> 5) & (PAIR_KEYMAP_WORDS - 1u)];
-      bool hit = jvalid && ((word >> (jkey & 31u)) & 1u);
-      PairJStage<NT>& S = stage[w];
-      float4 rec = make_float4(pjx, pjy, pjz, qj);
-      S.pq[lane] = rec; S.pq[lane + 64] = rec;
-      if constexpr (NT > 1) {
-        // the same products load_row forms for an i-atom of type ti
-#pragma unroll
-        for (int ti = 0; ti < NT; ++ti) {
-          float f12[NT], f6[NT];
-#pragma unroll
-          for (int u = 0; u < NT; ++u) {
-            int k = (ti < P.ntypes && u < P.ntypes) ? ti * P.ntypes + u : 0;
-            f12[u] = 12.0f * P.c12[k];
-            f6[u] = 6.0f * P.c6[k];
-          }
-          float2 c = make_float2(pick<NT>(f12, jtype), pick<NT>(f6, jtype));
-          S.lj[ti][lane] = c; S.lj[ti][lane + 64] = c;
-        }
-      }
-      if (EV == 1 || NT == 0) { S.type[lane] = jtype; S.type[lane + 64] = jtype; }
-      S.key[lane] = jkey; S.key[lane + 64] = jkey;
-      wave_lds_sync();
-      const float2* jl = &S.lj[(NT > 1) ? itype : 0u][lane];
-      bool xk = P.excl_span > PAIR_KEYMAP_SPAN || __any(hit);
-      const unsigned* jt = &S.type[lane];
-      const unsigned* jk = &S.key[lane];
-      if (P.uniform == 2) {
-        if (xk)
-          uc_steps<EV, NT, true, false>(R, pix, piy, piz, ikey, P.excl_span, kqi, P.uc_rc2, P.cg,
-                                        P.pa, two_a_sqrtpi, &S.pq[lane], jl, jt, jk, efx, efy,
-                                        efz, jfx, jfy, jfz, ee, je);
-        else
-          uc_steps<EV, NT, false, false>(R, pix, piy, piz, ikey, P.excl_span, kqi, P.uc_rc2,
-                                         P.cg, P.pa, two_a_sqrtpi, &S.pq[lane], jl, jt, jk, efx,
-                                         efy, efz, jfx, jfy, jfz, ee, je);
-      } else {
-        if (xk)
-          uc_steps<EV, NT, true, true>(R, pix, piy, piz, ikey, P.excl_span, kqi, P.uc_rc2, P.cg,
-                                       P.pa, two_a_sqrtpi, &S.pq[lane], jl, jt, jk, efx, efy, efz,
-                                       jfx, jfy, jfz, ee, je);
-        else
-          uc_steps<EV, NT, false, true>(R, pix, piy, piz, ikey, P.excl_span, kqi, P.uc_rc2, P.cg,
-                                        P.pa, two_a_sqrtpi, &S.pq[lane], jl, jt, jk, efx, efy,
-                                        efz, jfx, jfy, jfz, ee, je);
-      }
-      // every lane's reads of this entry precede the next entry's writes
-      wave_lds_sync();
-    } else {
-#pragma unroll 4
-    for (int t = 0; t < 64; ++t) {
-      float dx = pix - pjx, dy = piy - pjy, dz = piz - pjz;
-      if (!SPC) {
-        if (P.ortho) {
-          dx = pair_axis_disp(pix, pjx, L.lx, ilx);
-          dy = pair_axis_disp(piy, pjy, L.ly, ily);
-          dz = pair_axis_disp(piz, pjz, L.lz, ilz);
-        } else {
-          pair_tri_disp(pix, piy, piz, pjx, pjy, pjz, L, ilx, ily, ilz, dx, dy, dz);
-        }
-      }
-      float r2 = dx * dx + dy * dy + dz * dz;
-      float inv_r = __builtin_amdgcn_rsqf(r2);
-      float inv_r2 = inv_r * inv_r;
-      // LJ (lj.rs:237-247, 250-287) from the i-row, column = j type
-      float ir6 = inv_r2 * inv_r2 * inv_r2;
-      float flj = inv_r2 * ir6 * (lj_f12(R, jtype) * ir6 - lj_f6(R, jtype));
-      float elj = 0.f;
-      if (EV == 1 || SW) elj = ir6 * (lj_c12(R, jtype) * ir6 - lj_c6(R, jtype));
-      if (SW) {
-        float rs2 = lj_rsw2(R, jtype), idl = lj_idl(R, jtype);
-        float tau = fmaxf((r2 - rs2) * idl, 0.0f);
-        float omt = 1.0f - tau;
-        float s = omt * omt * (1.0f + 2.0f * tau);
-        float chain = 12.0f * tau * omt * idl;
-        flj = s * flj + chain * elj;
-        elj = s * elj;
-      }
-      bool lj_on = r2 <= lj_cut2(R, jtype);
+    if (COUL) {
       // real-space Coulomb, f32 Hastings erfc (spme.rs:744-770)
-      float r = r2 * inv_r;
-      float qq = kqi * qj;
-      float ar = alpha * r;
-      float gauss = __expf(-(ar * ar));
-      float tt = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * ar);
-      float erfc_ar =
+      const float r = r2 * inv_r, qq = I.kq * jq, ar = I.alpha * r;
+      const float gauss = __expf(-(ar * ar));
+      const float tt = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * ar);
+      const float erfc_ar =
           (0.254829592f +
            (-0.284496736f + (1.421413741f + (-1.453152027f + 1.061405429f * tt) * tt) * tt) * tt) *
           tt * gauss;
-      float ec = qq * erfc_ar * inv_r;
-      float fc = qq * inv_r2 * (erfc_ar * inv_r + two_a_sqrtpi * gauss);
-      bool c_on = r2 <= coul_rc2;
-      // excluded when |key_j - key_i| <= span (span 0: equal molecule keys)
-      bool ok = (jkey - ikey + P.excl_span) > 2u * P.excl_span;
-      if (!SPC) ok = ok & (max(jkey, ikey) < HD_SENTINEL - 1u);
-      float factor = (ok & lj_on) ? flj : 0.f;
-      factor += (ok & c_on) ? fc : 0.f;
-      // i and j sides as fused multiply-adds of +-factor * d
-      float nfactor = -factor;
-      efx = fmaf(factor, dx, efx); efy = fmaf(factor, dy, efy); efz = fmaf(factor, dz, efz);
-      jfx = fmaf(nfactor, dx, jfx); jfy = fmaf(nfactor, dy, jfy); jfz = fmaf(nfactor, dz, jfz);
-      if (EV == 1) {
-        float energy = (ok & lj_on) ? elj : 0.f;
-        energy += (ok & c_on) ? ec : 0.f;
-        ee = fmaf(0.5f, energy, ee);
-        je = fmaf(0.5f, energy, je);
-      }
-      if (EV && !SPC) {
-        float fr2 = factor * r2;
-        ew = fmaf(0.5f, fr2, ew);
-        jw = fmaf(0.5f, fr2, jw);
-      }
-      pjx = hd_rot1(pjx); pjy = hd_rot1(pjy); pjz = hd_rot1(pjz); qj = hd_rot1(qj);
-      jkey = hd_rot1_u(jkey);
-      if (NT != 1) jtype = hd_rot1_u(jtype);
-      jfx = hd_rot1(jfx); jfy = hd_rot1(jfy); jfz = hd_rot1(jfz);
-      if (EV == 1) je = hd_rot1(je);
-      if (EV && !SPC) jw = hd_rot1(jw);
+      const bool on = r2 <= I.coul_rc2;
+      const float fc = qq * inv_r2 * (erfc_ar * inv_r + I.k2 * gauss);
+      factor += on ? fc : 0.f;
+      if (EV == 1) energy += on ? qq * erfc_ar * inv_r : 0.f;
     }
-    }
-    if (EV && SPC) {
-      // the entry's pair virial sum_ij F_ij . (r_i - r_j) split by atom: both
-      // positions are relative to the block centre (j in the image nearest
-      // it), so the i side is r_i . F_i(entry) and the j side r_j . F_j(entry)
-      // (j partials are back in their loading lanes, and so are the j
-      // positions); pairs inside the block are evaluated from both sides and
-      // their j sides dropped, which again leaves F_ij . r_ij once
-      ew = pix * efx + piy * efy + piz * efz;
-      jw = pjx * jfx + pjy * jfy + pjz * jfz;
-    }
-    ai_fx += hd_to_fixed48(efx);
-    ai_fy += hd_to_fixed48(efy);
-    ai_fz += hd_to_fixed48(efz);
-    if (EV) {
-      ai_e += hd_to_fixed48(ee);
-      ai_w += hd_to_fixed48(ew);
-    }
-    // Newton's third law: the j-side sums of atoms that belong to block b
-    // are dropped (their pairs were evaluated from both sides as i-pairs)
-    if (jvalid && !jin) {
-      unsigned long long* d = fpj + (size_t)jslot * 4;
-      long long vx = hd_to_fixed48(jfx), vy = hd_to_fixed48(jfy), vz = hd_to_fixed48(jfz);
-      if (vx) atomicAdd(d + 0, (unsigned long long)vx);
-      if (vy) atomicAdd(d + 1, (unsigned long long)vy);
-      if (vz) atomicAdd(d + 2, (unsigned long long)vz);
-      if (EV) {
-        long long ve = hd_to_fixed48(je), vw = hd_to_fixed48(jw);
-        if (EV == 1 && ve) atomicAdd(fpj_ew + (size_t)jslot * 2, (unsigned long long)ve);
-        if (vw) atomicAdd(fpj_ew + (size_t)jslot * 2 + 1, (unsigned long long)vw);
-      }
-    }
+  }
+  S.fx = fmaf(factor, dx, S.fx);
+  S.fy = fmaf(factor, dy, S.fy);
+  S.fz = fmaf(factor, dz, S.fz);
+  if (EV == 1) S.e += energy;
+  if (EV) S.w = fmaf(factor, r2, S.w);
+}
+
+// Chunks [k0, k1) of the wave's rows, the next chunk's load in flight while
+// one is evaluated.
+template <int EV, int KIND, bool COUL, bool LJ>
+__device__ __forceinline__ void row_chunks(const RowI& I, const int4* __restrict__ jrec,
+                                           const uint2* __restrict__ rp, unsigned k0,
+                                           unsigned k1, RowSum& S) {
+  if (k0 >= k1) return;
+  uint2 nx = rp[k0 * (HD_ROW_CHUNK / 4u)];
+  for (unsigned k = k0; k < k1; ++k) {
+    const uint2 c = nx;
+    if (k + 1 < k1) nx = rp[(k + 1) * (HD_ROW_CHUNK / 4u)];
+    row_pair<EV, KIND, COUL, LJ>(I, jrec, c.x & 0xFFFFu, S);
+    row_pair<EV, KIND, COUL, LJ>(I, jrec, c.x >> 16, S);
+    row_pair<EV, KIND, COUL, LJ>(I, jrec, c.y & 0xFFFFu, S);
+    row_pair<EV, KIND, COUL, LJ>(I, jrec, c.y >> 16, S);
   }
 }
 
-template <int EV, int NT, bool SW>
-__global__ void __launch_bounds__(256) k_pair(
+// sum over the 8 lanes that share an i-atom (lane bits 0..2), in every lane
+__device__ __forceinline__ float row_sum8(float v) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true));
+  return v;
+}
+
+// One workgroup of 8 waves per unit of the row lists (k_build_rows): the
+// unit's j-atoms are staged once in LDS, relative to the block centre in
+// their own image; wave w holds i-atoms 8 w .. 8 w + 7, eight lanes each,
+// lane 8 r + s taking entries s of row r.  Both sides of every pair are
+// evaluated, so nothing is added to the j-atoms: the lanes' f32 sums (at
+// most 1/8 of a row each) are added over the 8 lanes, turned into fixed
+// point at 2^48 and added once per i-atom to its accumulator (one coalesced
+// 64-bit atomic instruction per wave).
+//
+// Positions are whole numbers of a power-of-two step relative to the block
+// centre (hd_rel_fixed): f32 offsets rounded the displacement of a pair at
+// the block's size, and the error of a force (rms, 64-bit reference) was
+// 8.2e-7 of the rms force in a tilted cell where it is now 5.7e-7.
+//
+// Bound by the vector ALU (about 34 instructions a slot of an LJ-active
+// j-atom, 27 of another, plus one LDS read): listing the active j-atoms
+// first lets a wave drop the LJ half for whole chunks.  54 VGPRs, so the
+// LDS of the j-list sets the occupancy.  Measured, us per launch (the
+// packed tiles it replaced): 196,608 atoms of water 130 beside the SPME
+// pipeline (208); 24,576 atoms 26 (78); 7,938 atoms 13 (68); 267 atoms 5.1
+// (16).
+template <int EV, int KIND, bool COUL>
+__global__ void __launch_bounds__(HD_ROW_THREADS) k_pair_rows(
     PairParams P, const float* __restrict__ lattice, const float4* __restrict__ tile_posq,
-    const unsigned* __restrict__ tile_type, const unsigned* __restrict__ tile_key,
+    const unsigned* __restrict__ tile_type, const unsigned char* __restrict__ tile_img,
     const float4* __restrict__ center, const float4* __restrict__ half,
-    const unsigned* __restrict__ entry_atoms, const unsigned* __restrict__ entry_count,
-    const unsigned* __restrict__ block_order, unsigned cap, unsigned n,
-    long long* __restrict__ fpi, long long* __restrict__ fpi_ew,
-    unsigned long long* __restrict__ fpj, unsigned long long* __restrict__ fpj_ew,
-    const float4* __restrict__ lj_tab) {
-  __shared__ long long red[PAIR_WAVES][5][64];
-  __shared__ unsigned keymap[PAIR_KEYMAP_WORDS];
-  __shared__ PairJStage<NT> stage[PAIR_WAVES];
-  __shared__ PairTab<NT> tab;
-  if constexpr (NT == 0) {
-    load_tab(tab, lj_tab, P.ntypes);
-    __syncthreads();
+    const unsigned* __restrict__ jslot, const unsigned* __restrict__ jcount,
+    const unsigned* __restrict__ rowhdr,
+    const unsigned short* __restrict__ rows, const unsigned* __restrict__ order, unsigned parts,
+    unsigned jcap, unsigned rcap, unsigned n, unsigned long long* __restrict__ fpj,
+    unsigned long long* __restrict__ fpj_ew, const float4* __restrict__ lj_tab) {
+  extern __shared__ float4 lds[];
+  int4* jrec = reinterpret_cast<int4*>(lds);
+  const unsigned nt2 = (unsigned)(P.ntypes * P.ntypes);
+  float4* tab_a = lds + jcap + 1;
+  float4* tab_b = tab_a + (KIND != 0 ? nt2 : 0u);
+  unsigned char* jt = reinterpret_cast<unsigned char*>(tab_b + (KIND == 2 ? nt2 : 0u));
+  const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  const unsigned unit = order[blockIdx.x];  // heaviest first
+  const unsigned b = unit / parts;
+  const HdLattice L = hd_load_lattice(lattice);
+  const float4 cb = center[b];
+  // scale: offsets reach the block's half extent, the search radius and what
+  // atoms moved since; 2^23 or 2^24 for a dense block (2^-24 Bohr is 1/8 of
+  // the rounding of a 4 Bohr displacement)
+  const float4 hb = half[b];
+  const int se = 28 - ilogbf(fmaxf(hb.x, fmaxf(hb.y, hb.z)) + P.reach);
+  const double scale = ldexp(1.0, se);
+  const float inv = ldexpf(1.0f, -se);
+  const unsigned jc = jcount[unit], nja = jc & 0xFFFFu;
+  const unsigned hdr = rowhdr[unit * HD_ROW_WAVES + w];
+  const unsigned islot = b * 64u + w * HD_ROW_I + (lane >> 3);
+  const bool ivalid = islot < n;
+  const float4 pi = tile_posq[islot];  // npad entries
+  const unsigned itype = ivalid ? tile_type[islot] : 0u;
+  // without Coulomb the j-atoms of inactive types are not read
+  const unsigned nj = nja + (COUL ? jc >> 16 : 0u);
+  for (unsigned q = t; q < nj; q += HD_ROW_THREADS) {
+    const unsigned k = q < nja ? q : jcap - 1u - (q - nja);
+    const unsigned js = jslot[(size_t)unit * jcap + k];
+    const unsigned s = js & (HD_ROW_SLOTS - 1u), code = js >> HD_ROW_SLOT_BITS;
+    const float4 p = tile_posq[s];
+    const int3 f = hd_rel_fixed(p.x, p.y, p.z, cb, code, tile_img[s], L, scale);
+    jrec[k] = make_int4(f.x, f.y, f.z, __float_as_int(p.w));
+    if (KIND != 0) jt[k] = (unsigned char)tile_type[s];
   }
-  unsigned b = block_order[blockIdx.x];  // heaviest blocks first
-  unsigned w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  HdLattice L = hd_load_lattice(lattice);
-  unsigned islot = b * 64 + lane;
-  bool ivalid = islot < n;
-  float4 pi = tile_posq[ivalid ? islot : 0u];
-  unsigned itype = ivalid ? tile_type[islot] : 0u;
-  unsigned ikey = ivalid ? tile_key[islot] : (HD_SENTINEL - 1u);
-  float4 cb = center[b], hb = half[b];
-  bool spc = (L.xy == 0.f && L.xz == 0.f && L.yz == 0.f) &&
-             (0.5f * L.lx - hb.x >= P.spc_margin) && (0.5f * L.ly - hb.y >= P.spc_margin) &&
-             (0.5f * L.lz - hb.z >= P.spc_margin);
-  float pix = pi.x, piy = pi.y, piz = pi.z, qi = ivalid ? pi.w : 0.f;
-  if (!ivalid) { pix = cb.x; piy = cb.y; piz = cb.z; }
-  if (spc) {
-    hd_rel_to_center(pix, piy, piz, cb.x, cb.y, cb.z, L, pix, piy, piz);
-    if (!ivalid) pix = piy = piz = PAIR_FAR_I;
+  if (t == 0) {
+    jrec[jcap] = make_int4(HD_FIXED_FAR, 0, 0, 0);
+    if (KIND != 0) jt[jcap] = 0;
   }
-  LjRow<NT> R = load_row<NT>(P, itype, ivalid, tab);
-  unsigned nent = entry_count[b];
-  const unsigned* ents = entry_atoms + (size_t)b * cap * 64;
-  long long ax = 0, ay = 0, az = 0, ae = 0, aw = 0;
-  // the regrouped loop: one cutoff, no switch
-  constexpr bool UCOK = !SW;
-  bool uc = UCOK && spc && P.uniform;  // uniform over the workgroup
-  if (uc) {
-    if constexpr (UCOK) {
-      for (unsigned k = threadIdx.x; k < PAIR_KEYMAP_WORDS; k += 64 * PAIR_WAVES) keymap[k] = 0u;
-      __syncthreads();
-      if (w == 0 && ivalid && P.excl_span <= PAIR_KEYMAP_SPAN)
-        for (unsigned d = 0; d <= 2u * P.excl_span; ++d) {
-          unsigned key = ikey - P.excl_span + d;
-          atomicOr(&keymap[(key >> 5) & (PAIR_KEYMAP_WORDS - 1u)], 1u << (key & 31u));
-        }
-      __syncthreads();
-      pair_entries<EV, NT, SW, true, true>(P, L, b, w, lane, pix, piy, piz, qi, ikey, R, cb,
-                                           tile_posq, tile_type, tile_key, ents, nent, n, fpj,
-                                           fpj_ew, ax, ay, az, ae, aw, keymap, stage, itype);
+  if (KIND != 0)
+    for (unsigned k = t; k < nt2; k += HD_ROW_THREADS) {
+      tab_a[k] = lj_tab[2 * k];
+      if (KIND == 2) tab_b[k] = lj_tab[2 * k + 1];
     }
-  } else if (spc)
-    pair_entries<EV, NT, SW, true, false>(P, L, b, w, lane, pix, piy, piz, qi, ikey, R, cb,
-                                          tile_posq, tile_type, tile_key, ents, nent, n, fpj,
-                                          fpj_ew, ax, ay, az, ae, aw, keymap, stage, itype);
-  else
-    pair_entries<EV, NT, SW, false, false>(P, L, b, w, lane, pix, piy, piz, qi, ikey, R, cb,
-                                           tile_posq, tile_type, tile_key, ents, nent, n, fpj,
-                                           fpj_ew, ax, ay, az, ae, aw, keymap, stage, itype);
-  red[w][0][lane] = ax;
-  red[w][1][lane] = ay;
-  red[w][2][lane] = az;
-  if (EV) {
-    red[w][3][lane] = ae;
-    red[w][4][lane] = aw;
+  RowI I;
+  const int3 fi = hd_rel_fixed(pi.x, pi.y, pi.z, cb, HD_IMAGE_NONE, tile_img[islot], L, scale);
+  // a slot without atom, or an atom out of reach, on the other side of the
+  // far j-atoms
+  I.x = !ivalid || fi.x == HD_FIXED_FAR ? -HD_FIXED_FAR : fi.x;
+  I.y = fi.y;
+  I.z = fi.z;
+  I.inv2 = inv * inv;
+  I.kq = P.kc * pi.w;
+  if (KIND == 0) {
+    const float4 c = lj_tab[2 * (itype * (unsigned)P.ntypes + (unsigned)P.active_type)];
+    I.f12 = c.x;
+    I.f6 = c.y;
+    I.c12 = c.z;
+    I.c6 = c.w;
+  } else {
+    I.ta = tab_a + itype * (unsigned)P.ntypes;
+    I.tb = tab_b + itype * (unsigned)P.ntypes;
+    I.jt = jt;
   }
+  I.rc2 = P.uc_rc2;
+  I.cg = P.cg;
+  I.pa = P.pa;
+  I.k2 = 2.0f * P.alpha * 0.5641895835477563f;
+  I.alpha = P.alpha;
+  I.coul_rc2 = P.coul_rc2;
   __syncthreads();
-  if (w == 0) {
-    long long s[5] = {0, 0, 0, 0, 0};
-#pragma unroll
-    for (int k = 0; k < PAIR_WAVES; ++k) {
-      s[0] += red[k][0][lane];
-      s[1] += red[k][1][lane];
-      s[2] += red[k][2][lane];
-      if (EV) {
-        s[3] += red[k][3][lane];
-        s[4] += red[k][4][lane];
-      }
+  const uint2* rp = reinterpret_cast<const uint2*>(
+                        rows + ((size_t)unit * 64u + w * HD_ROW_I + (lane >> 3)) *
+                                   rcap) +
+                    (lane & 7u);
+  RowSum S = {0.f, 0.f, 0.f, 0.f, 0.f};
+  const unsigned hu = (unsigned)__builtin_amdgcn_readfirstlane((int)hdr);
+  row_chunks<EV, KIND, COUL, true>(I, jrec, rp, 0u, hu & 0xFFFFu, S);
+  // without Coulomb the j-atoms of inactive types contribute nothing
+  if (COUL) row_chunks<EV, KIND, COUL, false>(I, jrec, rp, hu & 0xFFFFu, hu >> 16, S);
+  // the force factors multiplied displacements in 1 / scale
+  const float fx = inv * row_sum8(S.fx), fy = inv * row_sum8(S.fy), fz = inv * row_sum8(S.fz);
+  float v = (lane & 7u) == 0u ? fx : ((lane & 7u) == 1u ? fy : fz);
+  unsigned long long* dst = fpj + (size_t)islot * 4 + (lane & 7u);
+  bool mine = ivalid && (lane & 7u) < 3u;
+  if (EV) {
+    // each side of a pair carries half of its energy and virial
+    const float e = 0.5f * row_sum8(S.e), wv = 0.5f * row_sum8(S.w);
+    if ((lane & 7u) >= 3u) {
+      v = (lane & 7u) == 3u ? e : wv;
+      dst = fpj_ew + (size_t)islot * 2 + ((lane & 7u) - 3u);
     }
-    reinterpret_cast<longlong2*>(fpi)[2 * islot] = make_longlong2(s[0], s[1]);
-    reinterpret_cast<longlong2*>(fpi)[2 * islot + 1] = make_longlong2(s[2], 0);
-    if (EV) reinterpret_cast<longlong2*>(fpi_ew)[islot] = make_longlong2(s[3], s[4]);
+    mine = ivalid && (lane & 7u) < 5u && (EV == 1 || (lane & 7u) != 3u);
   }
+  const long long f = hd_to_fixed48(v);
+  if (mine && f) atomicAdd(dst, (unsigned long long)f);
 }
 
 // Atom-list mode: one workgroup of 4 waves per 64-atom i-block, lane =
@@ -1088,31 +935,38 @@ void hd_launch_excl_scaled(hipStream_t st, const float4* posq, const float* latt
 }
 
 // Diagnostic: number of distinct pairs of the current list with
-// r^2 <= r_max^2 that are neither excluded nor padding (the "useful" pairs
-// the pair kernel evaluates).  One wave per i-block, plain loops.
-__global__ void __launch_bounds__(64) k_count_pairs(
-    float rmax2, unsigned excl_span, const float* __restrict__ lattice, const float4* __restrict__ tile_posq,
-    const unsigned* __restrict__ tile_key, const unsigned* __restrict__ entry_atoms,
-    const unsigned* __restrict__ entry_count, unsigned cap, unsigned n,
-    unsigned long long* __restrict__ out) {
-  unsigned b = blockIdx.x, lane = threadIdx.x;
-  unsigned islot = b * 64 + lane;
+// r^2 <= r_max^2 (the "useful" pairs).  Every pair is in both atoms' rows:
+// counted from the lower slot.
+__global__ void __launch_bounds__(HD_ROW_THREADS) k_count_rows(
+    float rmax2, const float* __restrict__ lattice, const float4* __restrict__ tile_posq,
+    const unsigned char* __restrict__ tile_img, const float4* __restrict__ center,
+    const unsigned* __restrict__ jslot,
+    const unsigned* __restrict__ rowhdr,
+    const unsigned short* __restrict__ rows, unsigned parts, unsigned jcap, unsigned rcap,
+    unsigned n, unsigned long long* __restrict__ out) {
+  const unsigned unit = blockIdx.x, b = unit / parts;
+  const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  const unsigned islot = b * 64u + w * HD_ROW_I + (lane >> 3);
   if (islot >= n) return;
-  HdLattice L = hd_load_lattice(lattice);
-  float4 pi = tile_posq[islot];
-  unsigned ikey = tile_key[islot];
-  unsigned nent = entry_count[b];
-  const unsigned* ents = entry_atoms + (size_t)b * cap * 64;
+  const HdLattice L = hd_load_lattice(lattice);
+  const float4 cb = center[b], pi = tile_posq[islot];
+  float ix, iy, iz;
+  hd_rel_image(pi.x, pi.y, pi.z, cb, HD_IMAGE_NONE, tile_img[islot], L, ix, iy, iz);
+  const unsigned nk = rowhdr[unit * HD_ROW_WAVES + w] >> 16;
+  const unsigned short* rp =
+      rows + ((size_t)unit * 64u + w * HD_ROW_I + (lane >> 3)) * rcap;
   unsigned long long cnt = 0;
-  for (unsigned e = 0; e < nent; ++e)
-    for (unsigned t = 0; t < 64; ++t) {
-      unsigned js = ents[(size_t)e * 64 + t];
-      if (js >= n) continue;
-      if ((js >> 6) == b && js <= islot) continue;
-      if (tile_key[js] - ikey + excl_span <= 2u * excl_span) continue;
+  for (unsigned k = 0; k < nk; ++k)
+    for (unsigned u = 0; u < 4; ++u) {
+      unsigned j = rp[k * HD_ROW_CHUNK + (lane & 7u) * 4u + u] >> 4;
+      if (j >= jcap) continue;
+      const unsigned code = jslot[(size_t)unit * jcap + j] >> HD_ROW_SLOT_BITS;
+      const unsigned js = jslot[(size_t)unit * jcap + j] & (HD_ROW_SLOTS - 1u);
+      if (js <= islot) continue;
       float4 pj = tile_posq[js];
-      float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-      hd_min_image(dx, dy, dz, L);
+      float jx, jy, jz;
+      hd_rel_image(pj.x, pj.y, pj.z, cb, code, tile_img[js], L, jx, jy, jz);
+      float dx = ix - jx, dy = iy - jy, dz = iz - jz;
       if (dx * dx + dy * dy + dz * dz <= rmax2) ++cnt;
     }
   atomicAdd(out, cnt);
@@ -1149,44 +1003,66 @@ void hd_launch_count_pairs(hipStream_t st, const HdPairArgs& a, unsigned long lo
                        (float)(a.rmax * a.rmax), a.lattice, a.tile_posq, a.entry_atoms,
                        a.entry_count, a.cap, a.n, out);
   else
-    hipLaunchKernelGGL(k_count_pairs, dim3(nblocks), dim3(64), 0, st, (float)(a.rmax * a.rmax),
-                       a.excl_span, a.lattice, a.tile_posq, a.tile_key, a.entry_atoms,
-                       a.entry_count, a.cap, a.n, out);
+    hipLaunchKernelGGL(k_count_rows, dim3(nblocks * a.parts), dim3(HD_ROW_THREADS), 0, st,
+                       (float)(a.rmax * a.rmax), a.lattice, a.tile_posq, a.tile_img, a.center,
+                       a.jslot, a.rowhdr, a.rows, a.parts, a.jcap, a.rcap, a.n, out);
 }
 
 template <int EV, int NT, bool SW>
-static void launch_pair_t(hipStream_t st, const HdPairArgs& a, const PairParams& P) {
+static void launch_alist_t(hipStream_t st, const HdPairArgs& a, const PairParams& P) {
   unsigned nblocks = a.npad / 64;
-  if (a.atom_lists) {
-    dim3 grid(nblocks);
-    if (P.ortho)
-      hipLaunchKernelGGL((k_pair_alist<EV, NT, SW, true>), grid, dim3(64 * PAIR_WAVES), 0, st, P,
-                         a.lattice, a.tile_posq, a.tile_type, a.entry_atoms, a.entry_count,
-                         a.cap, a.n, nblocks, a.fpi, a.fpi_ew, a.lj_tab);
-    else
-      hipLaunchKernelGGL((k_pair_alist<EV, NT, SW, false>), grid, dim3(64 * PAIR_WAVES), 0, st,
-                         P, a.lattice, a.tile_posq, a.tile_type, a.entry_atoms, a.entry_count,
-                         a.cap, a.n, nblocks, a.fpi, a.fpi_ew, a.lj_tab);
-    return;
-  }
-  hipLaunchKernelGGL((k_pair<EV, NT, SW>), dim3(nblocks), dim3(64 * PAIR_WAVES), 0, st, P,
-                     a.lattice, a.tile_posq, a.tile_type, a.tile_key, a.center, a.half,
-                     a.entry_atoms, a.entry_count, a.block_order, a.cap, a.n, a.fpi, a.fpi_ew,
-                     (unsigned long long*)a.fpj, (unsigned long long*)a.fpj_ew, a.lj_tab);
+  dim3 grid(nblocks);
+  if (P.ortho)
+    hipLaunchKernelGGL((k_pair_alist<EV, NT, SW, true>), grid, dim3(64 * PAIR_WAVES), 0, st, P,
+                       a.lattice, a.tile_posq, a.tile_type, a.entry_atoms, a.entry_count,
+                       a.cap, a.n, nblocks, a.fpi, a.fpi_ew, a.lj_tab);
+  else
+    hipLaunchKernelGGL((k_pair_alist<EV, NT, SW, false>), grid, dim3(64 * PAIR_WAVES), 0, st,
+                       P, a.lattice, a.tile_posq, a.tile_type, a.entry_atoms, a.entry_count,
+                       a.cap, a.n, nblocks, a.fpi, a.fpi_ew, a.lj_tab);
+}
+
+unsigned hd_pair_rows_lds(int nt, unsigned jcap) {
+  // the dummy record, the type-pair table and the j types
+  return 16u + (nt > 1 ? 32u * (unsigned)(nt * nt) + jcap + 1u : 0u);
+}
+
+template <int EV, int KIND>
+static void launch_rows_c(hipStream_t st, const HdPairArgs& a, const PairParams& P) {
+  dim3 grid(a.npad / 64 * a.parts), wg(HD_ROW_THREADS);
+  const size_t lds = (size_t)a.jcap * sizeof(float4) + hd_pair_rows_lds(P.ntypes, a.jcap);
+  if (P.coul_rc2 > 0.f)
+    hipLaunchKernelGGL((k_pair_rows<EV, KIND, true>), grid, wg, lds, st, P, a.lattice,
+                       a.tile_posq, a.tile_type, a.tile_img, a.center, a.half, a.jslot, a.jcount,
+                       a.rowhdr, a.rows, a.block_order, a.parts, a.jcap, a.rcap, a.n,
+                       (unsigned long long*)a.fpj, (unsigned long long*)a.fpj_ew, a.lj_tab);
+  else
+    hipLaunchKernelGGL((k_pair_rows<EV, KIND, false>), grid, wg, lds, st, P, a.lattice,
+                       a.tile_posq, a.tile_type, a.tile_img, a.center, a.half, a.jslot, a.jcount,
+                       a.rowhdr, a.rows, a.block_order, a.parts, a.jcap, a.rcap, a.n,
+                       (unsigned long long*)a.fpj, (unsigned long long*)a.fpj_ew, a.lj_tab);
 }
 
 template <int EV, int NT>
-static void launch_pair_nt(hipStream_t st, const HdPairArgs& a, const PairParams& P, bool sw) {
-  if (sw) launch_pair_t<EV, NT, true>(st, a, P);
-  else launch_pair_t<EV, NT, false>(st, a, P);
+static void launch_alist_nt(hipStream_t st, const HdPairArgs& a, const PairParams& P, bool sw) {
+  if (sw) launch_alist_t<EV, NT, true>(st, a, P);
+  else launch_alist_t<EV, NT, false>(st, a, P);
 }
 
 template <int EV>
 static void launch_pair_ev(hipStream_t st, const HdPairArgs& a, const PairParams& P, bool sw) {
-  if (P.ntypes <= 1) launch_pair_nt<EV, 1>(st, a, P, sw);
-  else if (P.ntypes == 2) launch_pair_nt<EV, 2>(st, a, P, sw);
-  else if (P.ntypes <= PAIR_MAXT) launch_pair_nt<EV, 4>(st, a, P, sw);
-  else launch_pair_nt<EV, 0>(st, a, P, sw);
+  if (!a.atom_lists) {
+    // one cutoff and no switch: the regrouped terms, with the coefficients
+    // in registers when a single type interacts
+    if (!P.uniform) launch_rows_c<EV, 2>(st, a, P);
+    else if (P.active_type < 0) launch_rows_c<EV, 1>(st, a, P);
+    else launch_rows_c<EV, 0>(st, a, P);
+    return;
+  }
+  if (P.ntypes <= 1) launch_alist_nt<EV, 1>(st, a, P, sw);
+  else if (P.ntypes == 2) launch_alist_nt<EV, 2>(st, a, P, sw);
+  else if (P.ntypes <= PAIR_MAXT) launch_alist_nt<EV, 4>(st, a, P, sw);
+  else launch_alist_nt<EV, 0>(st, a, P, sw);
 }
 
 // f32 coefficients of one type pair, as every pair kernel form uses them
@@ -1209,6 +1085,13 @@ static PairCoef pair_coef(double s, double e, double rc, double rs) {
 
 int hd_pair_table_max_types() { return PAIR_TAB_TYPES; }
 
+unsigned hd_pair_active_types(int nt, const double* sigma, const double* eps) {
+  unsigned m = 0;
+  for (int k = 0; k < nt * nt; ++k)
+    if (sigma[k] != 0.0 && eps[k] != 0.0) m |= 1u << (k / nt);
+  return m;
+}
+
 void hd_pair_lj_table(int nt, const double* sigma, const double* eps, const double* cut,
                       const double* rsw, float* out) {
   for (int k = 0; k < nt * nt; ++k) {
@@ -1230,8 +1113,8 @@ void hd_launch_pair(hipStream_t st, const HdPairArgs& a, int ev) {
     q[k] = pair_coef(a.sigma[k], a.eps[k], a.cut[k], a.rsw[k]);
     if (q[k].sw) any_switch = true;
   }
-  // up to four types the rows travel in the kernel arguments; beyond that
-  // the kernels read a.lj_tab (hd_pair_lj_table)
+  // atom lists: up to four types the rows travel in the kernel arguments;
+  // beyond that, and in the row-list kernel, a.lj_tab (hd_pair_lj_table)
   if (a.ntypes <= PAIR_MAXT)
     for (int k = 0; k < nt2; ++k) {
       P.c6[k] = q[k].c6;
@@ -1243,10 +1126,10 @@ void hd_launch_pair(hipStream_t st, const HdPairArgs& a, int ev) {
   P.kc = (float)a.kc;
   P.alpha = (float)a.alpha;
   P.coul_rc2 = a.coul_rc > 0.0 ? (float)(a.coul_rc * a.coul_rc) : -1.0f;
-  P.rmax2 = (float)(a.rmax * a.rmax);
-  P.spc_margin = (float)(a.rmax + 0.5 * a.r_skin);
-  P.excl_span = a.excl_span;
   P.ortho = a.ortho;
+  P.reach = (float)(a.rmax + 2.0 * a.r_skin + 1.0);
+  const unsigned act = hd_pair_active_types(a.ntypes, a.sigma, a.eps);
+  P.active_type = __builtin_popcount(act) <= 1 ? (act ? __builtin_ctz(act) : 0) : -1;
   bool uniform = P.coul_rc2 > 0.f && !any_switch;
   for (int k = 0; k < nt2; ++k)
     if (!(q[k].c6 == 0.f && q[k].c12 == 0.f) && q[k].cut2 != P.coul_rc2) uniform = false;

@@ -216,8 +216,7 @@ class Engine:
         self._chk(self._lib.hd_set_exclusion_span(self._ctx, int(span)), "hd_set_exclusion_span")
 
     def set_pair_list(self, mode):
-        """0: packed cluster list (half, j-side atomics); 1: per-atom full
-        lists."""
+        """0: row lists over 64-atom blocks; 1: per-atom full lists."""
         self._chk(self._lib.hd_set_pair_list(self._ctx, int(mode)), "hd_set_pair_list")
 
     def set_shake(self, groups):

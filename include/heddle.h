@@ -152,11 +152,11 @@ int hd_set_shake_tolerance(hd_ctx *ctx, double tol, double rattle_tol, int max_i
  * out[0..2] SHAKE total sweeps over all groups and calls, the largest
  * count, groups that hit the cap; out[3..5] the same for RATTLE. */
 int hd_get_constraint_stats(hd_ctx *ctx, uint64_t out[6]);
-/* Pair list form.  0: the packed 64-atom cluster list of the reference's
- * neighbour pipeline (kernels/neighbor.cu:416-631), half list with j-side
- * fixed-point atomics.  1: per-atom full lists, each pair listed from both
- * atoms and evaluated from both sides with no atomics (no counterpart in
- * the reference).  Both give the same forces to f32 rounding.  May be
+/* Pair list form.  0: row lists, the 64-atom blocks of the reference's
+ * neighbour pipeline (kernels/neighbor.cu:416-631) with one list of j-atoms
+ * per block and a row of indices into it per i-atom.  1: per-atom full
+ * lists, each pair listed from both atoms (no counterpart in the
+ * reference).  Both evaluate a pair from both sides.  Both give the same forces to f32 rounding.  May be
  * changed after hd_setup (the list is rebuilt). */
 int hd_set_pair_list(hd_ctx *ctx, int mode);
 /* Velocity Verlet (src/integrator/velocity_verlet.rs); lossless = the
@@ -415,7 +415,7 @@ int hd_get_lattice(hd_ctx *ctx, double lattice[6]);
  * energy, or minus the energy CSVR / Berendsen rescales injected),
  * out[6] neighbour rebuild count, out[7] neighbour status word. */
 int hd_get_scalars(hd_ctx *ctx, double out[8]);
-/* Canonical pair set of the current packed list: unique (min id, max id)
+/* Canonical pair set of the current list: unique (min id, max id)
  * pairs with min < max, excluding sentinels (neighbor_list.rs:1366-1506).
  * Returns the count in *n_pairs; writes at most cap pairs (2*cap u32). */
 int hd_get_pairs(hd_ctx *ctx, uint32_t *out, uint64_t cap, uint64_t *n_pairs);
