@@ -176,7 +176,7 @@ struct HdSpmeArgs {
   // voxel binning of the last neighbour rebuild (slot ranges per voxel)
   const unsigned *voxel_rank, *voxel_off;
   unsigned nv[3];
-  int mv[3];  // voxel margin per axis: >= half the skin in voxel units, plus one
+  float mv[3];  // voxel margin per axis: at least half the skin in voxel units
   int order;  // B-spline order, 4 or 5
   int splines_done;  // spl / sg already hold this evaluation's records
   int no_plane;      // FFT: separate c and b passes even where a plane fits in LDS

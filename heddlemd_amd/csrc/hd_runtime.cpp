@@ -546,8 +546,8 @@ static void enqueue_spme(hd_ctx* c, hipStream_t sst, bool timed, bool splines_do
   for (int d = 0; d < 3; ++d) {
     sa.nv[d] = c->nv[d];
     // atoms move at most r_skin/2 between rebuilds; 20 % slack for box
-    // changes since set-up, plus one voxel for the binning's rounding
-    sa.mv[d] = (int)floor(0.6 * c->r_skin * (double)c->nv[d] * inv_row_norm(c->lattice, d)) + 1;
+    // changes since set-up, and 1/64 voxel for the binning's rounding
+    sa.mv[d] = (float)(0.6 * c->r_skin * (double)c->nv[d] * inv_row_norm(c->lattice, d) + 0.015625);
   }
   stage_begin(c, "spme_recip", timed);
   if (c->dft_mode == 1) {
@@ -616,28 +616,19 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   // what it reads: it runs on the second stream, concurrent with them, and
   // joins before the finalize.  The stage-timing pass keeps one stream so
   // that every stage is timed alone.
-  //
-  // While the spread fits the chip (two workgroups per CU) it starts beside
-  // the build (24,576 atoms, 128 bricks: 152 us per step, 165 with the build
-  // first; 52,773 atoms, 250 bricks: 244 and 261).  A larger spread fills
-  // every CU's LDS, and the build's launch, idle on most steps, waited 30 to
-  // 40 us behind it: there the build goes first (196,608 atoms, 1,024
-  // bricks).
+  // Measured with the fork behind the build instead, us per pass: 24,576
+  // atoms 7320 (7030 here), 52,773 atoms 9900 (8940), 196,608 atoms 22280
+  // (20270).
   const bool fork = c->have_spme && !timed && c->spme_fork;
-  unsigned brick[3];
-  const bool fork_late =
-      fork && hd_spread_bricks(c->grid[0], c->grid[1], c->grid[2], brick) > 512u;
-  auto start_spme = [&] {
+  if (fork) {
     (void)hipEventRecord(c->ev_fork, st);
     (void)hipStreamWaitEvent(c->side, c->ev_fork, 0);
     enqueue_spme(c, c->side, false, small_nb);
     (void)hipEventRecord(c->ev_join, c->side);
-  };
-  if (fork && !fork_late) start_spme();
+  }
   stage_begin(c, "neighbor_build", timed);
   hd_launch_neighbor_build(st, na, !small_nb, small_nb);
   stage_end(c, timed);
-  if (fork_late) start_spme();
   HdPairArgs pa;
   memset(&pa, 0, sizeof(pa));
   pa.n = (unsigned)c->n;
