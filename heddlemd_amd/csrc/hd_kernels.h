@@ -55,7 +55,6 @@ struct HdNeighborArgs {
   unsigned excl_span;
   unsigned long long* block_mask;  // nblocks x hd_block_pair_chunks(nblocks) candidate masks
   unsigned* block_order;           // units by row chunks, heaviest first (rebuild steps)
-  unsigned* build_ticket;          // zeroed word for the folded rebuild-clear
 };
 unsigned hd_block_pair_chunks(unsigned nblocks);
 
@@ -65,28 +64,27 @@ void hd_launch_neighbor_update(hipStream_t st, const HdNeighborArgs& a, bool che
 void hd_launch_disp_check(hipStream_t st, const HdNeighborArgs& a);
 // number of chunk sums of the voxel-count scan (the buffer needs one more)
 unsigned hd_voxel_scan_parts(unsigned nvox);
-// block_pairs = false when hd_launch_neighbor_small already ran the
-// block-pair box tests of this step; fold_clear: with few units the row
-// build's last workgroup clears the rebuild request (no separate launch;
-// needs build_ticket)
-void hd_launch_neighbor_build(hipStream_t st, const HdNeighborArgs& a, bool block_pairs = true,
-                              bool fold_clear = false);
+// The list build; clear = false: the pair kernel that follows clears the
+// rebuild request (HdPairArgs::status) and the units keep their index order
+void hd_launch_neighbor_build(hipStream_t st, const HdNeighborArgs& a, bool clear = true);
+// up to this many units all run at once, so their order does not matter
+#define HD_ROW_UNORDERED 1024u
 void hd_launch_tile_gather(hipStream_t st, const float4* posq, const unsigned* sorted_id,
                            const float* lattice, float4* tile_posq, long long* fpj,
                            long long* fpj_ew, unsigned n, unsigned npad, float4* tile_ref,
                            unsigned char* tile_img);
 // the same, and on rebuild steps the slot types and keys and the blocks'
-// bounding boxes (which the neighbour build then uses)
+// bounding boxes (which the neighbour build then uses); spl != nullptr: also
+// the SPME spline records of a grid of na x nb x nc cells
 void hd_launch_tile_gather_rebuild(hipStream_t st, const HdNeighborArgs& a, long long* fpj,
-                                   long long* fpj_ew);
-// Systems of at most 8192 atoms and 8192 voxels: the displacement check
-// (when check), the gated voxel binning, the tile gather with its
-// rebuild-step extras and the block-pair box tests in one one-workgroup
-// launch, with the results of hd_launch_neighbor_update +
-// hd_launch_tile_gather_rebuild + the box tests of hd_launch_neighbor_build
+                                   long long* fpj_ew, float4* spl = nullptr,
+                                   unsigned* sg = nullptr, unsigned na = 0, unsigned nb = 0,
+                                   unsigned nc = 0);
+// Systems of at most 16384 atoms and 8192 voxels: the displacement check
+// (when check) and the gated voxel binning in one one-workgroup launch, which
+// for the smallest systems also does the tile gather, else launched behind
+// it; results as of hd_launch_neighbor_update + hd_launch_tile_gather_rebuild
 bool hd_neighbor_small(const HdNeighborArgs& a);
-// spl != nullptr: the gather also writes the SPME spline records of a grid
-// of na x nb x nc cells (k_spline_setup's output)
 void hd_launch_neighbor_small(hipStream_t st, const HdNeighborArgs& a, bool check, long long* fpj,
                               long long* fpj_ew, float4* spl = nullptr, unsigned* sg = nullptr,
                               unsigned na = 0, unsigned nb = 0, unsigned nc = 0);
@@ -109,6 +107,7 @@ struct HdPairArgs {
   int ortho;       // no box tilt
   unsigned parts, jcap, rcap;
   const unsigned *jslot, *jcount, *rowhdr;
+  unsigned *status, *rebuild_count;  // status: rebuild request to clear and count, or nullptr
   const unsigned char* tile_img;
   const unsigned short* rows;
   const unsigned* block_order;  // workgroup -> unit for the row-list kernel
@@ -178,11 +177,10 @@ struct HdSpmeArgs {
   unsigned nv[3];
   float mv[3];  // voxel margin per axis: at least half the skin in voxel units
   int order;  // B-spline order, 4 or 5
-  int splines_done;  // spl / sg already hold this evaluation's records
   int no_plane;      // FFT: separate c and b passes even where a plane fits in LDS
 };
 void hd_launch_spme(hipStream_t st, const HdSpmeArgs& a);
-// the spread half of hd_launch_spme (spline records + charge grid) alone
+// the charge grid alone
 void hd_launch_spme_spread(hipStream_t st, const HdSpmeArgs& a);
 void hd_launch_recip_reduce(hipStream_t st, const HdSpmeArgs& a, unsigned n_partials);
 

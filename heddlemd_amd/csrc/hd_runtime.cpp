@@ -435,7 +435,6 @@ HdNeighborArgs nb_args(hd_ctx* c) {
   a.max_count = c->ctrl + 2;
   a.status = c->ctrl;
   a.rebuild_count = c->ctrl + 1;
-  a.build_ticket = c->ctrl + 3;
   a.atom_lists = c->atom_lists;
   a.excl_span = c->excl_span;
   a.block_mask = c->block_mask;
@@ -513,10 +512,9 @@ void stage_end(hd_ctx* c, bool on) {
 }
 
 // The SPME reciprocal pipeline of one force evaluation, on stream sst.
-static void enqueue_spme(hd_ctx* c, hipStream_t sst, bool timed, bool splines_done) {
+static void enqueue_spme(hd_ctx* c, hipStream_t sst, bool timed) {
   HdSpmeArgs sa;
   memset(&sa, 0, sizeof(sa));
-  sa.splines_done = splines_done ? 1 : 0;
   sa.no_plane = c->dft_mode == 2 ? 1 : 0;
   sa.n = (unsigned)c->n;
   sa.order = c->spline_order;
@@ -595,20 +593,19 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   hipStream_t st = c->stream;
   HdNeighborArgs na = nb_args(c);
   const bool small_nb = c->small_neighbor && hd_neighbor_small(na);
+  float4* spl = c->have_spme ? c->spl : nullptr;
   if (small_nb) {
     stage_begin(c, "neighbor_update", timed);
-    if (c->have_spme)
-      hd_launch_neighbor_small(st, na, !disp_done, c->fpj, ev ? c->fpj_ew : nullptr, c->spl,
-                               c->sg, c->grid[0], c->grid[1], c->grid[2]);
-    else
-      hd_launch_neighbor_small(st, na, !disp_done, c->fpj, ev ? c->fpj_ew : nullptr);
+    hd_launch_neighbor_small(st, na, !disp_done, c->fpj, ev ? c->fpj_ew : nullptr, spl, c->sg,
+                             c->grid[0], c->grid[1], c->grid[2]);
     stage_end(c, timed);
   } else {
     stage_begin(c, "neighbor_update", timed);
     hd_launch_neighbor_update(st, na, !disp_done);
     stage_end(c, timed);
     stage_begin(c, "tile_gather", timed);
-    hd_launch_tile_gather_rebuild(st, na, c->fpj, ev ? c->fpj_ew : nullptr);
+    hd_launch_tile_gather_rebuild(st, na, c->fpj, ev ? c->fpj_ew : nullptr, spl, c->sg,
+                                  c->grid[0], c->grid[1], c->grid[2]);
     stage_end(c, timed);
   }
   // The SPME pipeline reads the tile positions, the lattice and the voxel
@@ -623,11 +620,12 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   if (fork) {
     (void)hipEventRecord(c->ev_fork, st);
     (void)hipStreamWaitEvent(c->side, c->ev_fork, 0);
-    enqueue_spme(c, c->side, false, small_nb);
+    enqueue_spme(c, c->side, false);
     (void)hipEventRecord(c->ev_join, c->side);
   }
   stage_begin(c, "neighbor_build", timed);
-  hd_launch_neighbor_build(st, na, !small_nb, small_nb);
+  const bool late_clear = !c->atom_lists && c->nblocks * c->parts <= HD_ROW_UNORDERED;
+  hd_launch_neighbor_build(st, na, !late_clear);
   stage_end(c, timed);
   HdPairArgs pa;
   memset(&pa, 0, sizeof(pa));
@@ -667,6 +665,8 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   pa.jslot = c->jslot;
   pa.tile_img = c->tile_img;
   pa.jcount = c->jcount;
+  pa.status = late_clear ? na.status : nullptr;
+  pa.rebuild_count = na.rebuild_count;
   pa.rowhdr = c->rowhdr;
   pa.rows = c->rows;
   stage_begin(c, "pair_force", timed);
@@ -686,7 +686,7 @@ void enqueue_forces(hd_ctx* c, int ev, bool kick, bool timed, bool disp_done = f
   if (fork)
     (void)hipStreamWaitEvent(st, c->ev_join, 0);
   else if (c->have_spme)
-    enqueue_spme(c, st, timed, small_nb);
+    enqueue_spme(c, st, timed);
   HdFinalizeArgs fa;
   memset(&fa, 0, sizeof(fa));
   fa.n = (unsigned)c->n;

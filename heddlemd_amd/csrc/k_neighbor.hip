@@ -40,6 +40,14 @@ __device__ __forceinline__ bool nb_rebuild_due_now(const unsigned* status) {
   return (*status & (NB_STATUS_REBUILD | NB_STATUS_FORCE)) != 0u;
 }
 
+// One atomic per launch in the main: waves that find the request set leave
+// it (device atomics on one word queue up, about 20 ns each).
+__device__ __forceinline__ void nb_request_rebuild(unsigned* status, bool over) {
+  if (__any(over) && (threadIdx.x & 63u) == 0 &&
+      !(*(volatile unsigned*)status & NB_STATUS_REBUILD))
+    atomicOr(status, NB_STATUS_REBUILD);
+}
+
 // Displacement check against the positions of the last rebuild.  A box
 // change since the rebuild (barostat) moves every minimum-image pair
 // vector by at most sqrt(3) * max|dL|, which is added to each atom's
@@ -61,7 +69,7 @@ __global__ void k_disp_check(const float4* __restrict__ posq, const float4* __re
     hd_min_image(dx, dy, dz, L);
     over = sqrtf(dx * dx + dy * dy + dz * dz) + 1.7320508f * dl > half_skin;
   }
-  if (__any(over) && (threadIdx.x & 63) == 0) atomicOr(status, NB_STATUS_REBUILD);
+  nb_request_rebuild(status, over);
 }
 
 // Curve rank of the fractional voxel that holds the atom (wrapped into the
@@ -342,11 +350,16 @@ __global__ void k_tile_gather(const float4* __restrict__ posq, const unsigned* _
                               unsigned* __restrict__ tile_type, unsigned* __restrict__ tile_key,
                               float4* __restrict__ center, float4* __restrict__ half,
                               float4* __restrict__ tile_ref,
-                              unsigned char* __restrict__ tile_img) {
+                              unsigned char* __restrict__ tile_img, float4* __restrict__ spl,
+                              unsigned* __restrict__ sg, unsigned gna, unsigned gnb,
+                              unsigned gnc) {
   unsigned s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= npad) return;  // whole waves: npad is a multiple of 64
   nb_gather_slot(s, status && nb_rebuild_due(status), posq, sorted_id, lattice, tile_posq, fpj,
                  fpj_ew, n, type, key, tile_type, tile_key, center, half, tile_ref, tile_img);
+  // the SPME spline record of the slot the thread has just written
+  if (spl && s < n)
+    hd_spline_record(tile_posq[s], hd_load_lattice(lattice), gna, gnb, gnc, spl, sg, s);
 }
 
 
@@ -417,17 +430,19 @@ __global__ void __launch_bounds__(256) k_block_pairs(const float4* __restrict__ 
 }
 
 // Systems of at most NB_SMALL_ATOMS atoms and NB_SMALL_VOX voxels: the
-// displacement check, the rebuild's voxel binning (keys, histogram, scan,
-// scatter, per-voxel sort), the tile gather (with the SPME spline records
-// when asked) and the block-pair box tests run in one workgroup, with
-// barriers between the phases in place of the nine launches of the general
-// path.  The histogram and the scatter cursors live in LDS (the
+// displacement check and the rebuild's voxel binning (keys, histogram, scan,
+// scatter, per-voxel sort) run in one workgroup, with barriers between the
+// phases in place of the general path's six launches.  Up to NB_SMALL_GATHER
+// atoms the tile gather (with the SPME spline records when asked) runs there
+// too; beyond that one CU takes longer over it than a launch of its own
+// costs (7,938 atoms: 29 us for everything in one workgroup, 7.4 + 4.2 apart).  The histogram and the scatter cursors live in LDS (the
 // global voxel_count stays zero, as the general path leaves it).  Results
 // are those of the general path: the per-atom arithmetic is shared with its
 // kernels, the scan is exact and the per-voxel sort makes the slot order
 // independent of the order of the atomics.
 #define NB_SMALL_THREADS 1024u
-#define NB_SMALL_ATOMS 8192u
+#define NB_SMALL_ATOMS 16384u
+#define NB_SMALL_GATHER 1024u
 #define NB_SMALL_VOX 8192u
 
 __global__ void __launch_bounds__(NB_SMALL_THREADS) k_nb_small(HdNeighborArgs a, int check,
@@ -450,16 +465,15 @@ __global__ void __launch_bounds__(NB_SMALL_THREADS) k_nb_small(HdNeighborArgs a,
 #pragma unroll
     for (int k = 0; k < 6; ++k) dl = fmaxf(dl, fabsf(a.lattice[k] - a.ref_lattice[k]));
     bool over = false;
+#pragma unroll 4
     for (unsigned i = t; i < a.n; i += NB_SMALL_THREADS) {
       float4 p = a.posq[i], r = a.ref_pos[i];
       float dx = p.x - r.x, dy = p.y - r.y, dz = p.z - r.z;
       hd_min_image(dx, dy, dz, L);
-      over = over || sqrtf(dx * dx + dy * dy + dz * dz) + 1.7320508f * dl > a.half_skin;
+      over |= sqrtf(dx * dx + dy * dy + dz * dz) + 1.7320508f * dl > a.half_skin;
     }
-    if (__any(over) && (t & 63u) == 0) {
-      atomicOr(a.status, NB_STATUS_REBUILD);
-      s_over = 1;
-    }
+    nb_request_rebuild(a.status, over);
+    if (over) s_over = 1;
   }
   __syncthreads();
   // one thread decides and every thread reads its decision, so the
@@ -512,6 +526,7 @@ __global__ void __launch_bounds__(NB_SMALL_THREADS) k_nb_small(HdNeighborArgs a,
       nb_sort_voxel(v, a.voxel_off, a.sorted_id, a.slot_of);
     __syncthreads();
   }
+  if (a.n > NB_SMALL_GATHER) return;  // k_tile_gather follows
   // npad is a multiple of 64 and so is the stride: each wave covers whole
   // blocks in every pass
   for (unsigned s = t; s < a.npad; s += NB_SMALL_THREADS)
@@ -523,13 +538,6 @@ __global__ void __launch_bounds__(NB_SMALL_THREADS) k_nb_small(HdNeighborArgs a,
     for (unsigned s = t; s < a.n; s += NB_SMALL_THREADS)
       hd_spline_record(a.tile_posq[s], L, gna, gnb, gnc, spl, sg, s);
   }
-  if (!rebuild) return;
-  __syncthreads();
-  // the box tests read every block's bounding box from the gather
-  const unsigned nblocks = a.npad / 64u, nchunks = (nblocks + 63u) / 64u;
-  for (unsigned wv = t >> 6; wv < nblocks * nchunks; wv += NB_SMALL_THREADS / 64u)
-    nb_block_pair_item(wv, a.center, a.half, L, a.rs2 * NB_BOX_MARGIN, a.block_mask, nblocks,
-                       nchunks);
 }
 
 bool hd_neighbor_small(const HdNeighborArgs& a) {
@@ -541,6 +549,8 @@ void hd_launch_neighbor_small(hipStream_t st, const HdNeighborArgs& a, bool chec
                               unsigned nb, unsigned nc) {
   hipLaunchKernelGGL(k_nb_small, dim3(1), dim3(NB_SMALL_THREADS), 0, st, a, check ? 1 : 0, fpj,
                      fpj_ew, spl, sg, na, nb, nc);
+  if (a.n > NB_SMALL_GATHER)
+    hd_launch_tile_gather_rebuild(st, a, fpj, fpj_ew, spl, sg, na, nb, nc);
 }
 
 #define NB_CAND_MAX 1024
@@ -607,11 +617,15 @@ __device__ __forceinline__ unsigned nb_collect(const unsigned long long* __restr
 // at 196,608 atoms and 0.14 nm, where that took 190.  The list is a pure
 // function of the positions.
 #define NB_PER_WAVE 2u
+// Up to this many mask words per block (512 blocks, one pass over them) a
+// unit tests every block's box itself: the mask's launch costs more than it
+// saves there (24,576 atoms, a frame with its rebuild: 417 us, 440 with the
+// mask; 10,000 argon atoms, a step: 29.5 and 31.7)
+#define NB_MASK_CHUNKS 8u
 #define NB_ROUND (HD_ROW_WAVES * NB_PER_WAVE)
 #define NB_STAGE 96u         // entries of a row staged in LDS: a rest below 32 and 64 hits
 #define NB_WORDS_MAX 512u    // mask words (64 blocks each) with candidates
 #define NB_IMAGES_MAX 1024u  // images listed from 512 blocks at a time
-#define NB_FOLD_MAX_UNITS 1024u  // unit counts whose build also clears the request
 
 __device__ __forceinline__ unsigned nb_scan512(unsigned v, unsigned* wsum, unsigned& total) {
   const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
@@ -681,11 +695,6 @@ __device__ __forceinline__ unsigned nb_images(float4 ci, float4 hi, float4 cj, f
   return m;
 }
 
-// FOLD (few units): the workgroup that takes the last ticket (*ticket, 0
-// between launches) clears the rebuild request and counts the rebuild once
-// every unit's list is written, in place of k_rebuild_clear; the units of
-// such a system all run at once, so they keep their index order.
-template <bool FOLD>
 __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs a,
                                                                   unsigned nchunks) {
   if (!nb_rebuild_due_now(a.status)) return;
@@ -705,11 +714,12 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
   const float4 cb = a.center[b], hb = a.half[b];
   const float rs2 = a.rs2 * NB_BOX_MARGIN, rs2p = a.rs2 * NB_ROW_MARGIN;
   if (t == 0) s_cost = s_need = 0u;
-  // 1. the mask words with candidates
+  // 1. the mask words with candidates (few blocks have no mask: all of them)
+  const bool all = nchunks <= NB_MASK_CHUNKS;
   unsigned nw = 0;
   for (unsigned base = 0; base < nchunks; base += HD_ROW_THREADS) {
     const unsigned c = base + t;
-    const bool nz = c < nchunks && a.block_mask[(size_t)b * nchunks + c] != 0ull;
+    const bool nz = c < nchunks && (all || a.block_mask[(size_t)b * nchunks + c] != 0ull);
     unsigned total;
     const unsigned o = nw + nb_scan512(nz ? 1u : 0u, wsum, total);
     if (nz && o < NB_WORDS_MAX) words[o] = c;
@@ -766,8 +776,11 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
       if (w0 + w < nw) {
         const unsigned c = words[w0 + w];
         jb = c * 64u + lane;
-        if ((a.block_mask[(size_t)b * nchunks + c] >> lane) & 1ull)
-          m = nb_images(cb, hb, a.center[jb], a.half[jb], L, rs2);
+        if (all ? jb < a.npad / 64u : (a.block_mask[(size_t)b * nchunks + c] >> lane) & 1ull) {
+          const float4 cj = a.center[jb], hj = a.half[jb];
+          // without a mask its test comes first: most waves end there
+          if (!all || nb_box_dist2(cb, hb, cj, hj, L) <= rs2) m = nb_images(cb, hb, cj, hj, L, rs2);
+        }
       }
       unsigned o = nb_scan512((unsigned)__popc(m), wsum, ne);
       for (; m; m &= m - 1u, ++o)
@@ -1009,15 +1022,6 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
       bits = NB_STATUS_HIGHWATER;
     if (bits & ~*(volatile unsigned*)a.status) atomicOr(a.status, bits);
   }
-  if (!FOLD) return;
-  if (t == 0) {
-    __threadfence();
-    if (atomicAdd(a.build_ticket, 1u) == gridDim.x - 1u) {
-      atomicAnd(a.status, ~(NB_STATUS_REBUILD | NB_STATUS_FORCE));
-      atomicAdd(a.rebuild_count, 1u);
-      atomicExch(a.build_ticket, 0u);
-    }
-  }
 }
 
 // Per-atom full lists (the atom-list mode): one wave per i-block, lane =
@@ -1211,28 +1215,28 @@ void hd_launch_tile_gather(hipStream_t st, const float4* posq, const unsigned* s
                            unsigned char* tile_img) {
   hipLaunchKernelGGL(k_tile_gather, dim3(cdiv(npad, 256)), dim3(256), 0, st, posq, sorted_id,
                      lattice, tile_posq, fpj, fpj_ew, n, npad, nullptr, nullptr, nullptr,
-                     nullptr, nullptr, nullptr, nullptr, tile_ref, tile_img);
+                     nullptr, nullptr, nullptr, nullptr, tile_ref, tile_img, nullptr, nullptr,
+                     0u, 0u, 0u);
 }
 
 void hd_launch_tile_gather_rebuild(hipStream_t st, const HdNeighborArgs& a, long long* fpj,
-                                   long long* fpj_ew) {
+                                   long long* fpj_ew, float4* spl, unsigned* sg, unsigned na,
+                                   unsigned nb, unsigned nc) {
   hipLaunchKernelGGL(k_tile_gather, dim3(cdiv(a.npad, 256)), dim3(256), 0, st, a.posq,
                      a.sorted_id, a.lattice, a.tile_posq, fpj, fpj_ew, a.n, a.npad, a.status,
                      a.type, a.key, a.tile_type, a.tile_key, a.center, a.half, a.tile_ref,
-                     a.tile_img);
+                     a.tile_img, spl, sg, na, nb, nc);
 }
 
 unsigned hd_block_pair_chunks(unsigned nblocks) { return cdiv(nblocks, 64); }
 
-void hd_launch_neighbor_build(hipStream_t st, const HdNeighborArgs& a, bool block_pairs,
-                              bool fold_clear) {
+void hd_launch_neighbor_build(hipStream_t st, const HdNeighborArgs& a, bool clear) {
   unsigned nblocks = a.npad / 64;
   const unsigned units = a.atom_lists ? nblocks : nblocks * a.parts;
-  const bool fold = fold_clear && !a.atom_lists && units <= NB_FOLD_MAX_UNITS;
   const size_t lds = (size_t)a.jcap * sizeof(float4);
   unsigned nchunks = hd_block_pair_chunks(nblocks);
   unsigned pair_waves = min(nblocks * nchunks, (unsigned)NB_PAIR_WAVES);
-  if (block_pairs)
+  if (a.atom_lists || nchunks > NB_MASK_CHUNKS)
     hipLaunchKernelGGL(k_block_pairs, dim3(cdiv(pair_waves * 64, 256)), dim3(256), 0, st,
                        a.center, a.half, a.lattice, a.rs2 * NB_BOX_MARGIN, a.block_mask, nblocks,
                        nchunks, a.status);
@@ -1241,11 +1245,9 @@ void hd_launch_neighbor_build(hipStream_t st, const HdNeighborArgs& a, bool bloc
                        a.tile_posq, a.tile_key, a.excl_span, a.center, a.half, a.lattice, a.rs2,
                        a.block_mask, nchunks, a.entry_atoms, a.entry_count, a.cap, a.max_count,
                        a.status, a.n, nblocks);
-  else if (fold)
-    hipLaunchKernelGGL(k_build_rows<true>, dim3(units), dim3(HD_ROW_THREADS), lds, st, a, nchunks);
   else
-    hipLaunchKernelGGL(k_build_rows<false>, dim3(units), dim3(HD_ROW_THREADS), lds, st, a, nchunks);
-  if (!fold)
+    hipLaunchKernelGGL(k_build_rows, dim3(units), dim3(HD_ROW_THREADS), lds, st, a, nchunks);
+  if (clear)
     hipLaunchKernelGGL(k_rebuild_clear, dim3(1), dim3(NB_ORDER_BINS), 0, st, a.status,
                        a.rebuild_count, a.entry_count, units, a.block_order);
 }

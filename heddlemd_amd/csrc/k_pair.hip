@@ -359,7 +359,19 @@ __global__ void __launch_bounds__(HD_ROW_THREADS) k_pair_rows(
     const unsigned* __restrict__ rowhdr,
     const unsigned short* __restrict__ rows, const unsigned* __restrict__ order, unsigned parts,
     unsigned jcap, unsigned rcap, unsigned n, unsigned long long* __restrict__ fpj,
-    unsigned long long* __restrict__ fpj_ew, const float4* __restrict__ lj_tab) {
+    unsigned long long* __restrict__ fpj_ew, const float4* __restrict__ lj_tab, unsigned* status,
+    unsigned* rebuild_count) {
+  // End of a rebuild with few units: the request is cleared and counted here
+  // (nothing that runs beside this launch reads it).  A launch of its own cost
+  // 2.5 us of every step (10,000 argon atoms); a ticket in the build, whose
+  // units then wait for the returned count, 30 us of every rebuild.
+  if (status && blockIdx.x == 0 && threadIdx.x == 0) {
+    const unsigned s = *(volatile unsigned*)status;
+    if (s & (NB_STATUS_REBUILD | NB_STATUS_FORCE)) {
+      atomicAnd(status, ~(NB_STATUS_REBUILD | NB_STATUS_FORCE));
+      *rebuild_count += 1u;
+    }
+  }
   extern __shared__ float4 lds[];
   int4* jrec = reinterpret_cast<int4*>(lds);
   const unsigned nt2 = (unsigned)(P.ntypes * P.ntypes);
@@ -1035,12 +1047,14 @@ static void launch_rows_c(hipStream_t st, const HdPairArgs& a, const PairParams&
     hipLaunchKernelGGL((k_pair_rows<EV, KIND, true>), grid, wg, lds, st, P, a.lattice,
                        a.tile_posq, a.tile_type, a.tile_img, a.center, a.half, a.jslot, a.jcount,
                        a.rowhdr, a.rows, a.block_order, a.parts, a.jcap, a.rcap, a.n,
-                       (unsigned long long*)a.fpj, (unsigned long long*)a.fpj_ew, a.lj_tab);
+                       (unsigned long long*)a.fpj, (unsigned long long*)a.fpj_ew, a.lj_tab,
+                       a.status, a.rebuild_count);
   else
     hipLaunchKernelGGL((k_pair_rows<EV, KIND, false>), grid, wg, lds, st, P, a.lattice,
                        a.tile_posq, a.tile_type, a.tile_img, a.center, a.half, a.jslot, a.jcount,
                        a.rowhdr, a.rows, a.block_order, a.parts, a.jcap, a.rcap, a.n,
-                       (unsigned long long*)a.fpj, (unsigned long long*)a.fpj_ew, a.lj_tab);
+                       (unsigned long long*)a.fpj, (unsigned long long*)a.fpj_ew, a.lj_tab,
+                       a.status, a.rebuild_count);
 }
 
 template <int EV, int NT>

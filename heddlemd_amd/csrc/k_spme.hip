@@ -49,20 +49,12 @@ __device__ __forceinline__ float bspline_w(float x) {
   return v[0];
 }
 
-// Spline records, once per step in slot order: the FP64 spline origin
-// (hd_spline_origin) of every charged atom, as (t_a, t_b, t_c, q) plus
-// the packed origin cell g_a | g_b << 10 | g_c << 20 (SPME_NO_CELL for
-// uncharged atoms).  Read by the spread and by the force gather.
+// Spline records, once per step in slot order, written with the tile gather
+// (k_neighbor.hip): the FP64 spline origin (hd_spline_origin) of every
+// charged atom, as (t_a, t_b, t_c, q) plus the packed origin cell
+// g_a | g_b << 10 | g_c << 20 (SPME_NO_CELL for uncharged atoms).  Read by
+// the spread and by the force gather.
 #define SPME_NO_CELL HD_SPME_NO_CELL
-
-__global__ void k_spline_setup(const float4* __restrict__ tile_posq,
-                               const float* __restrict__ lattice, unsigned na, unsigned nb,
-                               unsigned nc, float4* __restrict__ spl, unsigned* __restrict__ sg,
-                               unsigned n) {
-  unsigned s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  hd_spline_record(tile_posq[s], hd_load_lattice(lattice), na, nb, nc, spl, sg, s);
-}
 
 // Spread: the reference accumulates each atom's p^3 contributions with
 // i64 atomics at 2^32, rounded to nearest (spme_spread_gather.cuh:151-221).
@@ -919,9 +911,6 @@ static unsigned ilog2u(unsigned v) {
 void hd_launch_spme_spread(hipStream_t st, const HdSpmeArgs& a) {
   unsigned brick[3];
   unsigned nbricks = hd_spread_bricks(a.na, a.nb, a.nc, brick);
-  if (a.n > 0 && !a.splines_done)
-    hipLaunchKernelGGL(k_spline_setup, dim3((a.n + 255) / 256), dim3(256), 0, st, a.tile_posq,
-                       a.lattice, a.na, a.nb, a.nc, a.spl, a.sg, a.n);
   if (a.order == 5)
     hipLaunchKernelGGL(k_spread<5>, dim3(nbricks), dim3(SPREAD_THREADS), 0, st, a.spl, a.sg,
                        a.na, a.nb, a.nc, brick[0], brick[1], brick[2], a.voxel_rank, a.voxel_off,

@@ -326,8 +326,8 @@ class Engine:
         self._chk(self._lib.hd_set_fused_settle(self._ctx, 1 if on else 0), "hd_set_fused_settle")
 
     def set_small_neighbor(self, on):
-        """Small systems: neighbour check, binning and gather in one
-        workgroup (default) or the general multi-kernel path (identical
+        """Small systems: neighbour check and binning in one workgroup
+        (default) or the general multi-kernel path (identical
         results)."""
         self._chk(self._lib.hd_set_small_neighbor(self._ctx, 1 if on else 0),
                   "hd_set_small_neighbor")

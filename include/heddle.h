@@ -298,9 +298,9 @@ int hd_use_graph(hd_ctx *ctx, int enable);
  * kernels run as one.  0 runs the separate kernels, with bit-identical
  * results.  No reference counterpart. */
 int hd_set_fused_settle(hd_ctx *ctx, int enable);
-/* Systems of at most 8192 atoms run the neighbour displacement check, the
- * rebuild's voxel binning and the slot-order gather in one one-workgroup
- * kernel (default on); 0 takes the general multi-kernel path, with
+/* Systems of at most 16384 atoms run the neighbour displacement check and
+ * the rebuild's voxel binning (up to 1024 atoms also the slot-order gather)
+ * in one one-workgroup kernel (default on); 0 takes the general multi-kernel path, with
  * identical results.  No reference counterpart. */
 int hd_set_small_neighbor(hd_ctx *ctx, int enable);
 int hd_sync(hd_ctx *ctx);
