@@ -17,7 +17,9 @@ constexpr int F = HD_MLP_IN;
 constexpr int H = HD_MLP_H;
 constexpr int NS = HD_MLP_SAMPLES;
 constexpr int HP = H + 1;  // padded LDS row pitch (conflict-free column reads)
-constexpr int QS = NS / 4; // samples per wave of a 256-thread block
+constexpr int GW = 16;      // waves of a gradient block
+constexpr int QS = NS / GW; // samples per wave
+constexpr int RB = 64;      // partials a reduction thread has in flight
 
 // nu1 columns (0..4) and rho (7) in units of the scale; the couplings
 // (5, 6) are O(1) already
@@ -75,10 +77,32 @@ __global__ __launch_bounds__(256) void k_mlp_predict(const float* __restrict__ P
   }
 }
 
-// One block = 64 samples, 256 threads (4 waves).  Forward activations stay
-// in LDS and are overwritten in place by their gradients; lane = hidden
-// unit throughout, so every LDS row access is contiguous or a broadcast.
-__global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ P,
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// One wave's 16 x 16 tile (wave / 4, wave % 4) of a 64 x 64 x 64 product in
+// f32 on the matrix cores: a(row, k), b(k, col), c = the initial values.
+// Lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] of every step of
+// four k and returns rows 16 (wave / 4) + 4 (l / 16) + r, column
+// 16 (wave % 4) + l % 16.
+template <class A, class B>
+__device__ __forceinline__ f32x4 tile64(A a, B b, f32x4 c) {
+  const unsigned lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+  const unsigned m = 16u * (wv >> 2) + (lane & 15u), n = 16u * (wv & 3u) + (lane & 15u);
+#pragma unroll
+  for (unsigned k0 = 0; k0 < (unsigned)H; k0 += 4u) {
+    const unsigned k = k0 + (lane >> 4);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a(m, k), b(k, n), c, 0, 0, 0);
+  }
+  return c;
+}
+static_assert(NS == 64 && H == 64 && GW == 16, "tile64 covers 64 x 64 with 16 waves");
+
+// One block = 64 samples, 1,024 threads (16 waves).  Forward activations stay
+// in LDS and are overwritten in place by their gradients.  The three 64 x
+// 64 x 64 products run on the matrix cores in f32: as multiply-adds of
+// broadcast LDS reads they kept the LDS busy for 22 us with these 16 waves
+// (27 with 4); now 13, a chain of short phases.
+__global__ __launch_bounds__(1024) void k_mlp_grad(const float* __restrict__ P,
                                                   const float* __restrict__ X,
                                                   const float* __restrict__ T, uint64_t n,
                                                   uint64_t first, unsigned count, uint64_t mul,
@@ -93,8 +117,10 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ P,
   __shared__ float h2[NS * HP];  // tanh of layer 2, then dL/d(pre-activation 2)
   __shared__ unsigned valid[NS];
   const unsigned t = threadIdx.x, lane = t & 63u, wv = t >> 6;
-  for (unsigned i = t; i < HD_MLP_NPARAM; i += 256) w[i] = P[i];
-  for (unsigned e = t; e < H * H; e += 256) {
+  // the lane's rows (row + r, r < 4) and column of the wave's tile
+  const unsigned row = 16u * (wv >> 2) + 4u * (lane >> 4), col = 16u * (wv & 3u) + (lane & 15u);
+  for (unsigned i = t; i < HD_MLP_NPARAM; i += 64 * GW) w[i] = P[i];
+  for (unsigned e = t; e < H * H; e += 64 * GW) {
     unsigned j = e / H, i = e % H;
     w2t[i * HP + j] = P[HD_MLP_W2 + e];
   }
@@ -119,14 +145,14 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ P,
     valid[t] = ok;
   }
   __syncthreads();
-  // layer 1: unit = lane, samples wv + 4 q
+  // layer 1: unit = lane, samples wv + 16 q
   {
     float wr[F];
 #pragma unroll
     for (int f = 0; f < F; ++f) wr[f] = w[HD_MLP_W1 + lane * F + f];
     float b = w[HD_MLP_B1 + lane];
     for (int q = 0; q < QS; ++q) {
-      unsigned sm = wv + 4u * q;
+      unsigned sm = wv + (unsigned)GW * q;
       float acc = b;
 #pragma unroll
       for (int f = 0; f < F; ++f) acc += wr[f] * u[sm][f];
@@ -134,24 +160,20 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ P,
     }
   }
   __syncthreads();
-  // layer 2
+  // layer 2: pre-activation [s][j] = b2[j] + sum_i h1[s][i] W2[j][i]
   {
-    float acc[QS];
-    float b = w[HD_MLP_B2 + lane];
+    const float b = w[HD_MLP_B2 + col];
+    const f32x4 d = tile64([&](unsigned s, unsigned i) { return h1[s * HP + i]; },
+                           [&](unsigned i, unsigned j) { return w2t[i * HP + j]; },
+                           f32x4{b, b, b, b});
 #pragma unroll
-    for (int q = 0; q < QS; ++q) acc[q] = b;
-    for (int i = 0; i < H; ++i) {
-      float wji = w2t[i * HP + lane];
-#pragma unroll
-      for (int q = 0; q < QS; ++q) acc[q] += wji * h1[(wv + 4u * q) * HP + i];
-    }
-#pragma unroll
-    for (int q = 0; q < QS; ++q) h2[(wv + 4u * q) * HP + lane] = tanhf(acc[q]);
+    for (int r = 0; r < 4; ++r) h2[(row + r) * HP + col] = tanhf(d[r]);
   }
   __syncthreads();
   // output, residual, dL/do
   if (t < NS) {
     float o = w[HD_MLP_B3];
+#pragma unroll 8
     for (int j = 0; j < H; ++j) o += w[HD_MLP_W3 + j] * h2[t * HP + j];
     float r = o - tgt[t];
     tgt[t] = valid[t] ? 2.0f * r * inv_count : 0.f;
@@ -161,10 +183,12 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ P,
   float* out = part + (size_t)blockIdx.x * HD_MLP_PSTRIDE;
   if (t < H) {
     float g = 0.f;
+#pragma unroll 8
     for (int sm = 0; sm < NS; ++sm) g += tgt[sm] * h2[sm * HP + t];
     out[HD_MLP_W3 + t] = g;
   } else if (t == H) {
     float g = 0.f, l = 0.f;
+#pragma unroll 8
     for (int sm = 0; sm < NS; ++sm) { g += tgt[sm]; l += sq[sm]; }
     out[HD_MLP_B3] = g;
     out[HD_MLP_NTRAIN] = l;
@@ -174,75 +198,71 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ P,
   {
     float w3 = w[HD_MLP_W3 + lane];
     for (int q = 0; q < QS; ++q) {
-      unsigned sm = wv + 4u * q;
+      unsigned sm = wv + (unsigned)GW * q;
       float hv = h2[sm * HP + lane];
       h2[sm * HP + lane] = tgt[sm] * w3 * (1.0f - hv * hv);
     }
   }
   __syncthreads();
-  // gW2[j][i] = sum_s D2[s][j] h1[s][i]: i = lane, j = 16 wv + q
+  // gW2[j][i] = sum_s D2[s][j] h1[s][i]
   {
-    float acc[16];
+    const f32x4 d = tile64([&](unsigned j, unsigned s) { return h2[s * HP + j]; },
+                           [&](unsigned s, unsigned i) { return h1[s * HP + i]; },
+                           f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = 0.f;
-    for (int sm = 0; sm < NS; ++sm) {
-      float hv = h1[sm * HP + lane];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) acc[q] += h2[sm * HP + 16u * wv + q] * hv;
-    }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) out[HD_MLP_W2 + (16u * wv + q) * H + lane] = acc[q];
+    for (int r = 0; r < 4; ++r) out[HD_MLP_W2 + (row + r) * H + col] = d[r];
     if (wv == 0) {
       float g = 0.f;
+#pragma unroll 8
       for (int sm = 0; sm < NS; ++sm) g += h2[sm * HP + lane];
       out[HD_MLP_B2 + lane] = g;
     }
   }
   __syncthreads();
-  // dL/d(pre-activation 1) in place of h1: unit i = lane
+  // dL/d(pre-activation 1) in place of h1:
+  // [s][i] = sum_j D2[s][j] W2[j][i] (1 - h1[s][i]^2)
   {
-    float acc[QS];
+    const f32x4 d = tile64([&](unsigned s, unsigned j) { return h2[s * HP + j]; },
+                           [&](unsigned j, unsigned i) { return w[HD_MLP_W2 + j * H + i]; },
+                           f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-    for (int q = 0; q < QS; ++q) acc[q] = 0.f;
-    for (int j = 0; j < H; ++j) {
-      float wji = w[HD_MLP_W2 + j * H + lane];
-#pragma unroll
-      for (int q = 0; q < QS; ++q) acc[q] += h2[(wv + 4u * q) * HP + j] * wji;
-    }
-#pragma unroll
-    for (int q = 0; q < QS; ++q) {
-      unsigned sm = wv + 4u * q;
-      float hv = h1[sm * HP + lane];
-      h1[sm * HP + lane] = acc[q] * (1.0f - hv * hv);
+    for (int r = 0; r < 4; ++r) {
+      const float hv = h1[(row + r) * HP + col];
+      h1[(row + r) * HP + col] = d[r] * (1.0f - hv * hv);
     }
   }
   __syncthreads();
-  // gW1[i][f] = sum_s D1[s][i] u[s][f]: i = lane, f = 2 wv, 2 wv + 1
-  {
-    float g0 = 0.f, g1 = 0.f;
-    unsigned f0 = 2u * wv;
-    for (int sm = 0; sm < NS; ++sm) {
-      float d = h1[sm * HP + lane];
-      g0 += d * u[sm][f0];
-      g1 += d * u[sm][f0 + 1];
-    }
-    out[HD_MLP_W1 + lane * F + f0] = g0;
-    out[HD_MLP_W1 + lane * F + f0 + 1] = g1;
-    if (wv == 0) {
-      float g = 0.f;
-      for (int sm = 0; sm < NS; ++sm) g += h1[sm * HP + lane];
-      out[HD_MLP_B1 + lane] = g;
-    }
+  // gW1[i][f] = sum_s D1[s][i] u[s][f]: i = lane, f = wv; then gB1
+  if (wv < (unsigned)F) {
+    float g = 0.f;
+#pragma unroll 8
+    for (int sm = 0; sm < NS; ++sm) g += h1[sm * HP + lane] * u[sm][wv];
+    out[HD_MLP_W1 + lane * F + wv] = g;
+  } else if (wv == (unsigned)F) {
+    float g = 0.f;
+#pragma unroll 8
+    for (int sm = 0; sm < NS; ++sm) g += h1[sm * HP + lane];
+    out[HD_MLP_B1 + lane] = g;
   }
 }
 
+// One parameter per thread, its partials in block order, RB loads in flight
+// (one at a time, 64 partials took 27 us of latency; now 6.9).
 __global__ void k_mlp_reduce(const float* __restrict__ part, unsigned nb, float* __restrict__ P,
                              float* __restrict__ grad_out, HdAdam adam, int use_adam,
                              double* __restrict__ loss_acc) {
   unsigned p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p < HD_MLP_NTRAIN) {
     float g = 0.f;
-    for (unsigned b = 0; b < nb; ++b) g += part[(size_t)b * HD_MLP_PSTRIDE + p];
+    unsigned b = 0;
+    for (; b + RB <= nb; b += RB) {
+      float v[RB];
+#pragma unroll
+      for (int k = 0; k < RB; ++k) v[k] = part[(size_t)(b + k) * HD_MLP_PSTRIDE + p];
+#pragma unroll
+      for (int k = 0; k < RB; ++k) g += v[k];
+    }
+    for (; b < nb; ++b) g += part[(size_t)b * HD_MLP_PSTRIDE + p];
     if (grad_out) grad_out[p] = g;
     if (use_adam) {
       float m = adam.b1 * adam.m[p] + (1.0f - adam.b1) * g;
@@ -253,6 +273,7 @@ __global__ void k_mlp_reduce(const float* __restrict__ part, unsigned nb, float*
     }
   } else if (p == HD_MLP_NTRAIN && loss_acc) {
     double l = 0.0;
+#pragma unroll 8
     for (unsigned b = 0; b < nb; ++b) l += (double)part[(size_t)b * HD_MLP_PSTRIDE + p];
     loss_acc[0] += l;
   }
@@ -262,7 +283,16 @@ __global__ __launch_bounds__(1024) void k_mlp_scale(const float* __restrict__ x,
                                                     float* __restrict__ P) {
   __shared__ double red[1024];
   double acc = 0.0;
-  for (uint64_t i = threadIdx.x; i < n; i += 1024) {
+  uint64_t i = threadIdx.x;
+  // 16 rows in flight per thread: 200,003 rows took 116 us one at a time
+  for (; i + 15u * 1024u < n; i += 16u * 1024u) {
+    float v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = x[(i + 1024u * k) * F];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc += (double)v[k] * (double)v[k];
+  }
+  for (; i < n; i += 1024) {
     double v = x[i * F];
     acc += v * v;
   }
@@ -312,7 +342,7 @@ unsigned hd_launch_mlp_grad(hipStream_t st, const float* params, const float* x,
                             uint64_t mul, uint64_t add, float inv_count, float* partials) {
   unsigned nb = (count + NS - 1) / NS;
   if (nb == 0) return 0;
-  hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), 0, st, params, x, t, n, first, count, mul,
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(64 * GW), 0, st, params, x, t, n, first, count, mul,
                      add, inv_count, partials);
   return nb;
 }
