@@ -2221,11 +2221,13 @@ static int alloc_rows(hd_ctx* c, unsigned parts, unsigned jcap, unsigned rcap) {
   return HD_OK;
 }
 
-// Largest j-list of a unit: 64 KB of LDS for its records beside the build's
-// candidate lists and the pair kernel's type table
+// Largest j-list of a unit: half a CU's LDS (the build's registers allow two
+// workgroups) for its records beside the build's candidate lists and the pair
+// kernel's type table
 static unsigned rows_jcap_max(const hd_ctx* c) {
-  unsigned build = (65536u - 21u * 1024u) / 16u;
-  unsigned pair = (65536u - hd_pair_rows_lds(c->ntypes, 0) - 64u) / (c->ntypes > 1 ? 17u : 16u);
+  const unsigned lds = 81920u;
+  unsigned build = (lds - 21u * 1024u) / 16u;
+  unsigned pair = (lds - hd_pair_rows_lds(c->ntypes, 0) - 64u) / (c->ntypes > 1 ? 17u : 16u);
   return std::min(std::min(build, pair), HD_ROW_JMAX) & ~7u;
 }
 
@@ -2261,7 +2263,7 @@ static int size_rows(hd_ctx* c) {
   const unsigned jmax = rows_jcap_max(c);
   double gj, gr;
   rows_guess(c, parts, &gj, &gr);
-  unsigned jcap = std::min(std::max(floor_j, (unsigned)std::min(1.8 * gj + 128.0, 1e6) & ~7u), jmax);
+  unsigned jcap = std::min(std::max(floor_j, (unsigned)std::min(1.35 * gj + 128.0, 1e6) & ~7u), jmax);
   unsigned rcap = std::max(floor_r, ((unsigned)std::min(1.8 * gr + 96.0, 1e6)) / HD_ROW_CHUNK *
                                         HD_ROW_CHUNK);
   for (int pass = 0; pass < 24; ++pass) {
@@ -2270,11 +2272,14 @@ static int size_rows(hd_ctx* c) {
     unsigned ctrl[8];
     HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
     const unsigned need_j = ctrl[4], need_r = ctrl[2];
-    // a whole neighbourhood varies little between rebuilds, its parts more
-    // (which candidates a part gets changes); the limit may cut the headroom
+    // a whole neighbourhood varies less between rebuilds than its parts
+    // (which candidates a part gets changes); its headroom is cut to what
+    // leaves room for three of the pair kernel's workgroups per CU, but not
+    // below 0.35
     unsigned want_j = parts > 1 ? ((unsigned)ceil(need_j * 1.75) + 64u + 7u) & ~7u
                                 : ((unsigned)ceil(need_j * 1.5) + 7u) & ~7u;
-    if (1.1 * need_j + 16.0 <= jmax) want_j = std::min(want_j, jmax);
+    if (parts == 1)
+      want_j = std::min(want_j, std::max(3328u, ((unsigned)ceil(need_j * 1.35) + 7u) & ~7u));
     unsigned want_r = ((unsigned)ceil(need_r * 1.5) + HD_ROW_CHUNK - 1u) / HD_ROW_CHUNK *
                       HD_ROW_CHUNK;
     if (want_j > jmax || ((ctrl[0] & NB_STATUS_OVERFLOW) && need_j <= jcap && need_r <= rcap)) {
