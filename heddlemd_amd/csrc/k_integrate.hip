@@ -1982,27 +1982,12 @@ __global__ void __launch_bounds__(512) k_lan_settle(HdIntegrateArgs ia, HdSettle
     }
   }
   const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-  const unsigned g = blockIdx.x * 64u + lane;
-  const bool on = g < a.n_groups;
+  // idle lanes of the last workgroup repeat its last molecule and store
+  // nothing: every wave meets the one barrier whole
+  const unsigned gl = blockIdx.x * 64u + lane;
+  const bool on = gl < a.n_groups;
+  const unsigned g = on ? gl : a.n_groups - 1u;
   const unsigned clo = (unsigned)(ctr & 0xFFFFFFFFull), chi = (unsigned)(ctr >> 32);
-  if (w > 0u) {
-    if (on) {
-      unsigned ids[3];
-      settle_load_ids(a, g, ids);
-      for (unsigned j = w - 1u; j < 9u; j += 7u) {
-        const unsigned k = j / 3u;
-        s_xi[j][lane] =
-            (float)philox_gaussian_f64(l.seed_lo, l.seed_hi, clo, chi,
-                                       k == 0u ? ids[0] : (k == 1u ? ids[1] : ids[2]), j - 3u * k);
-      }
-    }
-    __syncthreads();
-    return;
-  }
-  if (!on) {
-    __syncthreads();
-    return;
-  }
   HdLattice L = hd_load_lattice(a.lattice);
   float half_dt = ia.dt * 0.5f;
   unsigned ids[3];
@@ -2010,26 +1995,38 @@ __global__ void __launch_bounds__(512) k_lan_settle(HdIntegrateArgs ia, HdSettle
   int img[3][3];
   float4 p[3], q[3];
   float v[3][3];
+  SettleGeom G;
+  SettleOut o;
+  if (w > 0u) {
+    for (unsigned j = w - 1u; j < 9u; j += 7u) {
+      const unsigned k = j / 3u;
+      s_xi[j][lane] =
+          (float)philox_gaussian_f64(l.seed_lo, l.seed_hi, clo, chi,
+                                     k == 0u ? ids[0] : (k == 1u ? ids[1] : ids[2]), j - 3u * k);
+    }
+  } else {
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    unsigned i = ids[k];
-    float m = ia.mass[i];
-    float ax = ia.fx[i] / m, ay = ia.fy[i] / m, az = ia.fz[i] / m;
-    float vx = ia.vx[i] + ax * half_dt;
-    float vy = ia.vy[i] + ay * half_dt;
-    float vz = ia.vz[i] + az * half_dt;
-    float4 pq = ia.posq[i];
-    q[k] = pq;
-    float px = pq.x + vx * half_dt, py = pq.y + vy * half_dt, pz = pq.z + vz * half_dt;
-    int ka, kb, kc;
-    hd_wrap_with_image(px, py, pz, ka, kb, kc, L);
-    img[k][0] = ia.ix[i] + ka; img[k][1] = ia.iy[i] + kb; img[k][2] = ia.iz[i] + kc;
-    p[k] = make_float4(px, py, pz, pq.w);
-    v[k][0] = vx; v[k][1] = vy; v[k][2] = vz;
+    for (int k = 0; k < 3; ++k) {
+      unsigned i = ids[k];
+      float m = ia.mass[i];
+      float ax = ia.fx[i] / m, ay = ia.fy[i] / m, az = ia.fz[i] / m;
+      float vx = ia.vx[i] + ax * half_dt;
+      float vy = ia.vy[i] + ay * half_dt;
+      float vz = ia.vz[i] + az * half_dt;
+      float4 pq = ia.posq[i];
+      q[k] = pq;
+      float px = pq.x + vx * half_dt, py = pq.y + vy * half_dt, pz = pq.z + vz * half_dt;
+      int ka, kb, kc;
+      hd_wrap_with_image(px, py, pz, ka, kb, kc, L);
+      img[k][0] = ia.ix[i] + ka; img[k][1] = ia.iy[i] + kb; img[k][2] = ia.iz[i] + kc;
+      p[k] = make_float4(px, py, pz, pq.w);
+      v[k][0] = vx; v[k][1] = vy; v[k][2] = vz;
+    }
+    G = settle_geom(a, g);
+    o = settle_water_positions(G, L, p, q, v, a.dt);
   }
-  SettleGeom G = settle_geom(a, g);
-  SettleOut o = settle_water_positions(G, L, p, q, v, a.dt);
   __syncthreads();
+  if (w > 0u) return;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     unsigned i = ids[k];
@@ -2052,6 +2049,7 @@ __global__ void __launch_bounds__(512) k_lan_settle(HdIntegrateArgs ia, HdSettle
   }
   o = settle_water_positions(G, L, p, q, v, a.dt);
   settle_water_velocities<true>(G, L, o.p, o.v, o.w, a.dt);
+  if (!on) return;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     unsigned i = ids[k];
@@ -2082,33 +2080,33 @@ __global__ void __launch_bounds__(256) k_lan_free(HdIntegrateArgs a, HdLangevinA
     }
   }
   const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-  const unsigned i = blockIdx.x * 64u + lane;
-  const bool on = i < a.n;
+  // as in k_lan_settle: idle lanes repeat the last atom and store nothing
+  const unsigned il = blockIdx.x * 64u + lane;
+  const bool on = il < a.n;
+  const unsigned i = on ? il : a.n - 1u;
   const unsigned clo = (unsigned)(ctr & 0xFFFFFFFFull), chi = (unsigned)(ctr >> 32);
-  if (w > 0u) {
-    if (on)
-      s_xi[w - 1u][lane] =
-          (float)philox_gaussian_f64(l.seed_lo, l.seed_hi, clo, chi, i, w - 1u);
-    __syncthreads();
-    return;
-  }
-  if (!on) {
-    __syncthreads();
-    return;
-  }
   HdLattice L = hd_load_lattice(a.lattice);
-  float m = a.mass[i];
-  float ax = a.fx[i] / m, ay = a.fy[i] / m, az = a.fz[i] / m;
-  float half_dt = a.dt * 0.5f;
-  float vx = a.vx[i] + ax * half_dt;
-  float vy = a.vy[i] + ay * half_dt;
-  float vz = a.vz[i] + az * half_dt;
-  float4 pq = a.posq[i];
-  float px = pq.x + vx * half_dt, py = pq.y + vy * half_dt, pz = pq.z + vz * half_dt;
-  int ka, kb, kc;
-  hd_wrap_with_image(px, py, pz, ka, kb, kc, L);
-  int nx = a.ix[i] + ka, ny = a.iy[i] + kb, nz = a.iz[i] + kc;
+  float m = a.mass[i], half_dt = a.dt * 0.5f;
+  float vx, vy, vz, px, py, pz, pw;
+  int ka, kb, kc, nx, ny, nz;
+  if (w > 0u) {
+    s_xi[w - 1u][lane] =
+        (float)philox_gaussian_f64(l.seed_lo, l.seed_hi, clo, chi, i, w - 1u);
+  } else {
+    float ax = a.fx[i] / m, ay = a.fy[i] / m, az = a.fz[i] / m;
+    vx = a.vx[i] + ax * half_dt;
+    vy = a.vy[i] + ay * half_dt;
+    vz = a.vz[i] + az * half_dt;
+    float4 pq = a.posq[i];
+    px = pq.x + vx * half_dt, py = pq.y + vy * half_dt, pz = pq.z + vz * half_dt;
+    pw = pq.w;
+    hd_wrap_with_image(px, py, pz, ka, kb, kc, L);
+    nx = a.ix[i] + ka;
+    ny = a.iy[i] + kb;
+    nz = a.iz[i] + kc;
+  }
   __syncthreads();
+  if (w > 0u) return;
   float sigma = sqrtf((1.0f - l.alpha * l.alpha) * l.kt / m);
   float xi0 = s_xi[0][lane];
   float xi1 = s_xi[1][lane];
@@ -2118,14 +2116,15 @@ __global__ void __launch_bounds__(256) k_lan_free(HdIntegrateArgs a, HdLangevinA
   vz = l.alpha * vz + sigma * xi2;
   float qx = px + vx * half_dt, qy = py + vy * half_dt, qz = pz + vz * half_dt;
   hd_wrap_with_image(qx, qy, qz, ka, kb, kc, L);
+  if (!on) return;
   a.vx[i] = vx; a.vy[i] = vy; a.vz[i] = vz;
-  a.posq[i] = make_float4(qx, qy, qz, pq.w);
+  a.posq[i] = make_float4(qx, qy, qz, pw);
   a.ix[i] = nx + ka; a.iy[i] = ny + kb; a.iz[i] = nz + kc;
 }
 
 void hd_launch_lan_free(hipStream_t st, const HdIntegrateArgs& a, const HdLangevinArgs& l) {
-  // one block at least: the counter advances as with the separate kernels
-  hipLaunchKernelGGL(k_lan_free, dim3(a.n ? (a.n + 63) / 64 : 1), dim3(256), 0, st, a, l);
+  if (!a.n) return;
+  hipLaunchKernelGGL(k_lan_free, dim3((a.n + 63) / 64), dim3(256), 0, st, a, l);
 }
 
 void hd_launch_lan_settle(hipStream_t st, const HdIntegrateArgs& ia, const HdSettleArgs& a,
