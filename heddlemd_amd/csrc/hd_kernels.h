@@ -23,6 +23,7 @@
 #define HD_ROW_SLOT_BITS 27
 #define HD_ROW_SLOTS (1u << HD_ROW_SLOT_BITS)
 #define HD_ROW_JMAX 4094u  // largest jcap (16 * jcap fits 16 bits)
+#define HD_ROW_BUILD_LDS 21504u  // LDS bytes of k_build_rows beside its j records, at most
 
 struct HdNeighborArgs {
   unsigned n, npad, nvox, cap;

@@ -599,12 +599,13 @@ __device__ __forceinline__ unsigned nb_collect(const unsigned long long* __restr
 //      r_search: with an image per j-atom the pair kernel needs no minimum
 //      image, in narrow and tilted boxes too;
 //   2. the j-atoms within r_search of the box of one of the block's 16-atom
-//      quarters, in a fixed order, to the unit's
-//      j-list and to LDS: those of Lennard-Jones-active types from the front
-//      of the list, the others from its back;
+//      quarters (of one of its atoms where the box is wide), in a fixed
+//      order, to the unit's j-list and to LDS: those of Lennard-Jones-active
+//      types from the front of the list, the others from its back;
 //   3. rows: wave w owns i-atoms 8 w .. 8 w + 7, octet w (coordinates in
 //      scalar registers), queues the j-atoms within r_search of the octet's
-//      box and tests 64 of them at a time against each i-atom; the ballot of the hits gives every hit its place in the row.  A row
+//      box and tests 64 of them at a time against each i-atom; the ballot of
+//      the hits gives every hit its place in the row.  A row
 //      holds the hits' LDS byte offsets (16 index) among the active
 //      j-atoms, padded to a multiple of 32 entries common to the wave's 8
 //      rows, then those among the others, padded alike; padding points to
@@ -704,7 +705,8 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
   __shared__ unsigned wsum[HD_ROW_WAVES];
   __shared__ unsigned wcnt[2][HD_ROW_WAVES];
   __shared__ unsigned s_cost, s_need;
-  __shared__ float4 quart[4][2];
+  __shared__ float4 quart[4][2];  // centre, half; half.w: its atoms are tested one by one
+  __shared__ float ipos[3][64];   // the block's atoms relative to its centre
   __shared__ unsigned short ring[HD_ROW_WAVES][128];
   __shared__ __align__(16) unsigned short stage[HD_ROW_WAVES][HD_ROW_I][NB_STAGE];
   const unsigned t = threadIdx.x, lane = t & 63u, w = t >> 6;
@@ -753,11 +755,21 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
       ly = fminf(ly, __shfl_xor(ly, off)); hy = fmaxf(hy, __shfl_xor(hy, off));
       lz = fminf(lz, __shfl_xor(lz, off)); hz = fmaxf(hz, __shfl_xor(hz, off));
     }
-    if (w == 0 && (lane & 15u) == 0u) {
-      quart[lane >> 4][0] =
-          make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz), 0.f);
-      quart[lane >> 4][1] =
-          make_float4(0.5f * (hx - lx), 0.5f * (hy - ly), 0.5f * (hz - lz), 0.f);
+    if (w == 0) {
+      ipos[0][lane] = v ? p.x : 3.0e18f;
+      ipos[1][lane] = v ? p.y : 3.0e18f;
+      ipos[2][lane] = v ? p.z : 3.0e18f;
+      if ((lane & 15u) == 0u) {
+        const float qx = 0.5f * (hx - lx), qy = 0.5f * (hy - ly), qz = 0.5f * (hz - lz);
+        quart[lane >> 4][0] =
+            make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz), 0.f);
+        // wide: half a diagonal beyond the search radius.  In a liquid no
+        // quarter is (24,576 water atoms: 0 of 1,536); beside a void a
+        // quarter of a few vapour atoms has a box that spans the liquid
+        // (24,603 atoms in a slab: 24,196 j-atoms by the boxes, 2,920 so)
+        quart[lane >> 4][1] = make_float4(
+            qx, qy, qz, qx > 0.f && qx * qx + qy * qy + qz * qz > a.rs2 ? 1.f : 0.f);
+      }
     }
   }
   __syncthreads();
@@ -769,6 +781,12 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
   // others from the back.
   const unsigned pm = a.parts - 1u;
   unsigned nact = 0, nina = 0, e0 = 0, buf = 0;
+  // the wide quarters (bit = quarter) and the limit of their pairs, whose
+  // terms reach across the block
+  const unsigned wide = (unsigned)__builtin_amdgcn_readfirstlane(
+      (quart[0][1].w > 0.f ? 1 : 0) | (quart[1][1].w > 0.f ? 2 : 0) |
+      (quart[2][1].w > 0.f ? 4 : 0) | (quart[3][1].w > 0.f ? 8 : 0));
+  const float reach = sqrtf(rs2) + hb.x + hb.y + hb.z, rs2w = rs2 + 2.0e-6f * reach * reach;
   for (unsigned w0 = 0; w0 < nw; w0 += HD_ROW_WAVES) {
     unsigned ne;
     {
@@ -819,8 +837,18 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
 #pragma unroll
         for (int o = 0; o < 4; ++o) {
           const float4 qc = quart[o][0], qh = quart[o][1];
-          near = near || nb_box_gap2(p[u].x - qc.x, p[u].y - qc.y, p[u].z - qc.z, qh,
-                                     make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2;
+          bool in = nb_box_gap2(p[u].x - qc.x, p[u].y - qc.y, p[u].z - qc.z, qh,
+                                make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2;
+          if (((wide >> o) & 1u) && in) {
+            float d2 = 3.0e38f;
+            for (int i = 16 * o; i < 16 * o + 16; ++i) {
+              const float dx = p[u].x - ipos[0][i], dy = p[u].y - ipos[1][i],
+                          dz = p[u].z - ipos[2][i];
+              d2 = fminf(d2, dx * dx + dy * dy + dz * dz);
+            }
+            in = d2 <= rs2w;
+          }
+          near = near || in;
         }
         near = near && it < ne && slot < a.n && (((e0 + it) * 8u + (lane >> 3)) & pm) == part;
         const unsigned long long mn = __ballot(near),
@@ -879,7 +907,6 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
     float4 p = a.tile_posq[islot];
     unsigned key = a.tile_key[islot];
     hd_rel_image(p.x, p.y, p.z, cb, HD_IMAGE_NONE, HD_IMAGE_NONE, L, p.x, p.y, p.z);
-    const float reach = sqrtf(rs2) + hb.x + hb.y + hb.z;
     // no j-atom is within reach of a slot without atom
     float lim = islot < a.n ? rs2p + 2.0e-6f * reach * reach - (p.x * p.x + p.y * p.y + p.z * p.z)
                             : -3.0e38f;
