@@ -626,7 +626,7 @@ __device__ __forceinline__ unsigned nb_collect(const unsigned long long* __restr
 #define NB_ROUND (HD_ROW_WAVES * NB_PER_WAVE)
 #define NB_STAGE 96u         // entries of a row staged in LDS: a rest below 32 and 64 hits
 #define NB_WORDS_MAX 512u    // mask words (64 blocks each) with candidates
-#define NB_IMAGES_MAX 1024u  // images listed from 512 blocks at a time
+#define NB_IMAGES_MAX 1024u  // images of 512 blocks listed at a time
 
 __device__ __forceinline__ unsigned nb_scan512(unsigned v, unsigned* wsum, unsigned& total) {
   const unsigned lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
@@ -788,106 +788,107 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
       (quart[2][1].w > 0.f ? 4 : 0) | (quart[3][1].w > 0.f ? 8 : 0));
   const float reach = sqrtf(rs2) + hb.x + hb.y + hb.z, rs2w = rs2 + 2.0e-6f * reach * reach;
   for (unsigned w0 = 0; w0 < nw; w0 += HD_ROW_WAVES) {
-    unsigned ne;
-    {
-      unsigned m = 0, jb = 0;
-      if (w0 + w < nw) {
-        const unsigned c = words[w0 + w];
-        jb = c * 64u + lane;
-        if (all ? jb < a.npad / 64u : (a.block_mask[(size_t)b * nchunks + c] >> lane) & 1ull) {
-          const float4 cj = a.center[jb], hj = a.half[jb];
-          // without a mask its test comes first: most waves end there
-          if (!all || nb_box_dist2(cb, hb, cj, hj, L) <= rs2) m = nb_images(cb, hb, cj, hj, L, rs2);
-        }
+    unsigned total, m = 0, jb = 0;
+    if (w0 + w < nw) {
+      const unsigned c = words[w0 + w];
+      jb = c * 64u + lane;
+      if (all ? jb < a.npad / 64u : (a.block_mask[(size_t)b * nchunks + c] >> lane) & 1ull) {
+        const float4 cj = a.center[jb], hj = a.half[jb];
+        // without a mask its test comes first: most waves end there
+        if (!all || nb_box_dist2(cb, hb, cj, hj, L) <= rs2) m = nb_images(cb, hb, cj, hj, L, rs2);
       }
-      unsigned o = nb_scan512((unsigned)__popc(m), wsum, ne);
-      for (; m; m &= m - 1u, ++o)
-        if (o < NB_IMAGES_MAX) images[o] = jb * 32u + (unsigned)__builtin_ctz(m);
-      too_many = too_many || ne > NB_IMAGES_MAX;
-      ne = min(ne, NB_IMAGES_MAX);
     }
-    __syncthreads();
-    float4 np[NB_PER_WAVE];
-    unsigned nt[NB_PER_WAVE], nk[NB_PER_WAVE];
-    auto load = [&](unsigned r0) {
-#pragma unroll
-      for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
-        const unsigned it = r0 + w * NB_PER_WAVE + u;
-        // past the end: block 0, not used
-        const unsigned sl = (it < ne ? images[it] >> 5 : 0u) * 64u + lane;  // < npad
-        np[u] = a.tile_posq[sl];
-        nt[u] = a.tile_type[sl];
-        nk[u] = a.tile_key[sl];
-      }
-    };
-    load(0u);
-    for (unsigned r0 = 0; r0 < ne; r0 += NB_ROUND) {
-      float4 p[NB_PER_WAVE];
-      unsigned js[NB_PER_WAVE], ca = 0, ci = 0;
-      unsigned long long ma[NB_PER_WAVE], mi[NB_PER_WAVE];
-#pragma unroll
-      for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
-        const unsigned it = r0 + w * NB_PER_WAVE + u;
-        const unsigned img = it < ne ? images[it] : HD_IMAGE_NONE, slot = (img >> 5) * 64u + lane;
-        hd_rel_image(np[u].x, np[u].y, np[u].z, cb, img & 31u, HD_IMAGE_NONE, L, p[u].x, p[u].y,
-                     p[u].z);
-        p[u].w = __uint_as_float(nk[u]);
-        js[u] = slot | ((img & 31u) << HD_ROW_SLOT_BITS);
-        bool near = false;
-#pragma unroll
-        for (int o = 0; o < 4; ++o) {
-          const float4 qc = quart[o][0], qh = quart[o][1];
-          bool in = nb_box_gap2(p[u].x - qc.x, p[u].y - qc.y, p[u].z - qc.z, qh,
-                                make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2;
-          if (((wide >> o) & 1u) && in) {
-            float d2 = 3.0e38f;
-            for (int i = 16 * o; i < 16 * o + 16; ++i) {
-              const float dx = p[u].x - ipos[0][i], dy = p[u].y - ipos[1][i],
-                          dz = p[u].z - ipos[2][i];
-              d2 = fminf(d2, dx * dx + dy * dy + dz * dz);
+    const unsigned o0 = nb_scan512((unsigned)__popc(m), wsum, total);
+    // almost always one pass: a block that spans a narrow box meets most
+    // blocks in several images
+    for (unsigned l0 = 0; l0 < total; l0 += NB_IMAGES_MAX) {
+      const unsigned ne = min(total - l0, NB_IMAGES_MAX);
+      unsigned o = o0 - l0;  // wraps before the pass
+      for (unsigned k = m; k; k &= k - 1u, ++o)
+        if (o < NB_IMAGES_MAX) images[o] = jb * 32u + (unsigned)__builtin_ctz(k);
+      __syncthreads();  // after it every wave is done with the pass before
+      float4 np[NB_PER_WAVE];
+      unsigned nt[NB_PER_WAVE], nk[NB_PER_WAVE];
+      auto load = [&](unsigned r0) {
+  #pragma unroll
+        for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
+          const unsigned it = r0 + w * NB_PER_WAVE + u;
+          // past the end: block 0, not used
+          const unsigned sl = (it < ne ? images[it] >> 5 : 0u) * 64u + lane;  // < npad
+          np[u] = a.tile_posq[sl];
+          nt[u] = a.tile_type[sl];
+          nk[u] = a.tile_key[sl];
+        }
+      };
+      load(0u);
+      for (unsigned r0 = 0; r0 < ne; r0 += NB_ROUND) {
+        float4 p[NB_PER_WAVE];
+        unsigned js[NB_PER_WAVE], ca = 0, ci = 0;
+        unsigned long long ma[NB_PER_WAVE], mi[NB_PER_WAVE];
+  #pragma unroll
+        for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
+          const unsigned it = r0 + w * NB_PER_WAVE + u;
+          const unsigned img = it < ne ? images[it] : HD_IMAGE_NONE, slot = (img >> 5) * 64u + lane;
+          hd_rel_image(np[u].x, np[u].y, np[u].z, cb, img & 31u, HD_IMAGE_NONE, L, p[u].x, p[u].y,
+                       p[u].z);
+          p[u].w = __uint_as_float(nk[u]);
+          js[u] = slot | ((img & 31u) << HD_ROW_SLOT_BITS);
+          bool near = false;
+  #pragma unroll
+          for (int o = 0; o < 4; ++o) {
+            const float4 qc = quart[o][0], qh = quart[o][1];
+            bool in = nb_box_gap2(p[u].x - qc.x, p[u].y - qc.y, p[u].z - qc.z, qh,
+                                  make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2;
+            if (((wide >> o) & 1u) && in) {
+              float d2 = 3.0e38f;
+              for (int i = 16 * o; i < 16 * o + 16; ++i) {
+                const float dx = p[u].x - ipos[0][i], dy = p[u].y - ipos[1][i],
+                            dz = p[u].z - ipos[2][i];
+                d2 = fminf(d2, dx * dx + dy * dy + dz * dz);
+              }
+              in = d2 <= rs2w;
             }
-            in = d2 <= rs2w;
+            near = near || in;
           }
-          near = near || in;
+          near = near && it < ne && slot < a.n && (((e0 + it) * 8u + (lane >> 3)) & pm) == part;
+          const unsigned long long mn = __ballot(near),
+                                   mt = __ballot((a.active_types >> nt[u]) & 1u);
+          ma[u] = mn & mt;
+          mi[u] = mn & ~mt;
+          ca += (unsigned)__popcll(ma[u]);
+          ci += (unsigned)__popcll(mi[u]);
         }
-        near = near && it < ne && slot < a.n && (((e0 + it) * 8u + (lane >> 3)) & pm) == part;
-        const unsigned long long mn = __ballot(near),
-                                 mt = __ballot((a.active_types >> nt[u]) & 1u);
-        ma[u] = mn & mt;
-        mi[u] = mn & ~mt;
-        ca += (unsigned)__popcll(ma[u]);
-        ci += (unsigned)__popcll(mi[u]);
-      }
-      load(r0 + NB_ROUND);
-      if (lane == 0) wcnt[buf][w] = ca | (ci << 16);
-      __syncthreads();  // two buffers: the next round's counts land elsewhere
-      unsigned before = 0, all = 0;
-#pragma unroll
-      for (unsigned v = 0; v < HD_ROW_WAVES; ++v) {
-        const unsigned cv = wcnt[buf][v];
-        if (v < w) before += cv;
-        all += cv;
-      }
-      buf ^= 1u;
-      unsigned ja = nact + (before & 0xFFFFu), ji = nina + (before >> 16);
-#pragma unroll
-      for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
-        const bool act = __builtin_amdgcn_inverse_ballot_w64(ma[u]);
-        if (__builtin_amdgcn_inverse_ballot_w64(ma[u] | mi[u])) {
-          const unsigned k = act ? ja + hd_rank(ma[u]) : ji + hd_rank(mi[u]);
-          if (k < a.jcap) {
-            const unsigned o = act ? k : a.jcap - 1u - k;
-            jrec[o] = p[u];
-            a.jslot[(size_t)unit * a.jcap + o] = js[u];
+        load(r0 + NB_ROUND);
+        if (lane == 0) wcnt[buf][w] = ca | (ci << 16);
+        __syncthreads();  // two buffers: the next round's counts land elsewhere
+        unsigned before = 0, all = 0;
+  #pragma unroll
+        for (unsigned v = 0; v < HD_ROW_WAVES; ++v) {
+          const unsigned cv = wcnt[buf][v];
+          if (v < w) before += cv;
+          all += cv;
+        }
+        buf ^= 1u;
+        unsigned ja = nact + (before & 0xFFFFu), ji = nina + (before >> 16);
+  #pragma unroll
+        for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
+          const bool act = __builtin_amdgcn_inverse_ballot_w64(ma[u]);
+          if (__builtin_amdgcn_inverse_ballot_w64(ma[u] | mi[u])) {
+            const unsigned k = act ? ja + hd_rank(ma[u]) : ji + hd_rank(mi[u]);
+            if (k < a.jcap) {
+              const unsigned o = act ? k : a.jcap - 1u - k;
+              jrec[o] = p[u];
+              a.jslot[(size_t)unit * a.jcap + o] = js[u];
+            }
           }
+          ja += (unsigned)__popcll(ma[u]);
+          ji += (unsigned)__popcll(mi[u]);
         }
-        ja += (unsigned)__popcll(ma[u]);
-        ji += (unsigned)__popcll(mi[u]);
+        nact += all & 0xFFFFu;
+        nina += all >> 16;
       }
-      nact += all & 0xFFFFu;
-      nina += all >> 16;
+      e0 += ne;
     }
-    e0 += ne;
   }
   __syncthreads();
   const unsigned need_j = nact + nina;

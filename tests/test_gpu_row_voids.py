@@ -58,3 +58,31 @@ def test_vapour_beside_liquid(oracle, shape, side, n):
         check_forces(e.forces(), F, near, f"{shape} {vapour}")
         assert e.scalars()["pe"] == pytest.approx(E.sum(), abs=1e-5 * np.abs(E).sum())
     e.close()
+
+
+def test_block_that_meets_most_blocks_in_several_images():
+    # a dense cluster in a box hardly wider than twice the search radius, and
+    # 40 atoms around it: their blocks meet 512 others in about 1,500 images
+    rng = np.random.default_rng(2)
+    m, a, side = 32, 0.2 * NM, 12.0 * NM
+    L = np.full(3, systems.box_length(side))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3) - (m - 1) / 2
+    f = rng.uniform(-0.5, 0.5, (800, 3)) * L
+    f = f[np.abs(f).max(axis=1) > (m / 2 + 1.5) * a][:40]
+    x = np.concatenate([a * (g + rng.uniform(-0.04, 0.04, g.shape)), f])
+    n = len(x)
+    s = systems.argon_lattice(n_atoms=n, n_side=40, sigma_m=0.18e-9, cutoff_m=5.7e-9)
+    s.lattice = np.concatenate([L, np.zeros(3)])
+    s.posq[:, :3] = systems.wrap_into_box(x, L)
+    out = []
+    for pair_list in (0, 1):
+        print(f"case: {n} atoms, list {pair_list}", flush=True)
+        e = engine_for(s, dt=U.time(1e-15), r_skin=0.2 * NM, pair_list=pair_list)
+        e.force_eval(scalars=True)
+        out.append((e.forces().astype(np.float64), e.count_pairs(), e.scalars()["pe"]))
+        e.close()
+    (fr, nr, er), (fa, na, ea) = out
+    # pairs within rounding of the cutoff may fall on either side
+    assert abs(int(nr) - int(na)) <= 1e-6 * na
+    check_forces(fr, fa, None, "rows and atom lists")
+    assert er == pytest.approx(ea, rel=1e-5)
