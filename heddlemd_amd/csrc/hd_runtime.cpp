@@ -3508,7 +3508,8 @@ int hd_get_barostat(hd_ctx* c, double* out) {
 int hd_get_neighbor_stats(hd_ctx* c, uint64_t* out) {
   if (!c || !c->ready || !out) return fail(c, HD_ERR_STATE, "not set up");
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  // atom lists: 64-wide rows of a block; row lists: 32-entry chunks of 8 rows
+  // atom lists: 64-wide rows of a block; row lists: chunks (8 rows x 32
+  // entries) of a unit
   std::vector<unsigned> cnt(c->atom_lists ? c->nblocks : c->nblocks * c->parts);
   HIPCHK(c, hipMemcpy(cnt.data(), c->entry_count, cnt.size() * 4, hipMemcpyDeviceToHost));
   unsigned ctrl[4];
@@ -3519,7 +3520,7 @@ int hd_get_neighbor_stats(hd_ctx* c, uint64_t* out) {
     mx = std::max<uint64_t>(mx, v);
   }
   out[0] = c->nblocks;
-  out[1] = c->atom_lists ? c->cap : c->rcap;
+  out[1] = c->atom_lists ? c->cap : HD_ROW_WAVES * (c->rcap / HD_ROW_CHUNK);
   out[2] = mx;
   out[3] = tot;
   out[4] = ctrl[1];

@@ -425,8 +425,11 @@ int hd_count_pairs(hd_ctx *ctx, uint64_t *count);
 /* Barostat state: out[0] last mu, out[1] pressure, out[2] volume after the
  * move, out[3] cumulative P0*dV, out[4] Philox draw counter. */
 int hd_get_barostat(hd_ctx *ctx, double out[5]);
-/* out[0] blocks, out[1] entry capacity per block, out[2] max entries in a
- * block, out[3] total entries, out[4] rebuilds, out[5] status. */
+/* out[0] blocks of 64 atoms, out[1] capacity of a work unit, out[2] most a
+ * unit holds, out[3] total, out[4] rebuilds, out[5] status.  Row lists: a
+ * unit is a block or one part of its neighbourhood, out[1..3] count chunks
+ * of 8 rows x 32 entries; atom lists: a unit is a block, out[1..3] count
+ * rows of 64 entries. */
 int hd_get_neighbor_stats(hd_ctx *ctx, uint64_t out[6]);
 /* SPME grids of the last evaluation: rho (charge grid, na*nb*nc, from the
  * fixed-point spread) and V (potential grid after the convolution). */

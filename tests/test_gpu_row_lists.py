@@ -79,3 +79,17 @@ def check(oracle, s, tag):
     check_forces(f, F, near, tag)
     assert sc["pe"] == pytest.approx(E.sum(), abs=1e-5 * np.abs(E).sum())
     assert sc["virial"] == pytest.approx(W.sum(), abs=1e-5 * np.abs(W).sum())
+
+
+@pytest.mark.parametrize("pair_list", [0, 1])
+def test_neighbor_stats_share_a_unit(pair_list):
+    # capacity, largest and total in the same unit: at set-up the capacity is
+    # what the largest needed and some headroom
+    s = gas(4097, 17, 5.8e-9, "one", False)
+    e = engine_for(s, dt=U.time(1e-15), pair_list=pair_list)
+    e.force_eval(scalars=False)
+    st = e.neighbor_stats()
+    e.close()
+    print(f"case: list {pair_list}: {st}", flush=True)
+    assert 0 < st["max_entries"] <= st["capacity"] <= 4 * st["max_entries"] + 32
+    assert st["max_entries"] <= st["entries"]
