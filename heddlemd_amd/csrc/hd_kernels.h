@@ -47,6 +47,7 @@ struct HdNeighborArgs {
   unsigned *status, *rebuild_count;
   // row lists; entry_count then holds each unit's row chunks
   unsigned parts, jcap, rcap, active_types;  // active_types: bit per LJ type
+  unsigned jmark;                            // j-atoms of a unit that ask for more
   unsigned *jslot, *jcount, *rowhdr, *max_j;
   unsigned short* rows;
   // atom-list mode: entry_atoms holds per-block rows of per-atom neighbour

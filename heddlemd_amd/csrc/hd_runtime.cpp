@@ -189,6 +189,9 @@ struct hd_ctx {
   unsigned *entry_atoms = nullptr, *entry_count = nullptr;
   // row lists: parts per block, j-atoms per unit, entries per row
   unsigned parts = 1, jcap = 0, rcap = 0, active_types = 0;
+  unsigned jneed = 0, jmark = 0;  // j-atoms needed when sized; high-water mark
+  size_t rows_alloc[4] = {0, 0, 0, 0};  // values that jslot, jcount, rowhdr, rows have room for
+  unsigned units = 0;                   // that block_order and entry_count are for
   unsigned *jslot = nullptr, *jcount = nullptr, *rowhdr = nullptr;
   unsigned short* rows = nullptr;
   unsigned long long* block_mask = nullptr;  // block-pair candidate masks
@@ -305,6 +308,21 @@ void dfree(hd_ctx* c, void* p) {
   auto it = std::find(c->allocs.begin(), c->allocs.end(), p);
   if (it != c->allocs.end()) c->allocs.erase(it);
   (void)hipFree(p);
+}
+
+// A buffer of at least `need` values: the one there is where it is not much
+// too large (set-up sizes a list twice within a few percent, and hipFree waits
+// for the device).
+template <class T>
+static int reserve(hd_ctx* c, T*& p, size_t& have, size_t need) {
+  if (p && need <= have && (have <= need + need / 2 || have * sizeof(T) <= (1u << 20)))
+    return HD_OK;
+  dfree(c, p);
+  p = nullptr;
+  have = 0;
+  DALLOC(c, p, need);
+  have = need;
+  return HD_OK;
 }
 
 bool is_pow2(int v) { return v >= 2 && (v & (v - 1)) == 0; }
@@ -441,6 +459,7 @@ HdNeighborArgs nb_args(hd_ctx* c) {
   a.block_order = c->block_order;
   a.parts = c->parts;
   a.jcap = c->jcap;
+  a.jmark = c->jmark;
   a.rcap = c->rcap;
   a.active_types = c->active_types;
   a.jslot = c->jslot;
@@ -2181,14 +2200,18 @@ static int build_list(hd_ctx* c) {
 
 // The pair kernel's unit order: identity until a rebuild orders the units
 static int alloc_units(hd_ctx* c, unsigned units) {
+  if (units == c->units) return HD_OK;  // the order there is is one of these units
   dfree(c, c->block_order);
   dfree(c, c->entry_count);
   c->block_order = c->entry_count = nullptr;
+  c->units = 0;
   DALLOC(c, c->entry_count, units);
   DALLOC(c, c->block_order, units);
   std::vector<unsigned> ident(units);
   for (unsigned b = 0; b < units; ++b) ident[b] = b;
-  return upload(c, c->block_order, ident.data(), units);
+  int r = upload(c, c->block_order, ident.data(), units);
+  if (r == HD_OK) c->units = units;
+  return r;
 }
 
 static int alloc_entries(hd_ctx* c, unsigned cap) {
@@ -2201,11 +2224,15 @@ static int alloc_entries(hd_ctx* c, unsigned cap) {
   return HD_OK;
 }
 
-static int alloc_rows(hd_ctx* c, unsigned parts, unsigned jcap, unsigned rcap) {
+static void free_rows(hd_ctx* c) {
   for (void* p : {(void*)c->jslot, (void*)c->jcount, (void*)c->rowhdr, (void*)c->rows})
     dfree(c, p);
   c->jslot = c->jcount = c->rowhdr = nullptr;
   c->rows = nullptr;
+  for (size_t& n : c->rows_alloc) n = 0;
+}
+
+static int alloc_rows(hd_ctx* c, unsigned parts, unsigned jcap, unsigned rcap) {
   const size_t units = (size_t)c->nblocks * parts;
   if (units >= (1ull << 31) / HD_ROW_WAVES)
     return fail(c, HD_ERR_UNSUPPORTED, "row lists: %zu units", units);
@@ -2213,12 +2240,11 @@ static int alloc_rows(hd_ctx* c, unsigned parts, unsigned jcap, unsigned rcap) {
   c->jcap = jcap;
   c->rcap = rcap;
   int r = alloc_units(c, (unsigned)units);
-  if (r) return r;
-  DALLOC(c, c->jslot, units * jcap);
-  DALLOC(c, c->jcount, units);
-  DALLOC(c, c->rowhdr, units * HD_ROW_WAVES);
-  DALLOC(c, c->rows, units * 64 * rcap);
-  return HD_OK;
+  if (r || (r = reserve(c, c->jslot, c->rows_alloc[0], units * jcap)) ||
+      (r = reserve(c, c->jcount, c->rows_alloc[1], units)) ||
+      (r = reserve(c, c->rowhdr, c->rows_alloc[2], units * HD_ROW_WAVES)))
+    return r;
+  return reserve(c, c->rows, c->rows_alloc[3], units * 64 * rcap);
 }
 
 // Largest j-list of a unit: its records beside the build's candidate lists in
@@ -2252,60 +2278,98 @@ static void rows_guess(const hd_ctx* c, unsigned parts, double* nj, double* nr) 
   *nr = rho * sphere / parts;
 }
 
-// Row lists: probe the sizes with what there is, then give the j-lists and
-// rows headroom (never below the capacities they already have).  A j-list
-// beyond the LDS limit splits the blocks further.
+// Capacities for what a list needed: half as much again and 128 atoms shared
+// by the parts (the parts of a neighbourhood vary more between rebuilds than
+// the whole: which candidates a part gets changes), in a row at least one
+// chunk for each kind of j-atom.  The rebuild asks for more at 3/4 of them; a
+// call's steps may go on for two graph launches after that.
+//
+// An unsplit j-list beyond 3,328 atoms (52 KB of LDS) has 0.35 of headroom and
+// its mark at 0.85: more keeps the SPME kernels from sharing the CUs with the
+// pair kernel, or splits the block.  What it then lacks, eager force
+// evaluations make up for (check_forces).  Us per pass with 0.35, with 0.5
+// and split: 196,608 atoms at a 0.14 nm skin 20,600 / 21,300 / 21,200; 52,773
+// at 0.2 nm 8,700 / 8,950 / 9,160.
+#define ROWS_LDS_SHARE 3328u
+static unsigned rows_want_j(unsigned parts, double need, unsigned jmax) {
+  const double full = parts > 1 ? 1.75 * need + 64.0 : 1.5 * need + 128.0;
+  const double less = std::max((double)ROWS_LDS_SHARE, 1.35 * need);
+  return ((unsigned)ceil(parts == 1 && less <= jmax ? std::min(full, less) : full) + 7u) & ~7u;
+}
+static unsigned rows_want_r(unsigned parts, double need) {
+  const unsigned r = (unsigned)ceil(1.5 * need + 128.0 / parts);
+  return std::max(2u * HD_ROW_CHUNK, (r + HD_ROW_CHUNK - 1u) / HD_ROW_CHUNK * HD_ROW_CHUNK);
+}
+
+static int size_atom_lists(hd_ctx* c);
+
+// Row lists: builds the list with guessed capacities, or after a high-water
+// mark with what the mark asks for, and then in the sizes that it needs.  A
+// j-list that does not fit LDS with its headroom splits the blocks further.
+// A neighbourhood of so many atoms, or of so many periodic images, that
+// splitting does not help is left to the atom lists.
+#define ROWS_PARTS_MAX 256u
 static int size_rows(hd_ctx* c) {
   int r;
-  const unsigned floor_j = c->jcap, floor_r = c->rcap;  // 0 at set-up
-  unsigned parts = std::max(c->parts, rows_parts(c));
   const unsigned jmax = rows_jcap_max(c);
+  bool grow = c->jcap != 0;
+  unsigned parts = grow ? c->parts : rows_parts(c), jcap, rcap;
   double gj, gr;
-  rows_guess(c, parts, &gj, &gr);
-  unsigned jcap = std::min(std::max(floor_j, (unsigned)std::min(1.35 * gj + 128.0, 1e6) & ~7u), jmax);
-  unsigned rcap = std::max(floor_r, ((unsigned)std::min(1.8 * gr + 96.0, 1e6)) / HD_ROW_CHUNK *
-                                        HD_ROW_CHUNK);
+  if (grow) {
+    unsigned ctrl[8];
+    HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
+    jcap = std::max(c->jcap, std::min(rows_want_j(parts, ctrl[4], jmax), jmax));
+    rcap = std::max(c->rcap, rows_want_r(parts, ctrl[2]));
+  } else {
+    rows_guess(c, parts, &gj, &gr);
+    for (; rows_want_j(parts, std::min(1.25 * gj, 1e6), jmax) > jmax && parts < ROWS_PARTS_MAX;
+         parts *= 2)
+      rows_guess(c, 2 * parts, &gj, &gr);
+    jcap = std::min(rows_want_j(parts, std::min(1.4 * gj, 1e6), jmax), jmax);
+    rcap = rows_want_r(parts, std::min(1.2 * gr, 1e6));
+  }
   for (int pass = 0; pass < 24; ++pass) {
     if ((r = alloc_rows(c, parts, jcap, rcap))) return r;
     if ((r = build_list(c))) return r;
     unsigned ctrl[8];
     HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
     const unsigned need_j = ctrl[4], need_r = ctrl[2];
-    // a whole neighbourhood varies less between rebuilds than its parts
-    // (which candidates a part gets changes); its headroom is cut to what
-    // leaves room for three of the pair kernel's workgroups per CU, but not
-    // below 0.35
-    unsigned want_j = parts > 1 ? ((unsigned)ceil(need_j * 1.75) + 64u + 7u) & ~7u
-                                : ((unsigned)ceil(need_j * 1.5) + 7u) & ~7u;
-    if (parts == 1)
-      want_j = std::min(want_j, std::max(3328u, ((unsigned)ceil(need_j * 1.35) + 7u) & ~7u));
-    unsigned want_r = ((unsigned)ceil(need_r * 1.5) + HD_ROW_CHUNK - 1u) / HD_ROW_CHUNK *
-                      HD_ROW_CHUNK;
-    if (want_j > jmax || ((ctrl[0] & NB_STATUS_OVERFLOW) && need_j <= jcap && need_r <= rcap)) {
-      // the j-list does not fit LDS, or the candidates their list
-      if (parts >= 4096u) return fail(c, HD_ERR_OVERFLOW, "neighbour list overflow while sizing");
+    const bool over = (ctrl[0] & NB_STATUS_OVERFLOW) != 0u;
+    const unsigned want_j = rows_want_j(parts, need_j, jmax), want_r = rows_want_r(parts, need_r);
+    if ((over && need_j <= jcap && need_r <= rcap) ||  // more images than are listed
+        (want_j > jmax && parts >= ROWS_PARTS_MAX)) {
+      c->atom_lists = 1;
+      return size_atom_lists(c);
+    }
+    if (want_j > jmax) {
+      // half of what it took (the rows of a cut j-list tell less than that:
+      // then at the mean density)
       parts *= 2;
+      grow = false;
+      rows_guess(c, parts, &gj, &gr);
+      rcap = rows_want_r(parts, need_j > jcap ? std::max(1.2 * gr, 0.55 * need_r) : 0.55 * need_r);
+      jcap = std::min(rows_want_j(parts, 0.55 * need_j, jmax), jmax);
       continue;
     }
-    // kept when it fits and the guess was not far too large
-    const bool fits = !(ctrl[0] & NB_STATUS_OVERFLOW) && want_j <= jcap && want_r <= rcap;
-    if (fits && (pass > 0 || floor_r || (jcap <= 2u * want_j && rcap <= 2u * want_r))) {
-      // set-up builds the list twice, as a probe and in its final size
-      if (pass == 0 && !floor_r && (r = build_list(c))) return r;
+    const bool fits = !over && want_j <= jcap && want_r <= rcap;
+    if (fits && (grow || (want_j == jcap && want_r == rcap))) {
+      c->jneed = need_j;
+      c->jmark = 1.5 * need_j + 128.0 > jcap ? (unsigned)(0.85 * jcap) : jcap / 4u * 3u;
       unsigned zero = 0;
       HIPCHK(c, hipMemcpy(c->ctrl, &zero, sizeof(unsigned), hipMemcpyHostToDevice));
       return HD_OK;
     }
-    jcap = std::max(want_j, fits ? floor_j : jcap);
-    rcap = std::max(want_r, fits ? floor_r : rcap);
+    // set-up and a new split: the sizes needed; high water: never less
+    jcap = grow ? std::max(want_j, jcap) : want_j;
+    rcap = grow ? std::max(want_r, rcap) : want_r;
   }
   return fail(c, HD_ERR_OVERFLOW, "neighbour list overflow while sizing");
 }
 
 // Probe the list size, then size the regions with headroom.
-static int size_list(hd_ctx* c) {
+static int size_atom_lists(hd_ctx* c) {
   int r;
-  if (!c->atom_lists) return size_rows(c);
+  free_rows(c);
   if ((r = alloc_entries(c, 64))) return r;
   if ((r = build_list(c))) return r;
   unsigned ctrl[4];
@@ -2321,6 +2385,11 @@ static int size_list(hd_ctx* c) {
   unsigned zero = 0;
   HIPCHK(c, hipMemcpy(c->ctrl, &zero, sizeof(unsigned), hipMemcpyHostToDevice));
   return HD_OK;
+}
+
+static int size_list(hd_ctx* c) {
+  c->jcap = c->rcap = 0;  // row lists: sized anew
+  return c->atom_lists ? size_atom_lists(c) : size_rows(c);
 }
 
 static void drop_graphs(hd_ctx* c);
@@ -2654,6 +2723,25 @@ static int check_status(hd_ctx* c) {
   return HD_OK;
 }
 
+// The status behind an eager force evaluation (no kick, so that it can be
+// repeated).  An unsplit j-list with less headroom than the others have is
+// split where the evaluation needed what it lacks, and the forces are
+// evaluated again.
+static int check_forces(hd_ctx* c, int ev) {
+  unsigned ctrl[8];
+  HIPCHK(c, hipMemcpyAsync(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if ((ctrl[0] & NB_STATUS_OVERFLOW) && !c->atom_lists && ctrl[4] > c->jcap &&
+      ctrl[4] <= 1.5 * c->jneed + 128.0) {
+    drop_graphs(c);
+    int r = size_rows(c);
+    if (r) return r;
+    enqueue_forces(c, ev, false, false);
+    HIPCHK(c, hipGetLastError());
+  }
+  return check_status(c);
+}
+
 int hd_force_eval(hd_ctx* c, int want_scalars) {
   if (!c || !c->ready) return fail(c, HD_ERR_STATE, "hd_force_eval before hd_setup");
   HIPCHK(c, hipSetDevice(c->device));
@@ -2663,7 +2751,7 @@ int hd_force_eval(hd_ctx* c, int want_scalars) {
     hd_launch_ke(c->stream, (unsigned)c->n, c->vx, c->vy, c->vz, c->mass, c->red_partials,
                  c->scal + 0, nullptr, 0.f, nullptr);
   HIPCHK(c, hipGetLastError());
-  return check_status(c);
+  return check_forces(c, want_scalars != 0);
 }
 
 // Position-only constraint projection of the minimizer
@@ -2754,7 +2842,7 @@ int hd_mc_barostat_move(hd_ctx* c, double pressure, double kt, double max_dv, ui
   // U_old at the current positions
   enqueue_forces(c, 1, false, false);
   c->forces_valid = true;
-  int r = check_status(c);
+  int r = check_forces(c, 1);
   if (r) return r;
   float lat[6];
   double u_old = 0.0;
@@ -2792,7 +2880,7 @@ int hd_mc_barostat_move(hd_ctx* c, double pressure, double kt, double max_dv, ui
   HIPCHK(c, hipMemcpyAsync(c->d_lattice, lat_new, sizeof(lat_new), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->ctrl, &force, sizeof(unsigned), hipMemcpyHostToDevice, c->stream));
   enqueue_forces(c, 1, false, false);
-  if ((r = check_status(c))) return r;
+  if ((r = check_forces(c, 1))) return r;
   double u_new = 0.0;
   HIPCHK(c, hipMemcpyAsync(&u_new, c->scal + 1, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -2820,10 +2908,11 @@ int hd_mc_barostat_move(hd_ctx* c, double pressure, double kt, double max_dv, ui
 static int sd_eval(hd_ctx* c, double* energy, double* fmax) {
   enqueue_forces(c, 1, false, false);
   c->forces_valid = true;
+  HIPCHK(c, hipGetLastError());
+  int r = check_forces(c, 1);
+  if (r) return r;
   hd_launch_fmax2(c->stream, c->fx, c->fy, c->fz, (unsigned)c->n, c->sd_fmax2);
   HIPCHK(c, hipGetLastError());
-  int r = check_status(c);
-  if (r) return r;
   double pe = 0.0, f2 = 0.0;
   HIPCHK(c, hipMemcpyAsync(&pe, c->scal + 1, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(&f2, c->sd_fmax2, sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -3079,7 +3168,7 @@ static int mtk_steps(hd_ctx* c, int n_steps) {
   // W of the current positions (the forces are recomputed identically)
   enqueue_forces(c, 1, false, false);
   c->forces_valid = true;
-  int r = check_status(c);
+  int r = check_forces(c, 1);
   if (r) return r;
   for (int s = 0; s < n_steps; ++s) {
     double k, w;
@@ -3100,7 +3189,7 @@ static int mtk_steps(hd_ctx* c, int n_steps) {
                         c->d_lattice, (float)eb, (float)phx, (unsigned)c->n);
     c->mtk_eps += beta * dt;
     enqueue_forces(c, 1, false, false);
-    if ((r = check_status(c))) return r;
+    if ((r = check_forces(c, 1))) return r;
     if ((r = mtk_ke(c, &k)) || (r = mtk_virial(c, &w))) return r;
     vol = (double)(lat[0] * lat[1] * lat[2]);
     pres = (2.0 * k + w) / (3.0 * vol);
@@ -3149,7 +3238,7 @@ int hd_step(hd_ctx* c, int n_steps, int scalars_last) {
     // any step runs on the list
     enqueue_forces(c, false, false, false);
     c->forces_valid = true;
-    int r = check_status(c);
+    int r = check_forces(c, 0);
     if (r) {
       c->forces_valid = false;
       return r;
@@ -3734,7 +3823,11 @@ int hd_batch_step(hd_batch* b, int n_steps, int scalars_last) {
     if (!c->forces_valid) {
       enqueue_forces(c, false, false, false);
       c->forces_valid = true;
-      BCHK(b, hipStreamSynchronize(c->stream));
+      int r = check_forces(c, 0);
+      if (r) {
+        c->forces_valid = false;
+        return bfail(b, r, "replica %zu: %s", i, c->err.c_str());
+      }
     }
     if (c->d_sh_stats) BCHK(b, hipMemsetAsync(c->d_sh_stats, 0, 6 * sizeof(unsigned), c->stream));
     if (b->gen[i] != c->graph_gen) stale = true;

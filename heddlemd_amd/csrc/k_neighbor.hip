@@ -1045,9 +1045,7 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
     if (need_j > *(volatile unsigned*)a.max_j) atomicMax(a.max_j, need_j);
     unsigned bits = 0u;
     if (need_r > rcap || need_j > a.jcap || too_many) bits = NB_STATUS_OVERFLOW;
-    else if (4u * need_r > 3u * rcap ||
-             (a.parts > 1u ? 4u * need_j > 3u * a.jcap : 16u * need_j > 15u * a.jcap))
-      bits = NB_STATUS_HIGHWATER;
+    else if (4u * need_r > 3u * rcap || need_j > a.jmark) bits = NB_STATUS_HIGHWATER;
     if (bits & ~*(volatile unsigned*)a.status) atomicOr(a.status, bits);
   }
 }
