@@ -177,7 +177,7 @@ struct HdSpmeArgs {
   // voxel binning of the last neighbour rebuild (slot ranges per voxel)
   const unsigned *voxel_rank, *voxel_off;
   unsigned nv[3];
-  float mv[3];  // voxel margin per axis: at least half the skin in voxel units
+  float reach;  // how far atoms may be from their voxels: half the skin at least
   int order;  // B-spline order, 4 or 5
   int no_plane;      // FFT: separate c and b passes even where a plane fits in LDS
 };

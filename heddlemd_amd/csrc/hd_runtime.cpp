@@ -560,12 +560,8 @@ static void enqueue_spme(hd_ctx* c, hipStream_t sst, bool timed) {
   sa.w_share = c->w_share;
   sa.voxel_rank = c->voxel_rank;
   sa.voxel_off = c->voxel_off;
-  for (int d = 0; d < 3; ++d) {
-    sa.nv[d] = c->nv[d];
-    // atoms move at most r_skin/2 between rebuilds; 20 % slack for box
-    // changes since set-up, and 1/64 voxel for the binning's rounding
-    sa.mv[d] = (float)(0.6 * c->r_skin * (double)c->nv[d] * inv_row_norm(c->lattice, d) + 0.015625);
-  }
+  for (int d = 0; d < 3; ++d) sa.nv[d] = c->nv[d];
+  sa.reach = (float)(0.6 * c->r_skin);  // half the skin and 20 %
   stage_begin(c, "spme_recip", timed);
   if (c->dft_mode == 1) {
     hd_launch_spme_spread(sst, sa);

@@ -71,7 +71,9 @@ __device__ __forceinline__ float bspline_w(float x) {
 // coordinate (+1/2) lies in [c0/n, (c1 + p - 1)/n).  Atoms sit in the voxel
 // they were binned into at the last rebuild, and have moved less than half
 // the skin since (the rebuild criterion), so the window is widened by that
-// distance in voxel units (margin) on each side.
+// distance in voxel units on each side.  The voxels shrink and grow with the
+// box, whose present lattice is read here: a captured step goes on while a
+// barostat scales it.
 //
 // The work of a brick is a chain of dependent loads (voxel -> slots ->
 // origin cells -> records), so every stage is spread over all threads: the
@@ -102,8 +104,8 @@ template <int SPME_P>
 __global__ void __launch_bounds__(SPREAD_THREADS) k_spread(
     const float4* __restrict__ spl, const unsigned* __restrict__ sg, unsigned na, unsigned nb,
     unsigned nc, unsigned ba, unsigned bb, unsigned bc, const unsigned* __restrict__ voxel_rank,
-    const unsigned* __restrict__ voxel_off, unsigned nva, unsigned nvb, unsigned nvc, float mva,
-    float mvb, float mvc, unsigned long long* __restrict__ rho) {
+    const unsigned* __restrict__ voxel_off, unsigned nva, unsigned nvb, unsigned nvc,
+    const float* __restrict__ lattice, float reach, unsigned long long* __restrict__ rho) {
   __shared__ unsigned long long acc[SPREAD_BRICK_MAX];
   __shared__ unsigned list[SPREAD_LIST];
   __shared__ uint2 hits[SPREAD_LIST];  // slot; first stencil cell per axis, 8 bits each
@@ -117,6 +119,15 @@ __global__ void __launch_bounds__(SPREAD_THREADS) k_spread(
   const int c0a = (int)(bia * ba), c0b = (int)(bib * bb), c0c = (int)(bic * bc);
   const unsigned vol = ba * bb * bc;
   for (unsigned k = t; k < vol; k += SPREAD_THREADS) acc[k] = 0ull;
+  // the reach along the axes' fractional coordinates, in voxels, and 1/64 of
+  // one for the binning's rounding
+  const HdLattice L = hd_load_lattice(lattice);
+  const float ia = 1.0f / L.lx, ib = 1.0f / L.ly, ic = 1.0f / L.lz;
+  const float ab = L.xy * ia * ib, ac = (L.xy * L.yz - L.xz * L.ly) * ia * ib * ic,
+              bc_ = L.yz * ib * ic;
+  const float mva = reach * (float)nva * sqrtf(ia * ia + ab * ab + ac * ac) + 0.015625f,
+              mvb = reach * (float)nvb * sqrtf(ib * ib + bc_ * bc_) + 0.015625f,
+              mvc = reach * (float)nvc * ic + 0.015625f;
   // voxel window per axis (periodic), at most one full period
   auto low = [](int c, unsigned nv, unsigned n, float m) {
     return (int)floorf((float)c * (float)nv / (float)n - m);
@@ -914,12 +925,12 @@ void hd_launch_spme_spread(hipStream_t st, const HdSpmeArgs& a) {
   if (a.order == 5)
     hipLaunchKernelGGL(k_spread<5>, dim3(nbricks), dim3(SPREAD_THREADS), 0, st, a.spl, a.sg,
                        a.na, a.nb, a.nc, brick[0], brick[1], brick[2], a.voxel_rank, a.voxel_off,
-                       a.nv[0], a.nv[1], a.nv[2], a.mv[0], a.mv[1], a.mv[2],
+                       a.nv[0], a.nv[1], a.nv[2], a.lattice, a.reach,
                        (unsigned long long*)a.rho_fixed);
   else
     hipLaunchKernelGGL(k_spread<4>, dim3(nbricks), dim3(SPREAD_THREADS), 0, st, a.spl, a.sg,
                        a.na, a.nb, a.nc, brick[0], brick[1], brick[2], a.voxel_rank, a.voxel_off,
-                       a.nv[0], a.nv[1], a.nv[2], a.mv[0], a.mv[1], a.mv[2],
+                       a.nv[0], a.nv[1], a.nv[2], a.lattice, a.reach,
                        (unsigned long long*)a.rho_fixed);
 }
 

@@ -62,3 +62,25 @@ def test_spread_of_moved_atoms(oracle, skin_nm):
         e.step(steps)
         check(oracle, e, s, e.positions(), f"moved, skin {skin_nm} nm, {steps} steps")
     e.close()
+
+
+@pytest.mark.parametrize("axis", range(3))
+def test_spread_after_the_box_has_shrunk(oracle, axis):
+    # a barostat takes the box to 0.52 of its width; then atoms drift almost
+    # half the skin from where they were binned
+    s = ions(5000, 0, (40, 40, 40), 4)
+    squeeze = dict(pressure=1.0, tau=1.0, compressibility=0.015)
+    e = engine_for(s, dt=1.0, velocities=np.zeros((3, s.n), np.float32),
+                   berendsen_barostat=squeeze)
+    while float(e.lattice()[0]) > 0.52 * float(s.lattice[0]):
+        e.step(8)
+    e.set_berendsen_barostat(**{**squeeze, "compressibility": 1e-12})
+    e.set_positions(e.positions())
+    v = np.zeros((3, s.n), np.float32)
+    v[axis] = 0.3
+    e.set_velocities(v)
+    e.step(8)  # 2.4 Bohr, half the skin is 2.55
+    width = float(e.lattice()[0]) / float(s.lattice[0])
+    s.lattice = np.concatenate([e.lattice()[:3].astype(np.float64), np.zeros(3)])
+    check(oracle, e, s, e.positions(), f"box {width:.3f} of its width")
+    e.close()
