@@ -118,7 +118,7 @@ struct HdPairArgs {
 // Bit per LJ type with a nonzero interaction with any type: the j-atoms of
 // the others are listed apart, so that their pairs skip the LJ terms.
 unsigned hd_pair_active_types(int nt, const double* sigma, const double* eps);
-// LDS bytes of the row-list pair kernel beside its j records
+// LDS bytes of the row-list pair kernel beside its j records, at most
 unsigned hd_pair_rows_lds(int nt, unsigned jcap);
 // Largest type count of the pair kernels' LDS table.
 int hd_pair_table_max_types();

@@ -2248,7 +2248,7 @@ static int alloc_rows(hd_ctx* c, unsigned parts, unsigned jcap, unsigned rcap) {
 // pair kernel's type table in the 64 KB that a launch may ask for
 static unsigned rows_jcap_max(const hd_ctx* c) {
   unsigned build = (81920u - HD_ROW_BUILD_LDS) / 16u;
-  unsigned pair = (65536u - hd_pair_rows_lds(c->ntypes, 0) - 64u) / (c->ntypes > 1 ? 17u : 16u);
+  unsigned pair = (65536u - hd_pair_rows_lds(c->ntypes, 0) - 64u) / 17u;
   return std::min(std::min(build, pair), HD_ROW_JMAX) & ~7u;
 }
 

@@ -1062,15 +1062,18 @@ static void launch_alist_t(hipStream_t st, const HdPairArgs& a, const PairParams
                        a.cap, a.n, nblocks, a.fpi, a.fpi_ew, a.lj_tab);
 }
 
-unsigned hd_pair_rows_lds(int nt, unsigned jcap) {
-  // the dummy record, the type-pair table and the j types
-  return 16u + (nt > 1 ? 32u * (unsigned)(nt * nt) + jcap + 1u : 0u);
+// LDS beside the j records: the dummy record; KIND 1 and 2 also the type-pair
+// table (two float4 a pair in KIND 2) and the j types
+static unsigned rows_lds(int kind, int nt, unsigned jcap) {
+  return 16u + (kind ? (kind == 2 ? 32u : 16u) * (unsigned)(nt * nt) + jcap + 1u : 0u);
 }
+
+unsigned hd_pair_rows_lds(int nt, unsigned jcap) { return rows_lds(2, nt, jcap); }
 
 template <int EV, int KIND>
 static void launch_rows_c(hipStream_t st, const HdPairArgs& a, const PairParams& P) {
   dim3 grid(a.npad / 64 * a.parts), wg(HD_ROW_THREADS);
-  const size_t lds = (size_t)a.jcap * sizeof(float4) + hd_pair_rows_lds(P.ntypes, a.jcap);
+  const size_t lds = (size_t)a.jcap * sizeof(float4) + rows_lds(KIND, P.ntypes, a.jcap);
   if (P.coul_rc2 > 0.f)
     hipLaunchKernelGGL((k_pair_rows<EV, KIND, true>), grid, wg, lds, st, P, a.lattice,
                        a.tile_posq, a.tile_type, a.tile_img, a.center, a.half, a.jslot, a.jcount,

@@ -81,6 +81,18 @@ def check(oracle, s, tag):
     assert sc["virial"] == pytest.approx(W.sum(), abs=1e-5 * np.abs(W).sum())
 
 
+@pytest.mark.parametrize("n,n_side,box_m", [(40, 4, 2.3e-9), (343, 7, 2.5e-9), (1000, 10, 3.6e-9),
+                                            (2197, 13, 4.6e-9), (16400, 26, 9.0e-9)])
+@pytest.mark.parametrize("charged", [False, True])
+def test_one_type_with_a_switch(oracle, n, n_side, box_m, charged):
+    # the general pair terms with a single type: its table and the j types
+    # lie behind j-lists of several lengths
+    s = gas(n, n_side, box_m, "one", charged)
+    cut = np.full((1, 1), U.length(0.95 * RC if charged else RC))
+    s.lj = systems.LJTable(1, s.lj.sigma, s.lj.epsilon, cut, 0.85 * cut)
+    check(oracle, s, f"{n} atoms, one type, switched")
+
+
 @pytest.mark.parametrize("pair_list", [0, 1])
 def test_neighbor_stats_share_a_unit(pair_list):
     # capacity, largest and total in the same unit: at set-up the capacity is
