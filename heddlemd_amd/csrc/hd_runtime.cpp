@@ -199,7 +199,8 @@ struct hd_ctx {
   // [0] status, [1] rebuild count, [2] most entries of a list row, [3] build
   // ticket, [4] most j-atoms of a row-list unit
   unsigned* ctrl = nullptr;
-  long long *fpi = nullptr, *fpi_ew = nullptr, *fpj = nullptr, *fpj_ew = nullptr;
+  long long *fpi = nullptr, *fpi_ew = nullptr;  // atom lists only
+  long long *fpj = nullptr, *fpj_ew = nullptr;
   // device: SPME
   long long* rho_fixed = nullptr;
   float2* cgrid = nullptr;
@@ -2216,6 +2217,8 @@ static int alloc_entries(hd_ctx* c, unsigned cap) {
   c->cap = cap;
   int r = alloc_units(c, c->nblocks);
   if (r) return r;
+  if (!c->fpi) DALLOC(c, c->fpi, (size_t)c->npad * 4);
+  if (!c->fpi_ew) DALLOC(c, c->fpi_ew, (size_t)c->npad * 2);
   DALLOC(c, c->entry_atoms, (size_t)c->nblocks * cap * 64);
   return HD_OK;
 }
@@ -2527,8 +2530,8 @@ int hd_setup(hd_ctx* c) {
   DALLOC(c, c->center, c->nblocks); DALLOC(c, c->half, c->nblocks);
   DALLOC(c, c->block_mask, (size_t)c->nblocks * hd_block_pair_chunks(c->nblocks));
   DALLOC(c, c->ctrl, 8);
-  DALLOC(c, c->fpi, (size_t)c->npad * 4); DALLOC(c, c->fpj, (size_t)c->npad * 4);
-  DALLOC(c, c->fpi_ew, (size_t)c->npad * 2); DALLOC(c, c->fpj_ew, (size_t)c->npad * 2);
+  DALLOC(c, c->fpj, (size_t)c->npad * 4);
+  DALLOC(c, c->fpj_ew, (size_t)c->npad * 2);
   DALLOC(c, c->red_partials, 2 * HD_REDUCE_BLOCKS);
   DALLOC(c, c->fin_partials, 2 * (size_t)hd_finalize_blocks((unsigned)c->n, true));
   DALLOC(c, c->scal, 8);
