@@ -264,12 +264,6 @@ __device__ __forceinline__ int hd_rot1_i(int v) {
   // the "old" operand is never observed and bound_ctrl is irrelevant
   return __builtin_amdgcn_mov_dpp(v, 0x134, 0xF, 0xF, true);
 }
-__device__ __forceinline__ float hd_rot1(float v) {
-  return __int_as_float(hd_rot1_i(__float_as_int(v)));
-}
-__device__ __forceinline__ unsigned hd_rot1_u(unsigned v) {
-  return (unsigned)hd_rot1_i((int)v);
-}
 
 // f32 -> i64 fixed point at scale 2^48, truncating toward zero; the scale
 // is applied as two exact power-of-two products so no intermediate
@@ -301,8 +295,3 @@ __device__ __forceinline__ void hd_wave_sync() {
 
 // Two words that may alias anything (16-bit list entries moved four at a time).
 typedef unsigned hd_u32x2 __attribute__((ext_vector_type(2), may_alias));
-
-__device__ __forceinline__ unsigned long long hd_lane_mask_lt() {
-  unsigned lane = __lane_id();
-  return lane == 0 ? 0ull : (~0ull >> (64 - lane));
-}

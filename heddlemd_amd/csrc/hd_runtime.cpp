@@ -196,8 +196,8 @@ struct hd_ctx {
   unsigned short* rows = nullptr;
   unsigned long long* block_mask = nullptr;  // block-pair candidate masks
   unsigned* block_order = nullptr;           // pair workgroup -> unit
-  // [0] status, [1] rebuild count, [2] most entries of a list row, [3] build
-  // ticket, [4] most j-atoms of a row-list unit
+  // [0] status, [1] rebuild count, [2] most entries of a list row, [4] most
+  // j-atoms of a row-list unit
   unsigned* ctrl = nullptr;
   long long *fpi = nullptr, *fpi_ew = nullptr;  // atom lists only
   long long *fpj = nullptr, *fpj_ew = nullptr;
@@ -3745,10 +3745,12 @@ int hd_batch_set_lanes(hd_batch* b, int lanes) {
 }
 
 // Relative cost of one replica step in a batch graph: launches dominate
-// small replicas (about 4 us each), atoms and SPME grid points the large
-// ones (per-atom and per-point rates of the large single-system step).
+// small replicas (about 4 us each; with SPME spread, three FFT passes or more
+// beside them; the gather apart above 1,024 atoms), atoms and SPME grid points
+// the large ones (per-atom and per-point rates of the large single-system
+// step).
 static double batch_step_cost(const hd_ctx* c) {
-  double launches = c->have_spme ? 11.0 : 5.0;
+  double launches = (c->have_spme ? 9.0 : 5.0) + (c->n > 1024 ? 1.0 : 0.0);
   double us = 4.0 * launches + 0.002 * (double)c->n;
   if (c->have_spme) us += 0.0005 * (double)c->grid[0] * c->grid[1] * c->grid[2];
   return us;

@@ -1965,8 +1965,8 @@ void hd_launch_lan_ou_drift(hipStream_t st, const HdIntegrateArgs& a, const HdLa
 //
 // 64 molecules per workgroup of eight waves (two per SIMD: SETTLE needs more
 // registers than three would leave): waves 1 to 7 draw a molecule's nine FP64
-// Gaussians while wave 0 takes it through the first half (drawn one after the other behind it: 7,938 atoms 18.7 us, now 13.2;
-// 267 atoms 17.5, now 13.7).
+// Gaussians while wave 0 takes it through the first half (drawn one after the
+// other behind it: 7,938 atoms 18.7 us, now 13.2; 267 atoms 17.5, now 13.7).
 __global__ void __launch_bounds__(512) k_lan_settle(HdIntegrateArgs ia, HdSettleArgs a,
                                                     HdLangevinArgs l) {
   __shared__ unsigned long long s_ctr;

@@ -507,9 +507,9 @@ __global__ void __launch_bounds__(HD_ROW_THREADS) k_pair_rows(
 // and no atomic: the i-side f32 sums are folded into i64 fixed point at
 // 2^48 every 64 neighbours (the reference's per-entry fold), combined over
 // the 4 waves in LDS (integer sums, so the order does not matter) and
-// stored once.  Energy and virial are halved per side as in the packed
-// kernel.  Exclusions were applied when the lists were built.  The
-// displacement takes a per-pair minimum image (ORTHO: one rint per axis).
+// stored once.  Each side of a pair carries half of its energy and virial.
+// Exclusions were applied when the lists were built.  The displacement takes
+// a per-pair minimum image (ORTHO: one rint per axis).
 #define ALIST_U 4
 
 template <int EV, int NT, bool SW, bool ORTHO>
