@@ -810,7 +810,7 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
       float4 np[NB_PER_WAVE];
       unsigned nt[NB_PER_WAVE], nk[NB_PER_WAVE];
       auto load = [&](unsigned r0) {
-  #pragma unroll
+#pragma unroll
         for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
           const unsigned it = r0 + w * NB_PER_WAVE + u;
           // past the end: block 0, not used
@@ -825,7 +825,7 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
         float4 p[NB_PER_WAVE];
         unsigned js[NB_PER_WAVE], ca = 0, ci = 0;
         unsigned long long ma[NB_PER_WAVE], mi[NB_PER_WAVE];
-  #pragma unroll
+#pragma unroll
         for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
           const unsigned it = r0 + w * NB_PER_WAVE + u;
           const unsigned img = it < ne ? images[it] : HD_IMAGE_NONE, slot = (img >> 5) * 64u + lane;
@@ -833,23 +833,26 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
                        p[u].z);
           p[u].w = __uint_as_float(nk[u]);
           js[u] = slot | ((img & 31u) << HD_ROW_SLOT_BITS);
-          bool near = false;
-  #pragma unroll
+          unsigned hit = 0u;  // bit = quarter
+#pragma unroll
           for (int o = 0; o < 4; ++o) {
             const float4 qc = quart[o][0], qh = quart[o][1];
-            bool in = nb_box_gap2(p[u].x - qc.x, p[u].y - qc.y, p[u].z - qc.z, qh,
-                                  make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2;
-            if (((wide >> o) & 1u) && in) {
-              float d2 = 3.0e38f;
-              for (int i = 16 * o; i < 16 * o + 16; ++i) {
-                const float dx = p[u].x - ipos[0][i], dy = p[u].y - ipos[1][i],
-                            dz = p[u].z - ipos[2][i];
-                d2 = fminf(d2, dx * dx + dy * dy + dz * dz);
-              }
-              in = d2 <= rs2w;
-            }
-            near = near || in;
+            hit |= nb_box_gap2(p[u].x - qc.x, p[u].y - qc.y, p[u].z - qc.z, qh,
+                               make_float4(0.f, 0.f, 0.f, 0.f)) <= rs2
+                       ? 1u << o
+                       : 0u;
           }
+          if (wide && hit && !(hit & ~wide)) {
+            float d2 = 3.0e38f;
+            for (unsigned i = 0; i < 64u; ++i) {
+              if (!((hit >> (i >> 4)) & 1u)) continue;
+              const float dx = p[u].x - ipos[0][i], dy = p[u].y - ipos[1][i],
+                          dz = p[u].z - ipos[2][i];
+              d2 = fminf(d2, dx * dx + dy * dy + dz * dz);
+            }
+            hit = d2 <= rs2w ? hit : 0u;
+          }
+          bool near = hit != 0u;
           near = near && it < ne && slot < a.n && (((e0 + it) * 8u + (lane >> 3)) & pm) == part;
           const unsigned long long mn = __ballot(near),
                                    mt = __ballot((a.active_types >> nt[u]) & 1u);
@@ -862,7 +865,7 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
         if (lane == 0) wcnt[buf][w] = ca | (ci << 16);
         __syncthreads();  // two buffers: the next round's counts land elsewhere
         unsigned before = 0, all = 0;
-  #pragma unroll
+#pragma unroll
         for (unsigned v = 0; v < HD_ROW_WAVES; ++v) {
           const unsigned cv = wcnt[buf][v];
           if (v < w) before += cv;
@@ -870,7 +873,7 @@ __global__ void __launch_bounds__(HD_ROW_THREADS, 4) k_build_rows(HdNeighborArgs
         }
         buf ^= 1u;
         unsigned ja = nact + (before & 0xFFFFu), ji = nina + (before >> 16);
-  #pragma unroll
+#pragma unroll
         for (unsigned u = 0; u < NB_PER_WAVE; ++u) {
           const bool act = __builtin_amdgcn_inverse_ballot_w64(ma[u]);
           if (__builtin_amdgcn_inverse_ballot_w64(ma[u] | mi[u])) {
