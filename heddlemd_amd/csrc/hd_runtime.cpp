@@ -2183,9 +2183,8 @@ static int build_list(hd_ctx* c) {
   // force a rebuild and run the neighbour pipeline once
   unsigned force = 0x100u;
   HIPCHK(c, hipMemcpyAsync(c->ctrl, &force, sizeof(unsigned), hipMemcpyHostToDevice, c->stream));
-  unsigned zero = 0;
-  HIPCHK(c, hipMemcpyAsync(c->ctrl + 2, &zero, sizeof(unsigned), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->ctrl + 4, &zero, sizeof(unsigned), hipMemcpyHostToDevice, c->stream));
+  const unsigned zero[3] = {0u, 0u, 0u};
+  HIPCHK(c, hipMemcpyAsync(c->ctrl + 2, zero, sizeof(zero), hipMemcpyHostToDevice, c->stream));
   HdNeighborArgs na = nb_args(c);
   hd_launch_neighbor_update(c->stream, na);
   hd_launch_tile_gather_rebuild(c->stream, na, c->fpj, c->fpj_ew);
@@ -2691,10 +2690,13 @@ int hd_setup(hd_ctx* c) {
   return HD_OK;
 }
 
-static int check_status(hd_ctx* c) {
-  unsigned ctrl[8];
-  HIPCHK(c, hipMemcpyAsync(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, c->stream));
+static int read_ctrl(hd_ctx* c, unsigned ctrl[8]) {
+  HIPCHK(c, hipMemcpyAsync(ctrl, c->ctrl, 8 * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  return HD_OK;
+}
+
+static int act_on_status(hd_ctx* c, const unsigned ctrl[8]) {
   if (ctrl[0] & 8u) {
     if (c->atom_lists)
       return fail(c, HD_ERR_OVERFLOW,
@@ -2722,23 +2724,29 @@ static int check_status(hd_ctx* c) {
   return HD_OK;
 }
 
+static int check_status(hd_ctx* c) {
+  unsigned ctrl[8];
+  int r = read_ctrl(c, ctrl);
+  return r ? r : act_on_status(c, ctrl);
+}
+
 // The status behind an eager force evaluation (no kick, so that it can be
 // repeated).  An unsplit j-list with less headroom than the others have is
 // split where the evaluation needed what it lacks, and the forces are
 // evaluated again.
 static int check_forces(hd_ctx* c, int ev) {
   unsigned ctrl[8];
-  HIPCHK(c, hipMemcpyAsync(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  int r = read_ctrl(c, ctrl);
+  if (r) return r;
   if ((ctrl[0] & NB_STATUS_OVERFLOW) && !c->atom_lists && ctrl[4] > c->jcap &&
       ctrl[4] <= 1.5 * c->jneed + 128.0) {
     drop_graphs(c);
-    int r = size_rows(c);
-    if (r) return r;
+    if ((r = size_rows(c))) return r;
     enqueue_forces(c, ev, false, false);
     HIPCHK(c, hipGetLastError());
+    if ((r = read_ctrl(c, ctrl))) return r;
   }
-  return check_status(c);
+  return act_on_status(c, ctrl);
 }
 
 int hd_force_eval(hd_ctx* c, int want_scalars) {
