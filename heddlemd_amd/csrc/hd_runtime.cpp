@@ -2282,17 +2282,20 @@ static void rows_guess(const hd_ctx* c, unsigned parts, double* nj, double* nr) 
 // chunk for each kind of j-atom.  The rebuild asks for more at 3/4 of them; a
 // call's steps may go on for two graph launches after that.
 //
-// An unsplit j-list beyond 3,328 atoms (52 KB of LDS) has 0.35 of headroom and
-// its mark at 0.85: more keeps the SPME kernels from sharing the CUs with the
-// pair kernel, or splits the block.  What it then lacks, eager force
-// evaluations make up for (check_forces).  Us per pass with 0.35, with 0.5
-// and split: 196,608 atoms at a 0.14 nm skin 20,600 / 21,300 / 21,200; 52,773
-// at 0.2 nm 8,700 / 8,950 / 9,160.
+// An unsplit j-list beyond 3,328 atoms (52 KB of LDS) has 0.35 of headroom,
+// or what the LDS limit leaves down to 0.25, and its mark at 0.85: more keeps
+// the SPME kernels from sharing the CUs with the pair kernel, or splits the
+// block.  What it then lacks, eager force evaluations make up for
+// (check_forces).  Us per pass with 0.35, with 0.5 and split: 196,608 atoms at
+// a 0.14 nm skin 20,600 / 21,300 / 21,200; 52,773 at 0.2 nm 8,700 / 8,950 /
+// 9,160.  A split is undone when the state no longer needs it (act_on_status):
+// 196,608 atoms relaxed from a lattice went on at 0.431 ms a step, joined
+// 0.378.
 #define ROWS_LDS_SHARE 3328u
 static unsigned rows_want_j(unsigned parts, double need, unsigned jmax) {
   const double full = parts > 1 ? 1.75 * need + 64.0 : 1.5 * need + 128.0;
-  const double less = std::max((double)ROWS_LDS_SHARE, 1.35 * need);
-  return ((unsigned)ceil(parts == 1 && less <= jmax ? std::min(full, less) : full) + 7u) & ~7u;
+  const double less = std::max((double)ROWS_LDS_SHARE, std::min(1.35 * need, (double)jmax));
+  return ((unsigned)ceil(parts == 1 && 1.25 * need <= jmax ? std::min(full, less) : full) + 7u) & ~7u;
 }
 static unsigned rows_want_r(unsigned parts, double need) {
   const unsigned r = (unsigned)ceil(1.5 * need + 128.0 / parts);
@@ -2305,22 +2308,26 @@ static int size_atom_lists(hd_ctx* c);
 // mark with what the mark asks for, and then in the sizes that it needs.  A
 // j-list that does not fit LDS with its headroom splits the blocks further.
 // A neighbourhood of so many atoms, or of so many periodic images, that
-// splitting does not help is left to the atom lists.
+// splitting does not help is left to the atom lists.  join: the parts are
+// joined two by two.
 #define ROWS_PARTS_MAX 256u
-static int size_rows(hd_ctx* c) {
+static int size_rows(hd_ctx* c, bool join = false) {
   int r;
   const unsigned jmax = rows_jcap_max(c);
-  bool grow = c->jcap != 0;
-  unsigned parts = grow ? c->parts : rows_parts(c), jcap, rcap;
+  bool grow = c->jcap != 0 && !join;
+  unsigned parts = grow ? c->parts : (join ? c->parts / 2u : rows_parts(c)), jcap, rcap;
   double gj, gr;
-  if (grow) {
-    unsigned ctrl[8];
-    HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
+  unsigned ctrl[8];
+  HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
+  if (join) {
+    jcap = std::min(rows_want_j(parts, 2.0 * ctrl[4], jmax), jmax);
+    rcap = rows_want_r(parts, 2.0 * ctrl[2]);
+  } else if (grow) {
     jcap = std::max(c->jcap, std::min(rows_want_j(parts, ctrl[4], jmax), jmax));
     rcap = std::max(c->rcap, rows_want_r(parts, ctrl[2]));
   } else {
     rows_guess(c, parts, &gj, &gr);
-    for (; rows_want_j(parts, std::min(1.25 * gj, 1e6), jmax) > jmax && parts < ROWS_PARTS_MAX;
+    for (; rows_want_j(parts, std::min(1.35 * gj, 1e6), jmax) > jmax && parts < ROWS_PARTS_MAX;
          parts *= 2)
       rows_guess(c, 2 * parts, &gj, &gr);
     jcap = std::min(rows_want_j(parts, std::min(1.4 * gj, 1e6), jmax), jmax);
@@ -2329,7 +2336,6 @@ static int size_rows(hd_ctx* c) {
   for (int pass = 0; pass < 24; ++pass) {
     if ((r = alloc_rows(c, parts, jcap, rcap))) return r;
     if ((r = build_list(c))) return r;
-    unsigned ctrl[8];
     HIPCHK(c, hipMemcpy(ctrl, c->ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
     const unsigned need_j = ctrl[4], need_r = ctrl[2];
     const bool over = (ctrl[0] & NB_STATUS_OVERFLOW) != 0u;
@@ -2720,6 +2726,16 @@ static int act_on_status(hd_ctx* c, const unsigned ctrl[8]) {
     }
     unsigned zero = 0;
     HIPCHK(c, hipMemcpy(c->ctrl, &zero, sizeof(unsigned), hipMemcpyHostToDevice));
+  } else if (!c->atom_lists && c->parts > rows_parts(c) && ctrl[4]) {
+    // blocks split for a denser state: joined again once the rebuilds since
+    // the last look would have fitted with 0.35 of headroom.  The needs are
+    // maxima, so they start anew for the next look.
+    const unsigned jmax = rows_jcap_max(c), p = c->parts / 2u;
+    if (p > 1u ? rows_want_j(p, 2.0 * ctrl[4], jmax) <= jmax : 2.7 * ctrl[4] <= jmax) {
+      drop_graphs(c);
+      return size_rows(c, true);
+    }
+    HIPCHK(c, hipMemsetAsync(c->ctrl + 4, 0, sizeof(unsigned), c->stream));
   }
   return HD_OK;
 }

@@ -101,3 +101,30 @@ def test_memory_of_a_long_cutoff():
     e.close()
     print(f"case: 24,576 atoms, r_cut 1.2 nm: {used / 2 ** 20:.0f} MiB, {st}", flush=True)
     assert used <= 300 * 2 ** 20
+
+
+def test_split_blocks_are_joined_again():
+    # a frame that splits the blocks, then the set-up's again: the lists end
+    # as those of a context that never saw the dense frame, bits included
+    print("case: 8192 molecules, dense frame and back", flush=True)
+    s = systems.spc_water(n_mol=8192, n_side=21, grid=(40, 40, 40))
+    s.water_groups = None
+    dense = s.posq.copy()
+    dense[:, :3] = systems.wrap_into_box(dense[:, :3].astype(np.float64) * 1.4 ** (-1 / 3),
+                                         s.lattice)
+    moved = s.posq.copy()  # far enough for a rebuild
+    moved[:, :3] = systems.wrap_into_box(moved[:, :3].astype(np.float64) + 4.0, s.lattice)
+    out = []
+    for frames in ([s.posq], [dense, s.posq, moved, s.posq, moved, s.posq]):
+        e = engine_for(s, dt=U.time(1e-15), r_skin=0.2e-9 * U.length(1.0))
+        units = []
+        for p in frames:
+            e.set_positions(p)
+            e.force_eval(scalars=True)
+            units.append(e.neighbor_stats()["max_entries"])
+        st, sc = e.neighbor_stats(), e.scalars()
+        out.append((st["max_entries"], st["entries"], e.forces().tobytes(), sc["pe"]))
+        e.close()
+        print(f"  most of a unit, frame by frame: {units}", flush=True)
+    assert units[1] < 0.75 * units[-1]  # still split behind the dense frame
+    assert out[0] == out[1]
