@@ -2331,7 +2331,7 @@ static int size_rows(hd_ctx* c, bool join = false) {
          parts *= 2)
       rows_guess(c, 2 * parts, &gj, &gr);
     jcap = std::min(rows_want_j(parts, std::min(1.4 * gj, 1e6), jmax), jmax);
-    rcap = rows_want_r(parts, std::min(1.2 * gr, 1e6));
+    rcap = rows_want_r(parts, std::min(1.2 * gr + 40.0, 1e6));  // and its padding
   }
   for (int pass = 0; pass < 24; ++pass) {
     if ((r = alloc_rows(c, parts, jcap, rcap))) return r;
@@ -2351,7 +2351,8 @@ static int size_rows(hd_ctx* c, bool join = false) {
       parts *= 2;
       grow = false;
       rows_guess(c, parts, &gj, &gr);
-      rcap = rows_want_r(parts, need_j > jcap ? std::max(1.2 * gr, 0.55 * need_r) : 0.55 * need_r);
+      rcap = rows_want_r(parts, need_j > jcap ? std::max(1.2 * gr + 40.0, 0.55 * need_r)
+                                              : 0.55 * need_r + 16.0);
       jcap = std::min(rows_want_j(parts, 0.55 * need_j, jmax), jmax);
       continue;
     }
