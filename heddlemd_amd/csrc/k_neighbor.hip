@@ -613,10 +613,10 @@ __device__ __forceinline__ unsigned nb_collect(const unsigned long long* __restr
 // The pair kernel's lane 8 r + s reads entries 4 s .. 4 s + 3 of a 32-entry
 // chunk of row r as one 8-byte load: 64 contiguous bytes per row.
 // Bound by instruction issue (two 8-wave workgroups per CU; a unit's waves
-// spend 55 % of their cycles listing j-atoms and 45 % on the rows): 75 us at
-// 24,576 atoms and a 0.27 nm skin, 190 for the packed tiles' build; 250 us
-// at 196,608 atoms and 0.14 nm, where that took 190.  The list is a pure
-// function of the positions.
+// spend 55 % of their cycles listing j-atoms and 45 % on the rows): 79 us at
+// 24,576 atoms and a 0.27 nm skin, 190 for the packed tiles' build; 294 us
+// at 196,608 atoms and 0.14 nm beside the SPME kernels, where that took 170.
+// The list is a pure function of the positions.
 #define NB_PER_WAVE 2u
 // Up to this many mask words per block (512 blocks, one pass over them) a
 // unit tests every block's box itself: the mask's launch costs more than it

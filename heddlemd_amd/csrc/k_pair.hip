@@ -376,11 +376,12 @@ __device__ __forceinline__ long long row_sum8(long long v) {
 //
 // Bound by the vector ALU (about 34 instructions a slot of an LJ-active
 // j-atom, 27 of another, plus one LDS read): listing the active j-atoms
-// first lets a wave drop the LJ half for whole chunks.  54 VGPRs, so the
-// LDS of the j-list sets the occupancy.  Measured, us per launch (the
-// packed tiles it replaced): 196,608 atoms of water 130 beside the SPME
-// pipeline (208); 24,576 atoms 26 (78); 7,938 atoms 13 (68); 267 atoms 5.1
-// (16).
+// first lets a wave drop the LJ half for whole chunks.  The rows and j-atoms
+// are not far behind: 396 MB a launch at 196,608 atoms of water, 84 us of
+// its 118 alone at a large copy's 4.72 TB/s.  54 VGPRs, so the LDS of the
+// j-list sets the occupancy.  Measured, us per launch (the packed tiles it
+// replaced): 196,608 atoms of water 129 beside the SPME pipeline (209);
+// 24,576 atoms 29 (76); 7,938 atoms 13.5 (69); 267 atoms 5.1 (16).
 template <int EV, int KIND, bool COUL>
 __global__ void __launch_bounds__(HD_ROW_THREADS) k_pair_rows(
     PairParams P, const float* __restrict__ lattice, const float4* __restrict__ tile_posq,
